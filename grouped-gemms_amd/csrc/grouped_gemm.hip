@@ -14,24 +14,23 @@
 // with X on the B side and W on the A side of v_mfma_scale_f32_32x32x64_f8f6f4,
 // so that every lane of the accumulator holds 4 consecutive output columns.
 //
-// Main loop (ring_mainloop): the reduction runs in 64-element stages held in
-// an NS-deep LDS ring.  While stage s is multiplied out of registers, stage
-// s+1 is read from LDS and stages s+2 .. s+NS are in flight, so the copies of
-// a stage have NS-1 stage times to land and the copy engine always has
-// several stages queued.  (The two 64-byte halves of a 128-byte line, copied
-// a stage apart, move at ~80% of the full-line rate; copying stages in pairs
-// recovers the rate but shortens the prefetch, and measured slower.)
+// Main loop (step_mainloop): the reduction runs in 128-element steps, one
+// 128-byte line of every e4m3 row, that alternate between two LDS slots.
+// While a step's two halves are multiplied out of registers, the next step
+// lies in the other slot and the one after it is copied into the slot being
+// left.
 //   * X and W tiles go global -> LDS directly with 16-byte buffer_load ... lds;
 //     chunks outside the reduction range read as zero through the buffer
-//     range check.  LDS rows are 64 bytes (e4m3) or 32 bytes (packed e2m1)
-//     with 16-byte chunks XOR-swizzled by row: conflict-free fragment reads.
+//     range check.  16-byte chunks are XOR-swizzled by row: conflict-free
+//     fragment reads.
 //   * e8m0 scales: a re-layout kernel first writes the plain `to_mx` scales
 //     step-major, one dword (4 scale bytes = one 128-element step) per row:
 //     [step][row].  The scales of a tile for two steps are then a few
-//     contiguous 1 KB pieces, copied into a two-slot scale ring every four
-//     stages; each MFMA takes its lane's byte at op_sel 0.
-//   * one workgroup barrier per stage; fragment and scale registers alternate
-//     between two sets (loop body unrolled twice).
+//     contiguous 1 KB pieces, copied into a two-slot scale area every two
+//     steps (small calls copy the plain scales themselves, 8 steps of a row
+//     at a time); each MFMA picks its lane's byte with op_sel.
+//   * everything but the MFMAs is kept to four instructions per MFMA: one
+//     wave per SIMD issues them all.
 #include <mutex>
 #include <type_traits>
 
@@ -40,9 +39,8 @@
 
 namespace mxgg {
 
-constexpr int BKS = 64;        // reduction elements per stage
-constexpr int STEP = 128;      // reduction elements per scale dword (4 blocks of 32)
-constexpr int SCG = 2;         // steps per step-major scale group (one scale-ring slot)
+constexpr int STEP = 128;      // reduction elements per step: a scale dword (4 blocks of 32)
+constexpr int HALF = 64;       // half a step: reduction elements per MFMA
 
 // Split of the last, partial round.  With T tiles and P workgroups resident
 // at once, the rem = T % P tiles of the last round leave most of the chip idle
@@ -136,13 +134,12 @@ struct Cfg {
   static constexpr int WGM = WGM_;      // waves along rows
   static constexpr int WGN = WGN_;      // waves along columns
   static constexpr int WFMT = WFMT_;    // W element format (X is always e4m3)
-  static constexpr int NS = NS_;        // ring depth (stages)
+  static constexpr int NS = NS_;        // LDS slots (steps)
   // Scale source: false, step-major dwords [step][row] (the re-layout
   // kernel's output or the quantizer's native layout); true, the plain
   // to_mx scales (row r's byte b at r * ld + b, ld a multiple of 16), read
   // directly in 32-byte row pieces of 8 steps.
   static constexpr bool PS = PS_;
-  static constexpr bool XD = false;     // X in two-stage slots (XLine)
   static constexpr bool F4 = WFMT == MXGG_FMT_E2M1;
   static constexpr int NW = WGM * WGN;
   static constexpr int NT = NW * kWave;
@@ -150,85 +147,68 @@ struct Cfg {
   static constexpr int WTN = BN / WGN;
   static constexpr int FM = WTM / 32;
   static constexpr int FN = WTN / 32;
-  static constexpr int XROW = BKS;                  // bytes per X row per stage
-  static constexpr int WROW = F4 ? BKS / 2 : BKS;   // bytes per W row per stage
-  static constexpr int XBYTES = BM * XROW;
-  static constexpr int WBYTES = BN * WROW;
-  static constexpr int STAGE = XBYTES + WBYTES;
-  // scale ring after the data ring: two slots of GSTEPS steps each.
-  // Step-major: GSTEPS x BM X-row dwords ([step][row]) followed by GSTEPS x
-  // BN W-row dwords.  Plain: BM X rows then BN W rows of 32 bytes (steps
-  // 8c .. 8c+7 of the row, c = the group's chunk of the reduction), the two
-  // 16-byte halves of rows 8..15 of every 16 swapped (conflict-free reads of
-  // one step over 32 rows, two ways apart at most).
-  static constexpr int GSTEPS = PS ? 8 : SCG;           // steps per scale group (slot)
-  static constexpr int GSTAGES = GSTEPS * STEP / BKS;   // stages per scale group
+  static constexpr int NMMA = FM * FN;              // MFMAs per wave and half step
+  static constexpr int XROW = STEP;                 // bytes per X row per step
+  static constexpr int WROW = F4 ? STEP / 2 : STEP; // bytes per W row per step
+  static constexpr int XBYTES = BM * XROW;          // one X slot
+  static constexpr int WBYTES = BN * WROW;          // one W slot
+  static constexpr int WOFF = NS * XBYTES;          // X slots, then W slots, then scale slots
+  static constexpr int SOFF = WOFF + NS * WBYTES;
+  // Two scale slots of GSTEPS steps each.  Step-major: GSTEPS x BM X-row
+  // dwords ([step][row]) followed by GSTEPS x BN W-row dwords.  Plain: BM X
+  // rows then BN W rows of 32 bytes (8 steps of the row from the run's first
+  // step on), the two 16-byte halves of rows 8..15 of every 16 swapped
+  // (conflict-free reads of one step over 32 rows, two ways apart at most).
+  static constexpr int GSTEPS = PS ? 8 : 2;
   static constexpr int SSLOT = GSTEPS * (BM + BN) * 4;
-  static constexpr int SOFF = NS * STAGE;
   static constexpr int LDS = SOFF + 2 * SSLOT;
-  static constexpr int QX = XBYTES / 1024 / NW;     // 1 KB data copies per wave and stage
+  static constexpr int QX = XBYTES / 1024 / NW;     // 1 KB data copies per wave and step
   static constexpr int QW = WBYTES / 1024 / NW;
-  static constexpr int LPS = QX + QW;               // LDS-DMA loads per wave and stage
-  // step-major: 1 KB scale copies of the X part (waves 0 ..) and per group
-  static constexpr int NSX = PS ? 0 : SCG * BM * 4 / 1024;
-  static constexpr int NSD = PS ? 0 : SSLOT / 1024;
+  static constexpr int NC = QX + QW;
+  static constexpr int XCR = 1024 / XROW;           // rows per copy
+  static constexpr int WCR = 1024 / WROW;
+  // step-major: 1 KB scale copies of the X part and per group (wave w makes
+  // copy w % NSD)
+  static constexpr int NSX = PS ? 0 : GSTEPS * BM * 4 / 1024;
+  static constexpr int NSD = PS ? 1 : SSLOT / 1024;
   // plain: 1 KB scale copies (32 rows) per wave and group; waves 0 .. NXW-1
   // copy X rows, the others W rows
   static constexpr int SPW = PS ? (BM + BN) / 32 / NW : 0;
   static constexpr int NXW = PS ? BM / 32 / SPW : 0;
-  static_assert(XBYTES % (1024 * NW) == 0 && WBYTES % (1024 * NW) == 0, "tile/wave split");
-  static_assert(PS || ((SCG * BM * 4) % 1024 == 0 && (SCG * BN * 4) % 1024 == 0 && NSD <= NW),
-                "scale copies: one operand each, at most one per wave");
-  static_assert(!PS || (SPW >= 1 && (BM + BN) % (32 * NW) == 0 && (BM / 32) % SPW == 0),
-                "plain scale copies: whole 32-row pieces, one operand per wave");
-  static_assert(BM % 4 == 0 && BN % 4 == 0, "scale pieces stay in one step");
+  // Schedule of a step's 2 * NMMA MFMAs (see step_pos): reads of the second
+  // half step during the first RD, barrier B1 before MFMA PB1, the copies
+  // over the NMMA MFMAs from there, barrier B2 before MFMA PB2 and the next
+  // step's reads over the RD from there.
+  static constexpr int RD = NMMA / 2;
+  static constexpr int PB1 = (5 * NMMA + 7) / 8;
+  static constexpr int PB2 = 5 * NMMA / 4;
+  static_assert(NS == 2, "the main loop alternates between two slots");
+  static_assert(XBYTES % (4096 * NW) == 0 && WBYTES % (4096 * NW) == 0, "copies in runs of four");
+  static_assert(PS || ((GSTEPS * BM * 4) % 1024 == 0 && (GSTEPS * BN * 4) % 1024 == 0 && NW % NSD == 0),
+                "scale copies: one operand each, one per wave");
+  static_assert(!PS || ((SPW == 2 || SPW == 4) && (BM + BN) % (32 * NW) == 0 && (BM / 32) % SPW == 0),
+                "plain scale copies: whole 32-row pieces, one operand per wave, one per two steps");
+  static_assert(SOFF % (2 * SSLOT) == 0, "scale slots are told apart by one address bit");
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile");
-  static_assert(NS >= 3 && LDS <= 160 * 1024, "ring depth / LDS budget");
-  // a scale group is copied GSTAGES - 1 stages (or more) before its first
-  // read; the wait before that read covers it only if the stage read then was
-  // issued no earlier than the group
-  static_assert(NS <= GSTAGES + 1, "ring deeper than the scale prefetch");
-  static_assert((NS - 1) * LPS + 2 * (PS ? SPW : 1) <= 63, "vmcnt range");
-};
-
-// Configuration B with X in two-stage slots.  A row-major X row gives a
-// stage 64 bytes, half a 128-byte line, so the one-stage ring copies each X
-// line in two requests.  X slot q here holds stages 2q and 2q+1 of every
-// tile row as one 128-byte piece, copied as whole lines; W keeps one-stage
-// slots.  B::NS slots of each, in two regions (256 x 256 tiles: X 96 KB,
-// W 48 KB), then the step-major scale ring.  Slot layout: tile row m at
-// byte 128 m, its 16-byte unit u (stage 2q + u / 4, elements 16 (u % 4) ..
-// +15 of it) at unit u ^ (m % 8) ^ ((m / 8) % 2): one unit over 8 consecutive
-// rows hits 8 different 16-byte bank groups of 128 bytes, and over 16
-// consecutive rows 16 different ones of 256 bytes.
-template <class B>
-struct XLine : B {
-  static constexpr bool XD = true;
-  static constexpr int XSLOT = 2 * B::XBYTES;
-  static constexpr int WOFF = B::NS * XSLOT;
-  static constexpr int SOFF = WOFF + B::NS * B::WBYTES;
-  static constexpr int LDS = SOFF + 2 * B::SSLOT;
-  static_assert(!B::PS && !B::F4 && B::NS == 3, "two-stage X slots: e4m3, step-major scales, 3 slots");
-  static_assert(B::QX % 2 == 0, "even and odd X copies alternate in a half pair");
   static_assert(LDS <= 160 * 1024, "LDS budget");
-  static_assert(3 * B::QX + 2 * B::QW + 2 <= 63, "vmcnt range");
+  static_assert(XBYTES + 32 * (FM - 1) * XROW < 65536 && WBYTES + 32 * (FN - 1) * WROW < 65536, "ds_read offsets");
+  static_assert(PB1 >= RD && PB2 >= NMMA && PB2 + RD <= 2 * NMMA && PB1 + NMMA <= 2 * NMMA && NC + 2 <= 63,
+                "step schedule");
 };
 
-// 16-byte chunk swizzles: bijective on the chunk index for every 8-row and
-// every 16-row class, 64-byte rows (swz4) and 32-byte rows (swz2).  Both
-// depend on row % 16 only.
+// 16-byte chunk swizzle of 64-byte rows: bijective on the chunk index for
+// every 8-row and every 16-row class; depends on row % 16 only.
 __device__ __forceinline__ int swz4(int r) {
   return ((((r >> 2) ^ (r >> 3)) & 1) << 1) | (((r >> 1) ^ (r >> 2)) & 1);
 }
-__device__ __forceinline__ int swz2(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
 
 // A tile's rows of one operand in global memory, in one of three layouts,
 // G = 2**pl rows per group:
 //   rows  (pl = 0): byte k of row r at r * ld + k;
 //   pairs (pl = 1, e4m3) and quads (pl = 2, packed e2m1): the G rows of a
 //         group interleave in P = 128 / G byte pieces -- one 64-element
-//         stage of a row -- byte k of row r at (r / G) * G ld +
-//         (k / P) * 128 + (r % G) * P + k % P, so the stage pieces of a group
+//         half step of a row -- byte k of row r at (r / G) * G ld +
+//         (k / P) * 128 + (r % G) * P + k % P, so the half-step pieces of a group
 //         fill one 128-byte line and a copy touches whole lines instead of
 //         halves (pairs) or quarters (quads).
 // Local row r of the tile is row e = r + shift of the buffer `data`, which
@@ -237,10 +217,15 @@ __device__ __forceinline__ int swz2(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
 // return 0 except the other rows of that last group.
 struct Operand {
   __amdgpu_buffer_rsrc_t data;
+  __amdgpu_buffer_rsrc_t dma;    // data, starting kCopyBias bytes earlier (the main loop's copies)
   uint32_t ld;                   // bytes between rows (groups: between groups / G)
   uint32_t pl;                   // log2 G: 0 rows, 1 pairs, 2 quads
   uint32_t shift;                // row0 % G of the tile
 };
+
+// Added to the scalar offsets of the copies, and taken off the base, so that
+// the offsets stay non-negative less the immediate they are paired with.
+constexpr int kCopyBias = 3 * 1024;
 
 // Operand of rows row0 .. row0 + rows - 1 of the matrix at `base`.
 __device__ __forceinline__ Operand make_operand(const uint8_t* base, int64_t ld, int pl, int64_t row0, int rows) {
@@ -252,6 +237,7 @@ __device__ __forceinline__ Operand make_operand(const uint8_t* base, int64_t ld,
   const int64_t unit = ld << pl;                                  // bytes per group
   const uint32_t units = (uint32_t)(((int64_t)o.shift + rows + mask) >> pl);
   o.data = make_rsrc(base + (row0 >> pl) * unit, units * (uint32_t)unit);
+  o.dma = make_rsrc(base + (row0 >> pl) * unit - kCopyBias, units * (uint32_t)unit + kCopyBias);
   return o;
 }
 
@@ -274,157 +260,63 @@ struct ScaleSrc {
   uint32_t row0;    // first row of the tile
 };
 
+#define MXGG_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
+#define MXGG_WAIT_LGKM() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
+#define MXGG_BARRIER() asm volatile("s_barrier" ::: "memory")
+#define MXGG_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
+
 template <class C>
 struct Frags {
   v8i a[C::FN];   // W fragments (MFMA A operand)
   v8i b[C::FM];   // X fragments (MFMA B operand)
 };
 
-// Per-lane copy plan.  Data copy i of a wave covers rows q*R .. q*R+R-1
-// (q = wave*Q + i; R = 16 rows of 64 bytes, or 32 rows of 32 bytes for packed
-// e2m1 W); the lane's row inside a copy and its swizzled chunk do not depend
-// on i, so one per-lane offset serves all copies and the row step of copy i
-// (R rows: R * ld bytes in either layout, R being even) travels in the scalar
-// offset.  The chunk index rides in bits 28..31 (a lane's offset is at most
-// 31 rows, or 8 pairs, of a stride below 2**23 plus 112 bytes: below 2**28).
-// Scale copy of wave w, step-major (w < NSD): slot dwords 256 w .. 256 w +
-// 255, 4 per lane, of the X part (w < NSX) or the W part; lane l covers step
-// u and tile rows r .. r+3 of its operand, at byte s_base + t * s_step of that
-// operand's scale buffer for step t of the reduction.  Plain: copy i of wave
-// w fills slot rows 32 (w SPW + i) .. +31 (X rows for w < NXW, then W rows);
-// lane l holds 16 bytes of row l / 2 of the copy, the half (l ^ (l >> 4)) & 1
-// of the row's 32-byte piece, at byte s_base + i * s_step + 4 t of that
-// operand's scales for the piece starting at step t.
-// Two-stage X slots (C::XD): copy c of a pair covers tile rows 8c .. 8c+7
-// (128 bytes each), lane l row l / 8 of the copy and slot unit l % 8, which
-// holds unit (l % 8) ^ (l / 8) of the row's piece for even c (xoff) and
-// that ^ 1 for odd c (xoff2).
+// Per-wave and per-lane addresses of the main loop.
+// Data copy i of a wave fills 1 KB of a slot, rows (wave * Q + i) * R .. of
+// R = 1024 / row bytes: 8 rows of 128 bytes, whole cache lines of a row-major
+// operand (packed e2m1 W: 16 rows of 64 bytes).  Slot layout, 128-byte rows:
+// tile row m at byte 128 m, its 16-byte unit u (elements 16u .. 16u+15 of the
+// step) at unit u ^ (m % 8) ^ ((m / 8) % 2), so that one unit over 8
+// consecutive rows hits 8 different 16-byte bank groups of 128 bytes, and over
+// 16 rows 16 different ones of 256 bytes; the last term alternates from copy
+// to copy, hence two lane offsets (even, odd copies).  64-byte rows: unit u
+// (32 elements) at u ^ swz4(m).  The K position travels in the lane offsets,
+// the rows in scalar offsets that stay constant: copy i also adds 1024 (i % 4)
+// to the LDS and (taken off again in the scalar offset) to the global address
+// through the instruction's immediate, so M0 changes once in four copies.
 template <class C>
 struct Plan {
-  uint32_t xoff;
-  uint32_t xoff2;
-  uint32_t woff;
-  uint32_t s_base;
-  uint32_t s_step;
+  uint32_t xe, xo, we, wo;           // lane offsets of the X and W copies
+  uint32_t xs[C::QX], ws[C::QW];     // scalar offsets
+  uint32_t mxe, mxo, mwe, mwo;       // 0, or kOOB where the copy's chunk lies past the end in the last step
+  uint32_t xm0, wm0;                 // LDS address of the wave's copies into the slot of the step
+  uint32_t xa[4], wa[4];             // LDS addresses of units 2k + lane / 32 of row lane % 32 (F4: k / 2)
+                                     // in the slot read next (k / 2: the half step; each read toggles)
+  uint32_t sm0;                      // LDS address of the wave's scale copies in slot 0
+  uint32_t sx, sw;                   // LDS addresses of the lane's scale dwords in slot 0
+  uint32_t sv;                       // lane offset of the scale copies
+  uint32_t s_step;                   // step-major: bytes per step; plain: bytes per 32 rows
+  int ux, uw;                        // unit of the lane's X (even copies; odd: ux ^ 1) and W chunk
+  int sh;                            // 8 * (lane / 32)
 };
 
-template <class C>
-__device__ __forceinline__ void make_plan(Plan<C>& P, const Operand& X, const Operand& W,
-                                          const ScaleSrc& xs, const ScaleSrc& ws) {
-  const int lane = threadIdx.x % kWave;
-  if constexpr (C::XD) {
-    const int row = lane / 8;
-    const int ue = (lane & 7) ^ row, uo = ue ^ 1;
-    P.xoff = operand_off(X, (uint32_t)row, (uint32_t)ue * 16u) | ((uint32_t)ue << 28);
-    P.xoff2 = operand_off(X, (uint32_t)row, (uint32_t)uo * 16u) | ((uint32_t)uo << 28);
-  } else {
-    const int row = lane / 4;
-    const int c = (lane & 3) ^ swz4(row);
-    P.xoff = operand_off(X, (uint32_t)row, (uint32_t)c * 16u) | ((uint32_t)c << 28);
-    P.xoff2 = 0;
-  }
-  if constexpr (C::F4) {
-    const int row = lane / 2;
-    const int c = (lane & 1) ^ swz2(row);
-    P.woff = operand_off(W, (uint32_t)row, (uint32_t)c * 16u) | ((uint32_t)c << 28);
-  } else {
-    const int row = lane / 4;
-    const int c = (lane & 3) ^ swz4(row);
-    P.woff = operand_off(W, (uint32_t)row, (uint32_t)c * 16u) | ((uint32_t)c << 28);
-  }
-  const int wave = wave_id();
-  if constexpr (C::PS) {
-    const bool isx = wave < C::NXW;
-    const ScaleSrc& S = isx ? xs : ws;
-    const int row = (isx ? wave : wave - C::NXW) * C::SPW * 32 + lane / 2;   // operand row of the tile
-    const int h = (lane ^ (lane >> 4)) & 1;
-    P.s_step = S.rows * 32u;
-    P.s_base = (S.row0 + (uint32_t)row) * S.rows + (uint32_t)h * 16u;
-  } else {
-    const bool isx = wave < C::NSX;
-    const int R = isx ? C::BM : C::BN;              // tile rows of the lane's operand
-    const int q = (isx ? wave : wave - C::NSX) * 256 + 4 * lane;   // first dword of the lane in its part
-    const int u = q / R;                            // step of the group
-    const ScaleSrc& S = isx ? xs : ws;
-    const uint32_t r = S.row0 + (uint32_t)(q % R);
-    P.s_step = S.rows * 4u;
-    P.s_base = r * 4u + (uint32_t)u * P.s_step;
-  }
-}
-
-// Global -> LDS copies of stage `st` (elements [64 st, 64 st + 64)) into slot
-// `sb`.  A 16-byte chunk (16 elements, or 32 packed e2m1) is loaded iff it
-// lies inside [lo, hi); others -- and every chunk of a stage wholly outside,
-// e.g. a prefetch past the last stage -- read as zeros without touching memory.
-template <class C>
-__device__ __forceinline__ void issue_stage(uint8_t* sb, const Operand& X, const Operand& W,
-                                            const Plan<C>& P, int st, int lo, int hi) {
-  const int wave = wave_id();
-  const int kk = st * BKS;
-  constexpr int WE = C::F4 ? 32 : 16;              // elements per W chunk
-  constexpr int WR = C::F4 ? 32 : 16;              // W rows per copy
-  const int xlo = lo - kk <= 0 ? 0 : (lo - kk + 15) / 16;
-  const int xhi = hi - kk <= 0 ? 0 : (hi - kk) / 16;
-  const int wlo = lo - kk <= 0 ? 0 : (lo - kk + WE - 1) / WE;
-  const int whi = hi - kk <= 0 ? 0 : (hi - kk) / WE;
-  const int xc = (int)(P.xoff >> 28), wc = (int)(P.woff >> 28);
-  const uint32_t xo = (xc >= xlo && xc < xhi) ? (P.xoff & 0x0fffffffu) : kOOB;
-  const uint32_t wo = (wc >= wlo && wc < whi) ? (P.woff & 0x0fffffffu) : kOOB;
-#pragma unroll
-  for (int i = 0; i < C::QX; ++i) {
-    const int q = wave * C::QX + i;
-    const uint32_t so = ((uint32_t)st * C::XROW << X.pl) + (uint32_t)(q * 16) * X.ld;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(X.data, (lds_ptr_t)(sb + q * 1024), 16, xo, so, 0, 0);
-  }
-  uint8_t* wb = sb + C::XBYTES;
-#pragma unroll
-  for (int i = 0; i < C::QW; ++i) {
-    const int q = wave * C::QW + i;
-    const uint32_t so = ((uint32_t)st * C::WROW << W.pl) + (uint32_t)(q * WR) * W.ld;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(W.data, (lds_ptr_t)(wb + q * 1024), 16, wo, so, 0, 0);
-  }
-}
-
-// 16 bytes per lane global -> LDS at LDS byte address `lds` when `go` != 0.
-// The branch lives inside the asm statement, so the loop body stays a single
-// basic block for the compiler (a branch there costs the register allocator
-// dearly); M0 is saved and restored around the copy.  The copy is not known to
-// the compiler: callers order it with explicit vmcnt waits.
-__device__ __forceinline__ void dma16_if(int go, __amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t lds) {
+// Sets M0, the LDS base of the copies that follow (LDS DMA reads M0 one wait
+// state after a write at the earliest).  The copies are issued in asm: M0 then
+// changes where it must and not per copy, and the compiler, which does not
+// see them, adds no waits of its own.  Callers order them with vmcnt waits.
+__device__ __forceinline__ void set_m0(uint32_t lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t saved;
-  asm volatile(
-      "s_cmp_eq_u32 %1, 0\n\t"
-      "s_cbranch_scc1 1f\n\t"
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
-      "s_mov_b32 m0, %0\n"
-      "1:"
-      : "=&s"(saved)
-      : "s"(go), "v"(voff), "s"(lds), "s"(rsrc)
-      : "memory", "scc");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds));
 #endif
 }
 
-// dma16_if with a scalar byte offset `soff` added to the address.
-__device__ __forceinline__ void dma16_if_so(int go, __amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff,
-                                            uint32_t lds) {
+// 16 bytes per lane global -> LDS at M0 + IMM + 16 lane; global byte voff +
+// soff + IMM of rsrc (past its range: zeros).
+template <int IMM>
+__device__ __forceinline__ void copy16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t saved;
-  asm volatile(
-      "s_cmp_eq_u32 %1, 0\n\t"
-      "s_cbranch_scc1 1f\n\t"
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
-      "s_mov_b32 m0, %0\n"
-      "1:"
-      : "=&s"(saved)
-      : "s"(go), "v"(voff), "s"(lds), "s"(rsrc), "s"(soff)
-      : "memory", "scc");
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen offset:%3 lds" ::"v"(voff), "s"(rsrc), "s"(soff), "n"(IMM)
+               : "memory");
 #endif
 }
 
@@ -432,119 +324,253 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(lds_ptr_t)(const_cast<void*>(p));
 }
 
-// Scale group of steps tg .. tg+GSTEPS-1 into scale slot `ss` (ssr: the
-// scale buffer of the wave's operand).  Step-major: waves w < NSD copy 1 KB
-// each; plain: every wave copies SPW pieces of 32 rows (tg a multiple of 8).
+// Plan of a run that starts at step t0 of the reduction.
 template <class C>
-__device__ __forceinline__ void issue_scales(uint8_t* ss, __amdgpu_buffer_rsrc_t ssr, const Plan<C>& P,
-                                             int tg, bool live) {
-  const int wave = wave_id();
-  if constexpr (C::PS) {
-    const int go = uniform(live ? 1 : 0);
-    const uint32_t v = P.s_base + (uint32_t)tg * 4u;
-#pragma unroll
-    for (int i = 0; i < C::SPW; ++i)
-      dma16_if_so(go, ssr, v, (uint32_t)uniform((int)(P.s_step * (uint32_t)i)), lds_addr(ss + (wave * C::SPW + i) * 1024));
-  } else {
-    const int go = (live && wave < C::NSD) ? 1 : 0;
-    dma16_if(uniform(go), ssr, P.s_base + (uint32_t)tg * P.s_step, lds_addr(ss + wave * 1024));
-  }
-}
-
-// Plain scales: piece i (rows 32 (w SPW + i) .. +31 of the slot) of the group
-// of steps tg .. tg+7 into scale slot `ss`, when `live` (wave-uniform i).
-template <class C>
-__device__ __forceinline__ void issue_scale_piece(uint8_t* ss, __amdgpu_buffer_rsrc_t ssr, const Plan<C>& P,
-                                                  int tg, int i, bool live) {
-  static_assert(C::PS, "plain scales");
-  const int wave = wave_id();
-  dma16_if_so(uniform(live ? 1 : 0), ssr, P.s_base + (uint32_t)tg * 4u, (uint32_t)uniform((int)(P.s_step * (uint32_t)i)),
-              lds_addr(ss + (wave * C::SPW + i) * 1024));
-}
-
-// Fragments and raw scale dwords of the stage in data slot `sb`, whose step is
-// step u of the group held in scale slot `ss`.
-template <class C>
-__device__ __forceinline__ void read_stage(const uint8_t* sb, const uint8_t* ss, int u, Frags<C>& F,
-                                           uint32_t (&xs)[C::FM], uint32_t (&ws)[C::FN]) {
-  const int wave = wave_id();
+__device__ __forceinline__ void make_plan(Plan<C>& P, uint8_t* smem, const Operand& X, const Operand& W,
+                                          const ScaleSrc& xss, const ScaleSrc& wss, int t0) {
   const int lane = threadIdx.x % kWave;
+  const int wave = wave_id();
   const int wm = wave / C::WGN, wn = wave % C::WGN;
-  const int hsel = lane >> 5;
-  const int r32 = lane & 31;
-  const int sw = swz4(r32);
-  const int c0 = hsel ^ sw;            // elements 16 hsel .. +15
-  const int c1 = (2 + hsel) ^ sw;      // elements 32 + 16 hsel .. +15
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i) {
-    const uint8_t* row = sb + (wm * C::WTM + i * 32 + r32) * C::XROW;
-    v4i lo = *reinterpret_cast<const v4i*>(row + c0 * 16);
-    v4i hi = *reinterpret_cast<const v4i*>(row + c1 * 16);
-    F.b[i] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  const uint32_t lds0 = lds_addr(smem);
+  {
+    const int row = lane / 8;
+    P.ux = (lane & 7) ^ row;
+    P.xe = operand_off(X, (uint32_t)row, (uint32_t)(t0 * C::XROW + P.ux * 16));
+    P.xo = operand_off(X, (uint32_t)row, (uint32_t)(t0 * C::XROW + (P.ux ^ 1) * 16));
   }
-  const uint8_t* wb = sb + C::XBYTES;
-#pragma unroll
-  for (int j = 0; j < C::FN; ++j) {
-    const uint8_t* row = wb + (wn * C::WTN + j * 32 + r32) * C::WROW;
-    if constexpr (C::F4) {
-      // 32 packed fp4 values, elements 32 hsel .. +31: one 16-byte chunk
-      v4i lo = *reinterpret_cast<const v4i*>(row + (hsel ^ swz2(r32)) * 16);
-      F.a[j] = (v8i){lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0};
-    } else {
-      v4i lo = *reinterpret_cast<const v4i*>(row + c0 * 16);
-      v4i hi = *reinterpret_cast<const v4i*>(row + c1 * 16);
-      F.a[j] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    }
-  }
-  if constexpr (C::PS) {
-    // slot row m: 8 dwords, half (u / 4) ^ ((m >> 3) & 1) holding steps 4 (u / 4) ..
-    const uint32_t* s32 = reinterpret_cast<const uint32_t*>(ss);
-    const int d = ((((u >> 2) ^ (r32 >> 3)) & 1) << 2) | (u & 3);
-#pragma unroll
-    for (int i = 0; i < C::FM; ++i) xs[i] = s32[(wm * C::WTM + i * 32 + r32) * 8 + d];
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j) ws[j] = s32[(C::BM + wn * C::WTN + j * 32 + r32) * 8 + d];
+  if constexpr (C::F4) {
+    const int row = lane / 4;
+    P.uw = (lane & 3) ^ swz4(row);
+    P.we = P.wo = operand_off(W, (uint32_t)row, (uint32_t)(t0 * C::WROW + P.uw * 16));
   } else {
-    const uint32_t* sx = reinterpret_cast<const uint32_t*>(ss) + u * C::BM;
-    const uint32_t* sy = reinterpret_cast<const uint32_t*>(ss) + C::GSTEPS * C::BM + u * C::BN;
+    const int row = lane / 8;
+    P.uw = P.ux;
+    P.we = operand_off(W, (uint32_t)row, (uint32_t)(t0 * C::WROW + P.uw * 16));
+    P.wo = operand_off(W, (uint32_t)row, (uint32_t)(t0 * C::WROW + (P.uw ^ 1) * 16));
+  }
 #pragma unroll
-    for (int i = 0; i < C::FM; ++i) xs[i] = sx[wm * C::WTM + i * 32 + r32];
+  for (int i = 0; i < C::QX; ++i) P.xs[i] = (uint32_t)(C::XCR * (wave * C::QX + i)) * X.ld + (uint32_t)(kCopyBias - 1024 * (i % 4));
 #pragma unroll
-    for (int j = 0; j < C::FN; ++j) ws[j] = sy[wn * C::WTN + j * 32 + r32];
+  for (int i = 0; i < C::QW; ++i) P.ws[i] = (uint32_t)(C::WCR * (wave * C::QW + i)) * W.ld + (uint32_t)(kCopyBias - 1024 * (i % 4));
+  P.xm0 = lds0 + (uint32_t)(wave * C::QX * 1024);
+  P.wm0 = lds0 + (uint32_t)(C::WOFF + wave * C::QW * 1024);
+  const int h = lane >> 5, r32 = lane & 31;
+  const int g = (r32 & 7) ^ ((r32 >> 3) & 1);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    P.xa[k] = (uint32_t)((wm * C::WTM + r32) * C::XROW + (((2 * k + h) ^ g) * 16));
+    const int uw = C::F4 ? ((2 * (k / 2) + h) ^ swz4(r32)) : ((2 * k + h) ^ g);
+    P.wa[k] = (uint32_t)(C::WOFF + (wn * C::WTN + r32) * C::WROW + uw * 16);
+  }
+  P.sh = 8 * h;
+  if constexpr (C::PS) {
+    const bool isx = wave < C::NXW;
+    const ScaleSrc& S = isx ? xss : wss;
+    const int row = (isx ? wave : wave - C::NXW) * C::SPW * 32 + lane / 2;   // operand row of the tile
+    const int half = (lane ^ (lane >> 4)) & 1;
+    P.sv = (S.row0 + (uint32_t)row) * S.rows + (uint32_t)(4 * t0 + half * 16);
+    P.s_step = S.rows * 32u;
+    P.sm0 = lds0 + (uint32_t)(C::SOFF + wave * C::SPW * 1024);
+    const uint32_t sr = (uint32_t)(C::SOFF + r32 * 32 + ((r32 >> 3) & 1) * 16);
+    P.sx = sr + (uint32_t)(wm * C::WTM * 32);
+    P.sw = sr + (uint32_t)((C::BM + wn * C::WTN) * 32);
+  } else {
+    const int wq = wave % C::NSD;
+    const bool isx = wq < C::NSX;
+    const int R = isx ? C::BM : C::BN;              // tile rows of the lane's operand
+    const int q = (isx ? wq : wq - C::NSX) * 256 + 4 * lane;   // first dword of the lane in its part
+    const ScaleSrc& S = isx ? xss : wss;
+    P.s_step = S.rows * 4u;
+    P.sv = (S.row0 + (uint32_t)(q % R)) * 4u + (uint32_t)(t0 + q / R) * P.s_step;
+    P.sm0 = lds0 + (uint32_t)(C::SOFF + wq * 1024);
+    P.sx = (uint32_t)(C::SOFF + (wm * C::WTM + r32) * 4);
+    P.sw = (uint32_t)(C::SOFF + C::GSTEPS * C::BM * 4 + (wn * C::WTN + r32) * 4);
   }
 }
 
-// Move the scale byte of the lane's 32-element block of stage st (block
-// 2 st + hsel: byte 2 (st & 1) + hsel of the step's dword) to byte 0, where
-// op_sel 0 reads it; blocks wholly outside [lo, hi) get the neutral scale
-// 127, so zero-filled data never meets a NaN scale byte.  A block that only
-// partly overlaps [lo, hi) (a bound that is not a multiple of 32) keeps its
-// scale: its in-range elements are real data.
+// Lane offsets of one step's copies (the plan's, or masked ones).
+struct CopyOff {
+  uint32_t xe, xo, we, wo;
+};
+
+// Offsets of the copies of a step of which only units [xlo, xhi) of X and
+// [wlo, whi) of W lie inside the reduction range; the other chunks read as
+// zeros without touching memory.
 template <class C>
-__device__ __forceinline__ void finish_scales(uint32_t (&xs)[C::FM], uint32_t (&ws)[C::FN], int st, int lo,
-                                              int hi) {
-  const int hsel = (threadIdx.x % kWave) >> 5;
-  const int sh = 8 * hsel + 16 * (st & 1);
-  const int k = st * BKS + 32 * hsel;
-  const bool out = k + 32 <= lo || k >= hi;
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i) xs[i] = out ? 127u : (xs[i] >> sh);
-#pragma unroll
-  for (int j = 0; j < C::FN; ++j) ws[j] = out ? 127u : (ws[j] >> sh);
+__device__ __forceinline__ CopyOff mask_copies(const Plan<C>& P, int xlo, int xhi, int wlo, int whi) {
+  CopyOff o;
+  const int xo = P.ux ^ 1, wo = C::F4 ? P.uw : P.uw ^ 1;
+  o.xe = (P.ux >= xlo && P.ux < xhi) ? P.xe : kOOB;
+  o.xo = (xo >= xlo && xo < xhi) ? P.xo : kOOB;
+  o.we = (P.uw >= wlo && P.uw < whi) ? P.we : kOOB;
+  o.wo = (wo >= wlo && wo < whi) ? P.wo : kOOB;
+  return o;
 }
 
-// MFMAs B .. E-1 of a stage (fragment t: row block t / FN, column block
-// t % FN).  FIRST: the reduction's first stage, which starts each accumulator
-// from zero (the MFMA's C operand) instead of reading it.
-template <class C, int B, int E, bool FIRST = false>
-__device__ __forceinline__ void mfma_range(const Frags<C>& F, const uint32_t (&xs)[C::FM],
-                                           const uint32_t (&ws)[C::FN], v16f (&acc)[C::FM][C::FN]) {
-#pragma unroll
-  for (int t = B; t < E; ++t) {
-    const int i = t / C::FN, j = t % C::FN;
-    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(F.a[j], F.b[i], FIRST ? (v16f){} : acc[i][j], C::WFMT,
-                                                                 MXGG_FMT_E4M3, 0, (int)ws[j], 0, (int)xs[i]);
+// Copies I .. E-1 of a step (X, then W) into the slot at P.xm0 / P.wm0.
+template <class C, int I, int E>
+__device__ __forceinline__ void step_copies(const Operand& X, const Operand& W, const Plan<C>& P, const CopyOff& o) {
+  if constexpr (I < E) {
+    if constexpr (I < C::QX) {
+      if constexpr (I % 4 == 0) set_m0(P.xm0 + I * 1024);
+      copy16<(I % 4) * 1024>(X.dma, (I & 1) ? o.xo : o.xe, P.xs[I]);
+    } else {
+      constexpr int J = I - C::QX;
+      if constexpr (J % 4 == 0) set_m0(P.wm0 + J * 1024);
+      copy16<(J % 4) * 1024>(W.dma, (J & 1) ? o.wo : o.we, P.ws[J]);
+    }
+    step_copies<C, I + 1, E>(X, W, P, o);
   }
+}
+
+// Scale copy issued at step t (relative to the run's first step) when t is
+// even, of the group after t's.  Step-major: the wave's 1 KB.  Plain: one
+// 32-row piece of the wave (pieces 0 .. SPW-1 over the group's even steps).
+// The branch lives inside the asm, so the step stays one basic block for the
+// compiler (a branch there costs the register allocator dearly).
+template <class C>
+__device__ __forceinline__ void issue_scales(__amdgpu_buffer_rsrc_t ssr, const Plan<C>& P, int t) {
+  const int g = t / C::GSTEPS + 1;
+  const uint32_t i = C::PS ? (uint32_t)((t / 2) % (C::PS ? C::SPW : 1)) : 0u;
+  const uint32_t m0 = P.sm0 + (uint32_t)((g & 1) * C::SSLOT) + i * 1024u;
+  const uint32_t so = C::PS ? P.s_step * i + (uint32_t)(g * 32) : P.s_step * (uint32_t)(g * C::GSTEPS);
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_bitcmp1_b32 %0, 0\n\t"
+      "s_cbranch_scc1 1f\n\t"
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %2, %3, %4 offen lds\n"
+      "1:"
+      :
+      : "s"(t), "s"(m0), "v"(P.sv), "s"(ssr), "s"(so)
+      : "memory", "scc");
+#endif
+}
+
+// Takes the chunks past the end out of the lane offsets when step t is the
+// last of the run's n (a branch inside the asm, as above).
+template <class C>
+__device__ __forceinline__ void mask_last(Plan<C>& P, int t, int n) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "s_cmp_lg_u32 %4, %9\n\t"
+      "s_cbranch_scc1 1f\n\t"
+      "v_or_b32 %0, %0, %5\n\t"
+      "v_or_b32 %1, %1, %6\n\t"
+      "v_or_b32 %2, %2, %7\n\t"
+      "v_or_b32 %3, %3, %8\n"
+      "1:"
+      : "+v"(P.xe), "+v"(P.xo), "+v"(P.we), "+v"(P.wo)
+      : "s"(t), "v"(P.mxe), "v"(P.mxo), "v"(P.mwe), "v"(P.mwo), "s"(n - 1)
+      : "scc");
+#endif
+}
+
+// Fragments A .. B-1 (W's, then X's) of half step J of the step in the slot
+// P.wa / P.xa point to.
+// MFMA operand layout: lane half h holds elements 16h .. 16h+15 of the half
+// step in dwords 0-3 and 32+16h .. 32+16h+15 in dwords 4-7 (packed e2m1: 32h
+// .. 32h+31 in dwords 0-3).
+template <class C, int J, int A, int B>
+__device__ __forceinline__ void read_frags(const uint8_t* smem, const Plan<C>& P, Frags<C>& F) {
+  if constexpr (A < B) {
+    if constexpr (A < C::FN) {
+      constexpr int off = A * 32 * C::WROW;
+      if constexpr (C::F4) {
+        const v4i l = *reinterpret_cast<const v4i*>(smem + P.wa[2 * J] + off);
+        F.a[A] = (v8i){l[0], l[1], l[2], l[3], 0, 0, 0, 0};
+      } else {
+        const v4i l = *reinterpret_cast<const v4i*>(smem + P.wa[2 * J] + off);
+        const v4i h = *reinterpret_cast<const v4i*>(smem + P.wa[2 * J + 1] + off);
+        F.a[A] = (v8i){l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
+      }
+    } else {
+      constexpr int i = A - C::FN;
+      constexpr int off = i * 32 * C::XROW;
+      const v4i l = *reinterpret_cast<const v4i*>(smem + P.xa[2 * J] + off);
+      const v4i h = *reinterpret_cast<const v4i*>(smem + P.xa[2 * J + 1] + off);
+      F.b[i] = (v8i){l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
+    }
+    read_frags<C, J, A + 1, B>(smem, P, F);
+  }
+}
+
+// Point half step J's read addresses at the other slot.
+template <class C, int J>
+__device__ __forceinline__ void toggle_reads(Plan<C>& P) {
+#pragma unroll
+  for (int k = 2 * J; k < 2 * J + 2; ++k) {
+    P.xa[k] ^= (uint32_t)C::XBYTES;
+    P.wa[k] ^= (uint32_t)C::WBYTES;
+  }
+}
+
+// The lane's raw scale dwords of step t (relative to the run's first step).
+template <class C>
+__device__ __forceinline__ void read_scales(const uint8_t* smem, const Plan<C>& P, int t, uint32_t (&xs)[C::FM],
+                                            uint32_t (&ws)[C::FN]) {
+  const uint32_t slot = (uint32_t)(((t / C::GSTEPS) & 1) * C::SSLOT);
+  uint32_t ax, aw;
+  constexpr int row = C::PS ? 32 : 4;    // bytes between rows
+  if constexpr (C::PS) {
+    const uint32_t s = slot | (uint32_t)((t & 7) * 4);
+    ax = P.sx ^ s;
+    aw = P.sw ^ s;
+  } else {
+    ax = P.sx + (slot + (uint32_t)((t & 1) * C::BM * 4));
+    aw = P.sw + (slot + (uint32_t)((t & 1) * C::BN * 4));
+  }
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i) xs[i] = *reinterpret_cast<const uint32_t*>(smem + ax + i * 32 * row);
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j) ws[j] = *reinterpret_cast<const uint32_t*>(smem + aw + j * 32 * row);
+}
+
+// A step's dword holds the scales of its blocks 0 .. 3; lane half h supplies
+// block h of the first and 2 + h of the second half step.  Shifted down by 8h
+// they are bytes 0 and 2 on every lane, which op_sel picks per MFMA.  The
+// registers the previous MFMA reads its scales from, the last of each array,
+// are written last.
+template <class C>
+__device__ __forceinline__ void shift_scales(const Plan<C>& P, const uint32_t (&xn)[C::FM], const uint32_t (&wn)[C::FN],
+                                             uint32_t (&xs)[C::FM], uint32_t (&ws)[C::FN]) {
+#pragma unroll
+  for (int i = 0; i < C::FM - 1; ++i) xs[i] = xn[i] >> P.sh;
+#pragma unroll
+  for (int j = 0; j < C::FN - 1; ++j) ws[j] = wn[j] >> P.sh;
+  MXGG_SCHED_FENCE();
+  xs[C::FM - 1] = xn[C::FM - 1] >> P.sh;
+  ws[C::FN - 1] = wn[C::FN - 1] >> P.sh;
+}
+
+// Shifted scales of step `ta` (of the whole reduction), the run's first or
+// last: blocks wholly outside [lo, hi) get the neutral scale 127, so
+// zero-filled data never meets a NaN scale byte.  A block that only partly
+// overlaps [lo, hi) (a bound that is not a multiple of 32) keeps its scale:
+// its in-range elements are real data.
+template <class C>
+__device__ __forceinline__ void mask_scales(const Plan<C>& P, int ta, int lo, int hi, uint32_t (&xs)[C::FM],
+                                            uint32_t (&ws)[C::FN]) {
+  const int k0 = ta * STEP + 4 * P.sh, k1 = k0 + 64;   // block of the lane in each half step
+  uint32_t am = 0xffffffffu;
+  if (k0 + 32 <= lo || k0 >= hi) am &= 0xffffff00u;
+  if (k1 + 32 <= lo || k1 >= hi) am &= 0xff00ffffu;
+  const uint32_t om = 0x7f7f7f7fu & ~am;
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i) xs[i] = (xs[i] & am) | om;
+#pragma unroll
+  for (int j = 0; j < C::FN; ++j) ws[j] = (ws[j] & am) | om;
+}
+
+// MFMA T of a half step (row block T / FN, column block T % FN), scale byte
+// OPS of the shifted dwords.
+template <class C, int T, int OPS>
+__device__ __forceinline__ void mfma1(const Frags<C>& F, const uint32_t (&xs)[C::FM], const uint32_t (&ws)[C::FN],
+                                      v16f (&acc)[C::FM][C::FN]) {
+  constexpr int i = T / C::FN, j = T % C::FN;
+  acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(F.a[j], F.b[i], acc[i][j], C::WFMT, MXGG_FMT_E4M3, OPS,
+                                                               (int)ws[j], OPS, (int)xs[i]);
 }
 
 // Keep the MFMA operand registers of a region allocated until the region's
@@ -561,109 +587,17 @@ __device__ __forceinline__ void hold(const FR& F, const uint32_t (&xs)[NM], cons
 #endif
 }
 
-#define MXGG_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
-#define MXGG_BARRIER() asm volatile("s_barrier" ::: "memory")
-#define MXGG_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
-
-// Scheduling recipe: NM MFMAs with the ND DS reads spread over the first NMD
-// of them and the NV VMEM issues (LDS-DMA copies) over the rest, so every read
-// is issued before any copy.
-template <int I, int NM, int NMD, int ND, int NV>
-__device__ __forceinline__ void interleave_step() {
-  if constexpr (I < NM) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // 1 MFMA
-    if constexpr (I < NMD) {
-      constexpr int d = (ND * (I + 1)) / NMD - (ND * I) / NMD;
-      if constexpr (d > 0) __builtin_amdgcn_sched_group_barrier(0x100, d, 0);   // DS reads
-    } else {
-      constexpr int J = I - NMD, NR = NM - NMD;
-      constexpr int v = (NV * (J + 1)) / NR - (NV * J) / NR;
-      if constexpr (v > 0) __builtin_amdgcn_sched_group_barrier(0x010, v, 0);   // VMEM
-    }
-    interleave_step<I + 1, NM, NMD, ND, NV>();
-  }
-}
-
-// One stage: multiply stage s0 + r (Fc, xc, wc), read stage s0 + r + 1 into
-// (Fn, xn, wn), start the copies of stage s0 + r + NS and, when stage
-// s0 + r + 1 opens a scale group, the scales of the group after it.
-// (s0 is the ring's first stage, even, in slot 0; t0 = s0 / 2 its step.)
-// FIRST: stage s0, whose MFMAs start the accumulators from zero.  TAIL:
-// kStageFull as described; kStageNoCopy2 / 1 / 0, the fourth, third and
-// second stage from the end, start no copies (any would fetch a stage past the
-// run: zero fills that only load the LDS port), so the wait for the next
-// stage allows for the copies of 2 / 1 / 0 later stages only; kStageLast,
-// the last stage, only multiplies.
-constexpr int kStageFull = 0, kStageNoCopy2 = 1, kStageNoCopy1 = 2, kStageNoCopy0 = 3, kStageLast = 4;
-template <class C, bool FIRST = false, int TAIL = kStageFull>
-__device__ __forceinline__ void ring_stage(uint8_t* smem, const Operand& X, const Operand& W,
-                                           __amdgpu_buffer_rsrc_t ssr, const Plan<C>& P, int s0, int r,
-                                           int lo, int hi, Frags<C>& Fc, uint32_t (&xc)[C::FM],
-                                           uint32_t (&wc)[C::FN], Frags<C>& Fn, uint32_t (&xn)[C::FM],
-                                           uint32_t (&wn)[C::FN], v16f (&acc)[C::FM][C::FN]) {
-  constexpr int NMMA = C::FM * C::FN;
-  constexpr int NE = NMMA >= 8 ? 2 : 1;       // MFMAs issued ahead of the barrier
-  constexpr int NDS = C::FM * 2 + (C::F4 ? C::FN : C::FN * 2) + C::FM + C::FN;
-  const int rn = r + 1;
-  uint8_t* cur = smem + (r % C::NS) * C::STAGE;
-  const uint8_t* nxt = smem + (rn % C::NS) * C::STAGE;
-  // scale groups: GSTAGES stages each, counted from the ring's first stage
-  // (step-major) or from the 8-step piece holding it (plain: g0 stages into
-  // it; its first step tb a multiple of 8)
-  const int g0 = C::PS ? (s0 & (C::GSTAGES - 1)) : 0;
-  const int gr = g0 + rn;
-  const uint8_t* snx = smem + C::SOFF + ((gr / C::GSTAGES) & 1) * C::SSLOT;
-  if constexpr (TAIL == kStageLast) {
-    mfma_range<C, 0, NMMA, FIRST>(Fc, xc, wc, acc);
-    hold(Fc, xc, wc);
-    MXGG_SCHED_FENCE();
-    return;
-  }
-  mfma_range<C, 0, NE, FIRST>(Fc, xc, wc, acc);
-  MXGG_SCHED_FENCE();
-  // this wave's copies of stage r+1 have landed (the copies of the NS-2
-  // stages after it may still be in flight; in the tail, of those issued)
-  if constexpr (TAIL == kStageNoCopy1)
-    MXGG_WAIT_VM(C::LPS);
-  else if constexpr (TAIL == kStageNoCopy0)
-    MXGG_WAIT_VM(0);
-  else
-    MXGG_WAIT_VM((C::NS - 2) * C::LPS);
-  MXGG_BARRIER();                           // ... every wave's; and stage r's slot is free
-  MXGG_SCHED_FENCE();
-  // LDS reads first, then the copies: a read issued after an LDS-DMA load
-  // may otherwise be given the load's offset register as its destination
-  // while the load still uses it.
-  read_stage<C>(nxt, snx, (gr / 2) % C::GSTEPS, Fn, xn, wn);
-  // stage r+1 opening scale group g = gr / GSTAGES frees the slot of group g-1
-  // (last read, of stage r, before this barrier): group g+1 goes there
-  // (a group that starts past the reduction range is never read: not copied,
-  // so the drain after the last stage waits for no memory read)
-  if constexpr (TAIL == kStageFull) {
-    const int tg = (s0 - g0) / 2 + (gr / C::GSTAGES + 1) * C::GSTEPS;
-    uint8_t* sn = smem + C::SOFF + ((gr / C::GSTAGES + 1) & 1) * C::SSLOT;
-    if constexpr (C::PS) {
-      // plain: the group's SPW pieces one per stage over its first SPW
-      // stages (a burst of copies stalls the waves' issue); a group whose
-      // later pieces would fall on the copy-free last stages starts at or
-      // past the last stage, so it is never read (and tg * STEP >= hi)
-      const int gs = gr % C::GSTAGES;
-      issue_scale_piece<C>(sn, ssr, P, tg, gs < C::SPW ? gs : 0, gs < C::SPW && tg * STEP < hi);
-    } else {
-      const bool opens = gr % C::GSTAGES == 0 && tg * STEP < hi;
-      issue_scales<C>(sn, ssr, P, tg, opens);
-    }
-    issue_stage<C>(cur, X, W, P, s0 + r + C::NS, lo, hi);
-  }
-  mfma_range<C, NE, NMMA, FIRST>(Fc, xc, wc, acc);
-  interleave_step<0, NMMA - NE, (NMMA - NE) / 2, NDS, TAIL == kStageFull ? C::LPS : 0>();
-  static_assert(C::NS == 4, "the tail stages assume a 4-deep ring");
-  MXGG_SCHED_FENCE();
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  finish_scales<C>(xn, wn, s0 + rn, lo, hi);
-  // keep the current set allocated past the rewrite of the next one
-  hold(Fc, xc, wc);
-  MXGG_SCHED_FENCE();
+// Keep the accumulators in AGPRs here.  (Left alone, the allocator shuffles
+// all 256 of them, and spills fragments, on the way into the steps after the
+// loop and into the epilogue.)
+template <class C>
+__device__ __forceinline__ void pin_acc(v16f (&acc)[C::FM][C::FN]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) asm volatile("" : "+a"(acc[i][j]));
+#endif
 }
 
 template <class C>
@@ -674,261 +608,167 @@ __device__ __forceinline__ void zero_acc(v16f (&acc)[C::FM][C::FN]) {
     for (int j = 0; j < C::FN; ++j) acc[i][j] = (v16f){};
 }
 
-// ---------------------------------------------------------------------------
-// Main loop with X in two-stage slots (XLine).  Stage r of the run (stage
-// s0 + r, s0 even) issues the copies of W stage r + 3 into W slot r % 3 and
-// of half (r + 1) & 1 of X pair q = (r + 5) / 2 (stages 2q, 2q+1) into X slot
-// q % 3, the slot of pair (r - 1) / 2, whose stages the waves have read by
-// the stage's barrier; the prologue copies pairs 0 and 1, half 0 of pair 2 and
-// W stages 0 .. 2.  Every full stage thus issues QX + QW copies, and the wait
-// before reading stage r + 1 (W copies two stages earlier, X copies three or
-// more) allows the previous stage's copies in flight.
-// ---------------------------------------------------------------------------
-
-// Half h of the X copies of the pair whose first stage is st (even) into X
-// slot xb; the chunk bounds as in issue_stage.
-template <class C>
-__device__ __forceinline__ void issue_xhalf(uint8_t* xb, const Operand& X, const Plan<C>& P, int st, int h,
-                                            int lo, int hi) {
-  const int wave = wave_id();
-  const int kk = st * BKS;
-  const int xlo = lo - kk <= 0 ? 0 : (lo - kk + 15) / 16;
-  const int xhi = hi - kk <= 0 ? 0 : (hi - kk) / 16;
-  const int ue = (int)(P.xoff >> 28), uo = (int)(P.xoff2 >> 28);
-  const uint32_t xe = (ue >= xlo && ue < xhi) ? (P.xoff & 0x0fffffffu) : kOOB;
-  const uint32_t xo = (uo >= xlo && uo < xhi) ? (P.xoff2 & 0x0fffffffu) : kOOB;
-  const int c0 = (wave * 2 + h) * C::QX;   // first copy (even)
-#pragma unroll
-  for (int i = 0; i < C::QX; ++i) {
-    const uint32_t so = ((uint32_t)st * C::XROW << X.pl) + (uint32_t)((c0 + i) * 8) * X.ld;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(X.data, (lds_ptr_t)(xb + (c0 + i) * 1024), 16, (i & 1) ? xo : xe, so,
-                                             0, 0);
-  }
-}
-
-// W copies of stage st into W slot wb (issue_stage's W part, e4m3).
-template <class C>
-__device__ __forceinline__ void issue_wstage(uint8_t* wb, const Operand& W, const Plan<C>& P, int st, int lo,
-                                             int hi) {
-  const int wave = wave_id();
-  const int kk = st * BKS;
-  const int wlo = lo - kk <= 0 ? 0 : (lo - kk + 15) / 16;
-  const int whi = hi - kk <= 0 ? 0 : (hi - kk) / 16;
-  const int wc = (int)(P.woff >> 28);
-  const uint32_t wo = (wc >= wlo && wc < whi) ? (P.woff & 0x0fffffffu) : kOOB;
-#pragma unroll
-  for (int i = 0; i < C::QW; ++i) {
-    const int q = wave * C::QW + i;
-    const uint32_t so = ((uint32_t)st * C::WROW << W.pl) + (uint32_t)(q * 16) * W.ld;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(W.data, (lds_ptr_t)(wb + q * 1024), 16, wo, so, 0, 0);
-  }
-}
-
-// read_stage for two-stage X slots: the stage of parity h2 of X slot xb, the
-// W stage in wb, step u of the scale group in ss.
-template <class C>
-__device__ __forceinline__ void read_stage_xd(const uint8_t* xb, const uint8_t* wb, const uint8_t* ss, int u, int h2,
-                                              Frags<C>& F, uint32_t (&xs)[C::FM], uint32_t (&ws)[C::FN]) {
-  const int wave = wave_id();
-  const int lane = threadIdx.x % kWave;
-  const int wm = wave / C::WGN, wn = wave % C::WGN;
-  const int hsel = lane >> 5;
-  const int r32 = lane & 31;
-  const int g = (r32 & 7) ^ ((r32 >> 3) & 1);
-  const int x0 = ((h2 << 2) | hsel) ^ g;        // elements 16 hsel .. +15
-  const int x1 = ((h2 << 2) | 2 | hsel) ^ g;    // elements 32 + 16 hsel .. +15
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i) {
-    const uint8_t* row = xb + (wm * C::WTM + i * 32 + r32) * 128;
-    v4i lo = *reinterpret_cast<const v4i*>(row + x0 * 16);
-    v4i hi = *reinterpret_cast<const v4i*>(row + x1 * 16);
-    F.b[i] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  }
-  const int sw = swz4(r32);
-  const int c0 = hsel ^ sw;
-  const int c1 = (2 + hsel) ^ sw;
-#pragma unroll
-  for (int j = 0; j < C::FN; ++j) {
-    const uint8_t* row = wb + (wn * C::WTN + j * 32 + r32) * C::WROW;
-    v4i lo = *reinterpret_cast<const v4i*>(row + c0 * 16);
-    v4i hi = *reinterpret_cast<const v4i*>(row + c1 * 16);
-    F.a[j] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  }
-  const uint32_t* sx = reinterpret_cast<const uint32_t*>(ss) + u * C::BM;
-  const uint32_t* sy = reinterpret_cast<const uint32_t*>(ss) + C::GSTEPS * C::BM + u * C::BN;
-#pragma unroll
-  for (int i = 0; i < C::FM; ++i) xs[i] = sx[wm * C::WTM + i * 32 + r32];
-#pragma unroll
-  for (int j = 0; j < C::FN; ++j) ws[j] = sy[wn * C::WTN + j * 32 + r32];
-}
-
-// One stage of the two-stage-X ring, as ring_stage: multiply stage s0 + r,
-// read stage s0 + r + 1, issue the copies described above.  TAIL: kXdFull;
-// kXdNoCopy1 / kXdNoCopy0, the third and second stage from the end, issue
-// nothing and wait for the copies of one / no later stage; kXdLast only
-// multiplies.
-constexpr int kXdFull = 0, kXdNoCopy1 = 1, kXdNoCopy0 = 2, kXdLast = 3;
-template <class C, bool FIRST = false, int TAIL = kXdFull>
-__device__ __forceinline__ void ring_stage_xd(uint8_t* smem, const Operand& X, const Operand& W,
-                                              __amdgpu_buffer_rsrc_t ssr, const Plan<C>& P, int s0, int r,
-                                              int lo, int hi, Frags<C>& Fc, uint32_t (&xc)[C::FM],
-                                              uint32_t (&wc)[C::FN], Frags<C>& Fn, uint32_t (&xn)[C::FM],
-                                              uint32_t (&wn)[C::FN], v16f (&acc)[C::FM][C::FN]) {
-  constexpr int NMMA = C::FM * C::FN;
-  constexpr int NE = NMMA >= 8 ? 2 : 1;
-  constexpr int NDS = C::FM * 2 + C::FN * 2 + C::FM + C::FN;
-  const int rn = r + 1;
-  const uint8_t* xnx = smem + ((rn >> 1) % C::NS) * C::XSLOT;
-  const uint8_t* wnx = smem + C::WOFF + (rn % C::NS) * C::WBYTES;
-  const uint8_t* snx = smem + C::SOFF + ((rn / C::GSTAGES) & 1) * C::SSLOT;
-  if constexpr (TAIL == kXdLast) {
-    mfma_range<C, 0, NMMA, FIRST>(Fc, xc, wc, acc);
-    hold(Fc, xc, wc);
-    MXGG_SCHED_FENCE();
-    return;
-  }
-  mfma_range<C, 0, NE, FIRST>(Fc, xc, wc, acc);
-  MXGG_SCHED_FENCE();
-  if constexpr (TAIL == kXdNoCopy0)
-    MXGG_WAIT_VM(0);
-  else
-    MXGG_WAIT_VM(C::LPS);
-  MXGG_BARRIER();
-  MXGG_SCHED_FENCE();
-  read_stage_xd<C>(xnx, wnx, snx, (rn / 2) % C::GSTEPS, rn & 1, Fn, xn, wn);
-  if constexpr (TAIL == kXdFull) {
-    const int tg = s0 / 2 + (rn / C::GSTAGES + 1) * C::GSTEPS;
-    uint8_t* sn = smem + C::SOFF + ((rn / C::GSTAGES + 1) & 1) * C::SSLOT;
-    issue_scales<C>(sn, ssr, P, tg, rn % C::GSTAGES == 0 && tg * STEP < hi);
-    const int q = (r + 5) >> 1;
-    issue_xhalf<C>(smem + (q % C::NS) * C::XSLOT, X, P, s0 + 2 * q, (r + 1) & 1, lo, hi);
-    issue_wstage<C>(smem + C::WOFF + (r % C::NS) * C::WBYTES, W, P, s0 + r + 3, lo, hi);
-  }
-  mfma_range<C, NE, NMMA, FIRST>(Fc, xc, wc, acc);
-  interleave_step<0, NMMA - NE, (NMMA - NE) / 2, NDS, TAIL == kXdFull ? C::LPS : 0>();
-  MXGG_SCHED_FENCE();
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  finish_scales<C>(xn, wn, s0 + rn, lo, hi);
-  hold(Fc, xc, wc);
-  MXGG_SCHED_FENCE();
-}
-
-// ring_mainloop for two-stage X slots (the same range, padding and ZSTART
-// meaning; a run of n stages runs n rounded up to even, at least 6).
-template <class C, bool ZSTART>
-__device__ __forceinline__ void ring_mainloop_xd(uint8_t* smem, const Operand& X, const Operand& W,
-                                                 const ScaleSrc& xss, const ScaleSrc& wss, int s0, int s1,
-                                                 int lo, int hi, v16f (&acc)[C::FM][C::FN]) {
-  if (s0 >= s1) s1 = s0 + 1;
-  s0 &= ~1;
-  Plan<C> P;
-  make_plan<C>(P, X, W, xss, wss);
-  const __amdgpu_buffer_rsrc_t ssr = wave_id() < C::NSX ? xss.rsrc : wss.rsrc;
-  issue_scales<C>(smem + C::SOFF, ssr, P, s0 / 2, true);
-  issue_scales<C>(smem + C::SOFF + C::SSLOT, ssr, P, s0 / 2 + C::GSTEPS, true);
-  issue_xhalf<C>(smem, X, P, s0, 0, lo, hi);
-  issue_xhalf<C>(smem, X, P, s0, 1, lo, hi);
-  issue_wstage<C>(smem + C::WOFF, W, P, s0, lo, hi);
-  issue_xhalf<C>(smem + C::XSLOT, X, P, s0 + 2, 0, lo, hi);
-  issue_xhalf<C>(smem + C::XSLOT, X, P, s0 + 2, 1, lo, hi);
-  issue_wstage<C>(smem + C::WOFF + C::WBYTES, W, P, s0 + 1, lo, hi);
-  issue_xhalf<C>(smem + 2 * C::XSLOT, X, P, s0 + 4, 0, lo, hi);
-  issue_wstage<C>(smem + C::WOFF + 2 * C::WBYTES, W, P, s0 + 2, lo, hi);
-  MXGG_WAIT_VM(3 * C::QX + 2 * C::QW);   // pair 0 and W stage 0 (and the scales before them)
-  MXGG_BARRIER();
-  Frags<C> Fa, Fb;
-  uint32_t xa[C::FM], wa[C::FN], xb[C::FM], wb[C::FN];
-  read_stage_xd<C>(smem, smem + C::WOFF, smem + C::SOFF, 0, 0, Fa, xa, wa);
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  finish_scales<C>(xa, wa, s0, lo, hi);
-  const int n = s1 - s0;
-  const int nr = n < 6 ? 6 : (n + 1) & ~1;
-  ring_stage_xd<C, ZSTART>(smem, X, W, ssr, P, s0, 0, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-#pragma nounroll
-  for (int r = 1; r < nr - 3; r += 2) {
-    ring_stage_xd<C>(smem, X, W, ssr, P, s0, r, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-    ring_stage_xd<C>(smem, X, W, ssr, P, s0, r + 1, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-  }
-  ring_stage_xd<C, false, kXdNoCopy1>(smem, X, W, ssr, P, s0, nr - 3, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-  ring_stage_xd<C, false, kXdNoCopy0>(smem, X, W, ssr, P, s0, nr - 2, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-  ring_stage_xd<C, false, kXdLast>(smem, X, W, ssr, P, s0, nr - 1, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-  MXGG_WAIT_VM(0);
-}
-
-// Reduction over the 64-element stages [s0, s1) restricted to the element
-// range [lo, hi) (chunks and scale blocks outside it are zero / neutral),
-// into acc.  ZSTART: the first stage's MFMAs start from zero, so acc needs no
-// clearing (256 accumulator writes per lane, which the compiler otherwise puts
-// between the tile set-up and the first copies, twice over when an empty range
-// has a path of its own); else the caller zeroes acc.  An empty range runs one
-// stage wholly outside [lo, hi).
-// The ring starts at the even stage s0 & ~1 so that scale groups cover whole
-// steps; an odd stage count runs one stage past s1.  Those extra stages are
-// wholly outside [lo, hi): zero data, neutral scales, exactly zero added.
-template <class C, bool ZSTART = true>
-__device__ __forceinline__ void ring_mainloop(uint8_t* smem, const Operand& X, const Operand& W,
-                                              const ScaleSrc& xss, const ScaleSrc& wss, int s0, int s1,
-                                              int lo, int hi, v16f (&acc)[C::FM][C::FN]) {
-  if constexpr (C::XD) {
-    ring_mainloop_xd<C, ZSTART>(smem, X, W, xss, wss, s0, s1, lo, hi, acc);
-  } else {
-    if (s0 >= s1) s1 = s0 + 1;
-    s0 &= ~1;
-    Plan<C> P;
-    make_plan<C>(P, X, W, xss, wss);
-    // the scale buffer this wave copies from (wave-uniform)
-    const __amdgpu_buffer_rsrc_t ssr = wave_id() < (C::PS ? C::NXW : C::NSX) ? xss.rsrc : wss.rsrc;
-    // scale groups 0 and 1, then stages s0 .. s0+NS-1 (scales first: every
-    // wait for a stage's copies then covers the scale copies issued before it)
-    const int g0 = C::PS ? (s0 & (C::GSTAGES - 1)) : 0;
-    const int tb = (s0 - g0) / 2;
-    issue_scales<C>(smem + C::SOFF, ssr, P, tb, true);
-    issue_scales<C>(smem + C::SOFF + C::SSLOT, ssr, P, tb + C::GSTEPS, true);
-  #pragma unroll
-    for (int i = 0; i < C::NS; ++i) issue_stage<C>(smem + i * C::STAGE, X, W, P, s0 + i, lo, hi);
-    MXGG_WAIT_VM((C::NS - 1) * C::LPS);
-    MXGG_BARRIER();
-    Frags<C> Fa, Fb;
-    uint32_t xa[C::FM], wa[C::FN], xb[C::FM], wb[C::FN];
-    read_stage<C>(smem, smem + C::SOFF, g0 / 2, Fa, xa, wa);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    finish_scales<C>(xa, wa, s0, lo, hi);
-    const int n = s1 - s0;
-    if constexpr (ZSTART) {
-      // stages run: n rounded up to even, at least 6 (those past s1 hold
-      // zeros); the last four start no copies (the prologue and the full
-      // stages already issued every stage of the run), the last reads nothing
-      const int nr = n < 6 ? 6 : (n + 1) & ~1;
-      ring_stage<C, true>(smem, X, W, ssr, P, s0, 0, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-      ring_stage<C>(smem, X, W, ssr, P, s0, 1, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-  #pragma nounroll
-      for (int r = 2; r < nr - 4; r += 2) {
-        ring_stage<C>(smem, X, W, ssr, P, s0, r, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-        ring_stage<C>(smem, X, W, ssr, P, s0, r + 1, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-      }
-      ring_stage<C, false, kStageNoCopy2>(smem, X, W, ssr, P, s0, nr - 4, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-      ring_stage<C, false, kStageNoCopy1>(smem, X, W, ssr, P, s0, nr - 3, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-      ring_stage<C, false, kStageNoCopy0>(smem, X, W, ssr, P, s0, nr - 2, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-      ring_stage<C, false, kStageLast>(smem, X, W, ssr, P, s0, nr - 1, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-    } else {
-  #pragma nounroll
-      for (int r = 0; r < n; r += 2) {
-        ring_stage<C>(smem, X, W, ssr, P, s0, r, lo, hi, Fa, xa, wa, Fb, xb, wb, acc);
-        ring_stage<C>(smem, X, W, ssr, P, s0, r + 1, lo, hi, Fb, xb, wb, Fa, xa, wa, acc);
-      }
+// MFMAs P0 .. of step t (relative to the run's first), with what is issued
+// beside each.  KIND: kStepFull also copies step t + 2 into this step's slot;
+// kStepNoCopy, the last but one, does not; kStepLast only multiplies.
+//   MFMA 0 .. RD-1:     read the second half step's fragments (F1)
+//   before MFMA PB1:    barrier: every wave has read this slot, so
+//   MFMA PB1 ..:        the copies of step t + 2 go into it, one per MFMA
+//   before MFMA PB2:    the copies of step t + 1 (older than the `issued`
+//                       ones of step t + 2) have landed; barrier
+//   MFMA PB2 ..:        read the first half step of step t + 1 (F0, free
+//                       since MFMA NMMA - 1) and its scales
+// A scheduling fence after every MFMA keeps the order.  With a wave alone on
+// its SIMD every other instruction between two MFMAs is issue time the matrix
+// core waits for: 256 x 256 e4m3 tiles issue about 150 per step of 32 MFMAs.
+constexpr int kStepFull = 0, kStepNoCopy = 1, kStepLast = 2;
+template <class C, int KIND, int P0>
+__device__ __forceinline__ void step_pos(uint8_t* smem, const Operand& X, const Operand& W, __amdgpu_buffer_rsrc_t ssr,
+                                         Plan<C>& P, int t, Frags<C>& F0, Frags<C>& F1, uint32_t (&xc)[C::FM],
+                                         uint32_t (&wc)[C::FN], uint32_t (&xn)[C::FM], uint32_t (&wn)[C::FN],
+                                         v16f (&acc)[C::FM][C::FN]) {
+  if constexpr (P0 < 2 * C::NMMA) {
+    constexpr int NF = C::FM + C::FN;
+    if constexpr (KIND == kStepFull && P0 == C::PB1) {
+      MXGG_WAIT_LGKM();
+      MXGG_BARRIER();
+      MXGG_SCHED_FENCE();
     }
-    // copies past the last stage (zero fills, scale groups) may still be
-    // writing LDS: drain them before the LDS is reused or released
-    MXGG_WAIT_VM(0);
+    if constexpr (KIND != kStepLast && P0 == C::PB2) {
+      constexpr int issued = KIND == kStepFull ? C::NC * (C::PB2 - C::PB1) / C::NMMA : 0;
+      MXGG_WAIT_VM(issued);
+      MXGG_BARRIER();
+      MXGG_SCHED_FENCE();
+    }
+    if constexpr (P0 < C::NMMA)
+      mfma1<C, P0, 0>(F0, xc, wc, acc);
+    else
+      mfma1<C, P0 - C::NMMA, 2>(F1, xc, wc, acc);
+    if constexpr (P0 < C::RD) read_frags<C, 1, P0 * NF / C::RD, (P0 + 1) * NF / C::RD>(smem, P, F1);
+    if constexpr (P0 == C::RD) toggle_reads<C, 1>(P);
+    if constexpr (KIND == kStepFull && P0 >= C::PB1 && P0 < C::PB1 + C::NMMA) {
+      constexpr int q = P0 - C::PB1;
+      if constexpr (q == 0) issue_scales<C>(ssr, P, t);
+      step_copies<C, q * C::NC / C::NMMA, (q + 1) * C::NC / C::NMMA>(X, W, P, CopyOff{P.xe, P.xo, P.we, P.wo});
+    }
+    if constexpr (KIND != kStepLast && P0 >= C::PB2 && P0 < C::PB2 + C::RD) {
+      constexpr int q = P0 - C::PB2;
+      read_frags<C, 0, q * NF / C::RD, (q + 1) * NF / C::RD>(smem, P, F0);
+      if constexpr (q == C::RD - 1) read_scales<C>(smem, P, t + 1, xn, wn);
+    }
+    MXGG_SCHED_FENCE();
+    step_pos<C, KIND, P0 + 1>(smem, X, W, ssr, P, t, F0, F1, xc, wc, xn, wn, acc);
   }
+}
+
+template <class C, int KIND>
+__device__ __forceinline__ void run_step(uint8_t* smem, const Operand& X, const Operand& W, __amdgpu_buffer_rsrc_t ssr,
+                                         Plan<C>& P, int t, Frags<C>& F0, Frags<C>& F1, uint32_t (&xc)[C::FM],
+                                         uint32_t (&wc)[C::FN], v16f (&acc)[C::FM][C::FN]) {
+  uint32_t xn[C::FM], wn[C::FN];
+  step_pos<C, KIND, 0>(smem, X, W, ssr, P, t, F0, F1, xc, wc, xn, wn, acc);
+  hold(F1, xc, wc);
+  if constexpr (KIND != kStepLast) {
+    toggle_reads<C, 0>(P);
+    shift_scales<C>(P, xn, wn, xc, wc);
+  }
+  MXGG_SCHED_FENCE();
+}
+
+// The plan's lane offsets moved on to the next step.
+template <class C>
+__device__ __forceinline__ void advance(Plan<C>& P, const Operand& X, const Operand& W) {
+  const uint32_t dx = (uint32_t)C::XROW << X.pl, dw = (uint32_t)C::WROW << W.pl;
+  P.xe += dx;
+  P.xo += dx;
+  P.we += dw;
+  P.wo += dw;
+}
+
+// acc = the reduction over the elements [lo, hi) (chunks and scale blocks
+// outside are zero / neutral), run as the whole 128-element steps it touches,
+// two at least (a step wholly outside adds zeros).  Steps alternate between
+// two LDS slots; while step t is multiplied, step t + 1 lies in the other slot
+// and the copies of step t + 2 go into t's own as soon as every wave has read
+// it, so they have about a step and a half to land.
+// Bound by power and MFMA issue: 256 x 256 e4m3 tiles, M = N = K = 8192, 2.9
+// PFLOP/s; 64-element stages in a 3- to 4-deep ring, whose 10 to 13
+// instructions per MFMA kept the matrix cores waiting, reached 2.45.
+template <class C>
+__device__ __forceinline__ void step_mainloop(uint8_t* smem, const Operand& X, const Operand& W, const ScaleSrc& xss,
+                                              const ScaleSrc& wss, int lo, int hi, v16f (&acc)[C::FM][C::FN]) {
+  lo = uniform(lo);
+  hi = uniform(hi);
+  const int t0 = lo / STEP;
+  int n = (hi + STEP - 1) / STEP - t0;   // steps of the run
+  if (n < 2) n = 2;
+  Plan<C> P;
+  make_plan<C>(P, smem, X, W, xss, wss, t0);
+  // the scale buffer this wave copies from (wave-uniform)
+  const __amdgpu_buffer_rsrc_t ssr =
+      (C::PS ? wave_id() < C::NXW : wave_id() % C::NSD < C::NSX) ? xss.rsrc : wss.rsrc;
+  // units of X (16 elements) and W (e2m1: 32) of a step inside [lo, hi): of
+  // the first step those from xlo / wlo on (and below its own end), of the
+  // last those below xhi / whi
+  constexpr int WE = C::F4 ? 32 : 16;
+  const int r0 = lo - t0 * STEP, h0 = hi - t0 * STEP, h1 = hi - (t0 + n - 1) * STEP;
+  const int xhi = h1 > 0 ? h1 / 16 : 0, whi = h1 > 0 ? h1 / WE : 0;
+  P.mxe = P.ux < xhi ? 0 : kOOB;
+  P.mxo = (P.ux ^ 1) < xhi ? 0 : kOOB;
+  P.mwe = P.uw < whi ? 0 : kOOB;
+  P.mwo = (C::F4 ? P.uw : P.uw ^ 1) < whi ? 0 : kOOB;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_nop 4" ::: "memory");   // scalar operands of the asm copies written by vector instructions
+#endif
+#pragma unroll
+  for (int i = 0; i < (C::PS ? C::SPW : 1); ++i) {   // scale group 0
+    set_m0(P.sm0 + (uint32_t)(i * 1024));
+    copy16<0>(ssr, P.sv, P.s_step * (uint32_t)i);
+  }
+  step_copies<C, 0, C::NC>(X, W, P, mask_copies<C>(P, (r0 + 15) / 16, h0 / 16, (r0 + WE - 1) / WE, h0 / WE));
+  P.xm0 ^= (uint32_t)C::XBYTES;
+  P.wm0 ^= (uint32_t)C::WBYTES;
+  advance<C>(P, X, W);
+  mask_last<C>(P, 1, n);
+  step_copies<C, 0, C::NC>(X, W, P, CopyOff{P.xe, P.xo, P.we, P.wo});
+  MXGG_SCHED_FENCE();
+  zero_acc<C>(acc);      // while the copies fly
+  MXGG_SCHED_FENCE();
+  MXGG_WAIT_VM(C::NC);
+  MXGG_BARRIER();
+  Frags<C> F0, F1;
+  uint32_t xc[C::FM], wc[C::FN];
+  read_frags<C, 0, 0, C::FM + C::FN>(smem, P, F0);
+  toggle_reads<C, 0>(P);
+  {
+    uint32_t xn[C::FM], wn[C::FN];
+    read_scales<C>(smem, P, 0, xn, wn);
+    shift_scales<C>(P, xn, wn, xc, wc);
+  }
+  mask_scales<C>(P, t0, lo, hi, xc, wc);
+  MXGG_SCHED_FENCE();
+  int t = 0;
+#pragma nounroll
+  for (; t < n - 2; ++t) {
+    advance<C>(P, X, W);
+    mask_last<C>(P, t + 2, n);
+    P.xm0 ^= (uint32_t)C::XBYTES;
+    P.wm0 ^= (uint32_t)C::WBYTES;
+    run_step<C, kStepFull>(smem, X, W, ssr, P, t, F0, F1, xc, wc, acc);
+  }
+  pin_acc<C>(acc);
+  run_step<C, kStepNoCopy>(smem, X, W, ssr, P, t, F0, F1, xc, wc, acc);
+  mask_scales<C>(P, t0 + n - 1, lo, hi, xc, wc);
+  run_step<C, kStepLast>(smem, X, W, ssr, P, t + 1, F0, F1, xc, wc, acc);
+  pin_acc<C>(acc);
 }
 
 // The in-range elements of the 16-element chunk at cs (a multiple of 16)
-// that straddles a bound of the reduction range [lo, hi).  The ring copies
+// that straddles a bound of the reduction range [lo, hi).  The main loop copies
 // whole chunks only, so a bound that is not a multiple of 16 leaves these
 // out; they are added here as one more 64-element MFMA step whose fragments
 // are loaded into registers, every element outside [lo, hi) and every other
-// chunk of the step zero.  MFMA operand layout (the one read_stage builds):
+// chunk of the step zero.  MFMA operand layout (the one read_frags builds):
 // lane half h holds elements 16h .. 16h+15 of the step in dwords 0-3 and
 // 32+16h .. 32+16h+15 in dwords 4-7, and supplies the scale of the step's
 // block h (elements 32h .. 32h+31).  e4m3 on both sides (the weight
@@ -942,7 +782,7 @@ __device__ __forceinline__ void edge_chunk(const Operand& X, const Operand& W, c
   const int lane = threadIdx.x % kWave;
   const int wm = wave / C::WGN, wn = wave % C::WGN;
   const int h = lane >> 5, r32 = lane & 31;
-  const int kb = cs & ~(BKS - 1);                  // the step holding the chunk
+  const int kb = cs & ~(HALF - 1);                 // the half step holding the chunk
   const int ci = (cs - kb) >> 4;                   // chunk of the step: half (ci & 1), dwords 4 (ci >> 1) ..
   const bool mine = h == (ci & 1);
   // bytes b of the chunk with lo <= cs + b < hi
@@ -992,7 +832,12 @@ __device__ __forceinline__ void edge_chunk(const Operand& X, const Operand& W, c
     const uint32_t s = __builtin_amdgcn_raw_buffer_load_b32(wss.rsrc, ((uint32_t)t * wss.rows + wss.row0 + row) * 4u, 0, 0);
     ws[j] = live ? (s >> (8 * blk)) & 0xffu : 127u;
   }
-  mfma_range<C, 0, C::FM * C::FN>(F, xs, ws, acc);
+#pragma unroll
+  for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j)
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(F.a[j], F.b[i], acc[i][j], C::WFMT, MXGG_FMT_E4M3, 0,
+                                                                   (int)ws[j], 0, (int)xs[i]);
   hold(F, xs, ws);
   // What follows (a second edge step, the epilogue) may reuse these operand
   // registers at once; the compiler does not count the scale operands as
@@ -1445,24 +1290,17 @@ __device__ __forceinline__ void fwd_tile_run(const FwdParams& p, uint8_t* smem, 
   const ScaleSrc ws{make_rsrc(p.bs + (int64_t)tl.expert * p.bs_expert, p.bs_expert), C::PS ? p.bs_ld : (uint32_t)p.N,
                     (uint32_t)n0};
 
-  v16f acc[C::FM][C::FN];   // set by ring_mainloop
+  v16f acc[C::FM][C::FN];   // set by step_mainloop
   const int K = (int)p.K;
   if constexpr (PIECES) {
     int a, b;
     split_range(0, (int)((p.K + STEP - 1) / STEP), piece, S, a, b);
     const int lo = STEP * a;
     const int hi = STEP * b < K ? STEP * b : K;
-    ring_mainloop<C>(smem, X, W, xs, ws, lo / BKS, (hi + BKS - 1) / BKS, lo, hi, acc);
+    step_mainloop<C>(smem, X, W, xs, ws, lo, hi, acc);
     store_partial<C>(acc, p.part + (int64_t)slot * (C::BM * C::BN));
   } else {
-    // the f32 epilogue's register allocation spills when the first stage is
-    // peeled: it keeps the accumulators zeroed up front
-    if constexpr (EPI == kEpiF32) {
-      zero_acc<C>(acc);
-      ring_mainloop<C, false>(smem, X, W, xs, ws, 0, (K + BKS - 1) / BKS, 0, K, acc);
-    } else {
-      ring_mainloop<C>(smem, X, W, xs, ws, 0, (K + BKS - 1) / BKS, 0, K, acc);
-    }
+    step_mainloop<C>(smem, X, W, xs, ws, 0, K, acc);
     if constexpr (EPI == kEpiBf16) {
       store_tile_lds<C, true>(acc, smem, p.out + (row0 * p.ldo + n0) * 2, p.ldo, rows, cols);
     } else if constexpr (EPI == kEpiF16) {
@@ -1943,7 +1781,7 @@ __global__ __launch_bounds__(C::NT) void wgrad_kernel(WgradParams p) {
 
   v16f acc[C::FM][C::FN];
   if (hi > lo)
-    ring_mainloop<C>(smem, X, W, xs, ws, lo / BKS, (hi + BKS - 1) / BKS, lo, hi, acc);
+    step_mainloop<C>(smem, X, W, xs, ws, lo, hi, acc);
   else
     zero_acc<C>(acc);
   // group bounds that are not multiples of 16 (any offsets are accepted, as
@@ -2088,25 +1926,20 @@ static size_t fwd_staging_bytes_a(int64_t M, int64_t N, int64_t K, int b_fmt) {
 
 namespace {
 
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 4> CfgF8_256;
-typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 4> CfgF8_128;
-// e2m1 weights: stages of 24 KB in a 4-deep ring, like e4m3 (a 5-deep ring
-// measured the same on BASELINE config 5, 650 vs 651 us, and spilled 8 bytes
-// per lane in the LDS-staged epilogues)
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 4> CfgF4_256;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 2> CfgF8_256;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 2> CfgF8_128;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 2> CfgF4_256;
 // The same tiles on plain to_mx scales (drop-in calls whose scale rows are
 // 16-byte multiples): no scale re-layout launch; 16 KB scale slots of 8 steps
 // (8 KB for 128 x 128 tiles).
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 4, true> CfgF8_256P;
-typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 4, true> CfgF8_128P;
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 4, true> CfgF4_256P;
-// 256 x 256 e4m3 tiles with X in two-stage slots, for row-major X (XLine)
-typedef XLine<Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 3>> CfgF8_256X;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 2, true> CfgF8_256P;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 2, true> CfgF8_128P;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 2, true> CfgF4_256P;
 
 // The scale-independent kernels of a configuration (the reduce): its
 // step-major twin.
 template <class C>
-using StepCfg = Cfg<C::BM, C::BN, C::WGM, C::WGN, C::WFMT, C::XD ? 4 : C::NS>;
+using StepCfg = Cfg<C::BM, C::BN, C::WGM, C::WGN, C::WFMT, C::NS>;
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -2232,8 +2065,7 @@ int launch_fwd(const FwdParams& p0, int grid_m_ub, int gm, int xcd, size_t part_
   // quarter tiles (quad_dp).  The device decides from the real tile count;
   // the host, from the usual one, only skips the launch where it cannot help.
   p.quads = 0;
-  constexpr bool kQuads = std::is_same<C, CfgF8_256>::value || std::is_same<C, CfgF8_256P>::value ||
-                          std::is_same<C, CfgF8_256X>::value;
+  constexpr bool kQuads = std::is_same<C, CfgF8_256>::value || std::is_same<C, CfgF8_256P>::value;
   typedef typename std::conditional<C::PS, CfgF8_128P, CfgF8_128>::type Q;
   if constexpr (kQuads) {
     if (nsteps < kMinSplitTotal && p.par > 0) {
@@ -2579,7 +2411,6 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
     return launch_fwd<CfgF8_128P>(p, gm128, c.group_m, c.xcd, pb, st);
   }
   if (b_fmt == MXGG_FMT_E2M1) return launch_fwd<CfgF4_256>(p, gm256, c.group_m, c.xcd, pb, st);
-  if (c.bm == 256 && p.a_pl == 0) return launch_fwd<CfgF8_256X>(p, gm256, c.group_m, c.xcd, pb, st);
   if (c.bm == 256) return launch_fwd<CfgF8_256>(p, gm256, c.group_m, c.xcd, pb, st);
   return launch_fwd<CfgF8_128>(p, gm128, c.group_m, c.xcd, pb, st);
 }
@@ -2881,14 +2712,11 @@ static WgradChoice wgrad_choice(int E, int64_t M, int64_t N, int64_t K, int64_t 
 
 // The wgrad launches of a checked call on step-major scales (gs: GO [T][N],
 // is: IA [T][K] dwords); part / part_bytes: room for the fp32 partial tiles
-// of tiles cut along the tokens (none: no tile is cut).  C: the 256 x 256
-// configuration (XLine where GO, the X side, is row-major); the plan, the
-// partial layout and the reduce are the one-stage configuration's, so both
-// give the same bits.
-template <class C>
-static int launch_wgrad_c(const uint8_t* go_t, int64_t ld_go, const uint8_t* gs, const uint8_t* ia_t, int64_t ld_ia,
-                          const uint8_t* is, const int32_t* offs, int E, int64_t M, int64_t N, int64_t K, void* out,
-                          int out_dtype, int layout, void* part_area, size_t part_bytes, hipStream_t st) {
+// of tiles cut along the tokens (none: no tile is cut).
+static int launch_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* gs, const uint8_t* ia_t, int64_t ld_ia,
+                        const uint8_t* is, const int32_t* offs, int E, int64_t M, int64_t N, int64_t K, void* out,
+                        int out_dtype, int layout, void* part_area, size_t part_bytes, hipStream_t st) {
+  typedef CfgF8_256 C;
   const int64_t T = cdiv(M, STEP);
   // no more room than the split plans of this shape can use (ws_layout)
   const size_t cap = wgrad_part_cap(E, M, N, K);
@@ -2940,16 +2768,6 @@ static int launch_wgrad_c(const uint8_t* go_t, int64_t ld_go, const uint8_t* gs,
   hipLaunchKernelGGL((wgrad_reduce_kernel<StepCfg<C>>), dim3((unsigned)(split_tiles_ub * ReduceShape<C>::CH)),
                      dim3(256), 0, st, p);
   return launch_status("wgrad");
-}
-
-static int launch_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* gs, const uint8_t* ia_t, int64_t ld_ia,
-                        const uint8_t* is, const int32_t* offs, int E, int64_t M, int64_t N, int64_t K, void* out,
-                        int out_dtype, int layout, void* part_area, size_t part_bytes, hipStream_t st) {
-  if (layout & MXGG_A_PAIRS)
-    return launch_wgrad_c<CfgF8_256>(go_t, ld_go, gs, ia_t, ld_ia, is, offs, E, M, N, K, out, out_dtype, layout,
-                                     part_area, part_bytes, st);
-  return launch_wgrad_c<CfgF8_256X>(go_t, ld_go, gs, ia_t, ld_ia, is, offs, E, M, N, K, out, out_dtype, layout,
-                                    part_area, part_bytes, st);
 }
 
 extern "C" int mxgg_wgrad_config(int E, int64_t M, int64_t N, int64_t K, int* block) {
