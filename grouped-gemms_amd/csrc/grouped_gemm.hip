@@ -432,8 +432,8 @@ template <class C>
 __device__ __forceinline__ void issue_scales(__amdgpu_buffer_rsrc_t ssr, const Plan<C>& P, int t) {
   const int g = t / C::GSTEPS + 1;
   const uint32_t i = C::PS ? (uint32_t)((t / 2) % (C::PS ? C::SPW : 1)) : 0u;
-  const uint32_t m0 = P.sm0 + (uint32_t)((g & 1) * C::SSLOT) + i * 1024u;
-  const uint32_t so = C::PS ? P.s_step * i + (uint32_t)(g * 32) : P.s_step * (uint32_t)(g * C::GSTEPS);
+  [[maybe_unused]] const uint32_t m0 = P.sm0 + (uint32_t)((g & 1) * C::SSLOT) + i * 1024u;
+  [[maybe_unused]] const uint32_t so = C::PS ? P.s_step * i + (uint32_t)(g * 32) : P.s_step * (uint32_t)(g * C::GSTEPS);
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile(
       "s_bitcmp1_b32 %0, 0\n\t"

@@ -21,6 +21,9 @@
 // The e4m3 cast is the hardware fp8 conversion of the clamped, exactly
 // scaled value (round to nearest even); blocks holding a NaN take the
 // bit-level path, which keeps the NaN's sign as the reference's cast does.
+// The e2m1 cast likewise (the bit-level one took about 20 vector instructions
+// per element and bound the kernel: (8, 2048, 5120) bf16 86 us = 2.5 TB/s,
+// now 46 us = 4.6 TB/s).
 //
 // Scales go out in the reference's plain layout (row-major (rows, blocks)
 // bytes) or step-major, the layout the GEMM kernels read (MXGG_SCALES_STEPS:
@@ -173,6 +176,30 @@ __device__ __forceinline__ uint32_t e4m3x4_sw(float a, float b, float c, float d
   return e4m3_code(a, mul) | (e4m3_code(b, mul) << 8) | (e4m3_code(c, mul) << 16) | (e4m3_code(d, mul) << 24);
 }
 
+// e2m1 codes of 8 values (nibble i: v[i]): clamp(v * mul, -6, 6) rounded to
+// nearest even by the hardware fp4 conversion (scale 1: the product is
+// already scaled, exactly), for every input but NaN, which the caller routes
+// to e2m1x8_sw.
+__device__ __forceinline__ uint32_t e2m1x8(const float (&v)[8], float mul) {
+  float y[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) y[i] = __builtin_amdgcn_fmed3f(v[i] * mul, -6.f, 6.f);
+  uint32_t w = 0;
+  w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, y[0], y[1], 1.f, 0);
+  w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, y[2], y[3], 1.f, 1);
+  w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, y[4], y[5], 1.f, 2);
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, y[6], y[7], 1.f, 3);
+}
+
+// The same eight codes by the bit-level conversion (any input, NaN included:
+// it saturates with its sign).
+__device__ __forceinline__ uint32_t e2m1x8_sw(const float (&v)[8], float mul) {
+  uint32_t w = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w |= e2m1_code(v[i], mul) << (4 * i);
+  return w;
+}
+
 // max |x| bit pattern of n fp32 values (NaN above inf, as the reference's amax
 // propagates NaN).
 template <int N>
@@ -256,9 +283,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const uint8_t* __restri
         if (pl && (bpr & 1) && cb == bpr - 1)
           *reinterpret_cast<uint2*>(q + q_off(r, col + 32, ld_q, pl)) = make_uint2(0, 0);
       } else {
-        uint32_t w = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) w |= e2m1_code(v[i], mul) << (4 * i);
+        const uint32_t w = m > 0x7f800000u ? e2m1x8_sw(v, mul) : e2m1x8(v, mul);
         *reinterpret_cast<uint32_t*>(q + q_off(r, col / 2, ld_q, pl)) = w;
         // row quads, odd block count: the last block's lanes zero the pad
         if (pl && (bpr & 1) && cb == bpr - 1) *reinterpret_cast<uint32_t*>(q + q_off(r, col / 2 + 16, ld_q, pl)) = 0u;

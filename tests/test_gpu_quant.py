@@ -84,6 +84,23 @@ def test_quant_e2m1_special(gpu):
     _check_rows(_special_blocks().to(torch.bfloat16), gpu, elem="e2m1")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_quant_e2m1_every_bf16_pattern(gpu, dtype):
+    """The hardware fp4 conversion against the oracle's rounding, bit for bit:
+    all 65536 bf16 patterns (NaN blocks included), and every tie of the e2m1
+    grid with its fp32 neighbours, both signs."""
+    rng = np.random.default_rng(4)
+    u = rng.permutation(np.arange(65536, dtype=np.uint16))
+    x = torch.from_numpy(u.view(np.int16).copy()).view(torch.bfloat16).reshape(512, 128)
+    _check_rows(x.to(dtype), gpu, elem="e2m1")
+    # finite values of one binade range, so that every block rounds on the grid
+    f = np.array([0.25, 0.5, 0.75, 1.0, 1.25, 1.5, 1.75, 2.0, 2.5, 3.0, 3.5, 4.0, 5.0, 6.0, 7.0, 7.9], np.float32)
+    f = np.concatenate([np.nextafter(f, np.float32(0)), f, np.nextafter(f, np.float32(8))])
+    f = np.concatenate([f, -f, f * np.float32(2.0 ** -20), np.zeros(16, np.float32)])
+    x = torch.from_numpy(np.stack([np.concatenate([rng.permutation(f)[:31], [4.0]]) for _ in range(512)]).astype(np.float32))
+    _check_rows(x.to(dtype), gpu, elem="e2m1")
+
+
 @pytest.mark.parametrize("shape", [(1024, 512), (64, 256), (2048, 40)])
 def test_quant_dim0_matches_transposed_rows(gpu, shape):
     import kernels
