@@ -1117,10 +1117,12 @@ __device__ __forceinline__ void pair_chunks(const PairJob& J, int w) {
 }
 
 // 64 rows x 16 steps per workgroup (256 threads): each thread reads 16
-// source bytes of one row (4 steps; one 16-byte load when the chunk is
-// aligned and inside the row), the tile is transposed through LDS, and each
-// thread writes the dwords of 4 consecutive rows for one step (one 16-byte
-// store when aligned and inside the operand).
+// source bytes of one row (4 steps; one 16-byte load, aligned or not, where
+// the chunk lies inside the row -- rows of K/32 = 90 or M/32 = 65, 520 bytes
+// are common, and byte loads took 14.9 us for E = 32, M = 16640, N = K = 2880
+// where this takes 9.3), the tile is transposed through LDS, and each thread
+// writes the dwords of 4 consecutive rows for one step (one 16-byte store
+// when aligned and inside the operand).
 __global__ __launch_bounds__(256) void scale_relayout_kernel(ScaleJobs js) {
   __shared__ uint32_t tile[16][65];
   int bid = blockIdx.x;
@@ -1147,9 +1149,8 @@ __global__ __launch_bounds__(256) void scale_relayout_kernel(ScaleJobs js) {
     uint32_t v[4] = {0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu};
     if (r < J.rows && blk0 < J.nblk) {
       const uint8_t* src = J.src + (int64_t)b * J.ld_b + (int64_t)r * J.ld_r + blk0;
-      if (blk0 + 16 <= J.nblk && ((uintptr_t)src & 15) == 0) {
-        const uint4 q = *(const uint4*)src;
-        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+      if (blk0 + 16 <= J.nblk) {
+        __builtin_memcpy(v, src, 16);   // one 16-byte load at any alignment
       } else {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -1904,9 +1905,26 @@ static size_t fwd_staging_bytes(int E, int64_t M, int64_t N, int64_t K, int b_fm
   return (size_t)E * (size_t)N * (size_t)staged_ld(K) + 256;
 }
 
-// Forward calls of at most this many multiply-adds (1.2e11 flop) that stage
-// nothing run on plain scales without a re-layout launch (run_grouped_mm).
+// Forward calls above this many multiply-adds (1.2e11 flop) may have A staged.
 constexpr int64_t kPlainMaxMacs = (int64_t)60000000000;
+
+// Whether a forward call that stages nothing runs on plain scales (where
+// plain_scales_ok) instead of after a scale re-layout launch.  The plain-scale
+// kernels copy their scales in 32-byte row pieces, four times the requests of
+// the step-major dwords: about 5% of the GEMM's time.  The launch takes about
+// 4.5 us and 2 (M + E N) K / 32 bytes at 4 TB/s.  The GEMM is priced at 2.3
+// PFLOP/s or, with few rows per expert, at one read of the weight at 5 TB/s.
+// Measured (MI355X, whole calls, re-laid / plain scales): (32, 2048, 8192,
+// 8192) 449 / 434 us, (1, 16640, 2048, 2048) 79.0 / 77.3, (8, 4096, 4096,
+// 4096) 99.0 / 98.3; past the line (8, 16640, 2048, 5120) 187 / 189, (8,
+// 16640, 8192, 5120) e2m1 552 / 564, (4, 16640, 8192, 8192) 885 / 900.
+static bool plain_pays(int E, int64_t M, int64_t N, int64_t K, int b_fmt) {
+  const double macs = (double)M * (double)N * (double)K;
+  const double weight = (double)E * (double)N * (double)K * (b_fmt == MXGG_FMT_E2M1 ? 0.5 : 1.0);
+  const double gemm = macs / 1.15e6 > weight / 5e3 ? macs / 1.15e6 : weight / 5e3;   // ns
+  const double relayout = 4500.0 + ((double)M + (double)E * (double)N) * (double)K / 16.0 / 4e3;
+  return 0.05 * gemm <= relayout;
+}
 
 // The same for A (M, K), or 0: its copy's time over the GEMM's is about
 // 400 / N, and staging it paid at N >= 8192 on every sweep shape (drop-in
@@ -2442,16 +2460,7 @@ static int run_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* A_s, int
   const bool staged_a = T > 0 && stage_a && wl.extra >= used_b + stage_a;
   if (staged_a)
     pa = PairJob{A, lda, 0, (uint8_t*)align256((size_t)(end - used_b - stage_a)), ldp, (int)(M / 2), 1, (int)K};
-  // The plain-scale kernels save the scale re-layout launch (4.4 us at the
-  // least, a quarter of the smallest expert-parallel shard call) but copy
-  // their scales in 32-byte row pieces, four times the copy requests of the
-  // step-major dwords, which slows the main loop by about 3%.  Measured on
-  // MI355X (drop-in forward, same bits either way): E = 1, M = 2080 calls of
-  // 1.7e10 .. 1.1e11 flop -13 to -1.5%, 1.7e11 +0.6 to +2.6%, and the
-  // 36-shape sweep (1.4e11 flop and up) +2.7% geomean.  So they run on calls
-  // that stage nothing (staging launches the re-layout kernel anyway) of at
-  // most kPlainMaxMacs multiply-adds.
-  const bool plain = !staged_a && !staged_b && M * N <= kPlainMaxMacs / (K > 0 ? K : 1) &&
+  const bool plain = !staged_a && !staged_b && plain_pays(E, M, N, K, b_fmt) &&
                      plain_scales_ok(A_s, ldas, B_s, ldbs_n, ldbs_e, E, M, N);
   if (T > 0 && !plain) {
     if (int rc = launch_relayout(scale_job(A_s, ldas, 0, wsd, M, 1, K / 32, T),
@@ -2515,12 +2524,10 @@ extern "C" int mxgg_grouped_mm_steps(const uint8_t* A, int64_t lda, const uint32
 
 // MXGG_NOALLOC_SCRATCH_BYTES per device, held from the library's load to the
 // end of the process: the re-laid scales of a call (4 * cdiv(K, 128) *
-// (M + E*N) bytes; 21 MB for the largest sweep shape), after them the fp32
-// partial tiles of a split last round, and, at the end, a weight staged in
-// row pairs when that fits as well (as for a caller's workspace of this
-// size).  Nothing in it needs clearing: every call writes the scales and the
-// staged weight before reading them, and a split call writes every partial
-// tile before the reduce reads it.
+// (M + E*N) bytes; 21 MB for the largest sweep shape) and after them the fp32
+// partial tiles of a split last round.  Nothing in it needs clearing: every
+// call writes the scales before reading them, and a split call writes every
+// partial tile before the reduce reads it.
 static __device__ __align__(256) uint8_t scratch[MXGG_NOALLOC_SCRATCH_BYTES];
 
 namespace {
@@ -2569,9 +2576,12 @@ extern "C" int mxgg_grouped_mm_noalloc(const uint8_t* A, int64_t lda, const uint
   if (int rc = require_device()) return rc;
   void* ws = nullptr;
   if (int rc = scratch_for_device(&ws)) return rc;
+  // the recommended size where it fits: no operand is staged (the copy costs
+  // more than it saves)
+  size_t bytes = mxgg_grouped_mm_workspace_size(E, M, N, K);
+  if (bytes > (size_t)MXGG_NOALLOC_SCRATCH_BYTES) bytes = (size_t)MXGG_NOALLOC_SCRATCH_BYTES;
   return run_grouped_mm(A, lda, A_s, ldas, B, b_fmt, ldb_n, ldb_e, B_s, ldbs_n, ldbs_e, offs, E, M, N, K, out,
-                        out_dtype, ldo, block_m, block_n, group_m, xcd, ws, (size_t)MXGG_NOALLOC_SCRATCH_BYTES,
-                        stream);
+                        out_dtype, ldo, block_m, block_n, group_m, xcd, ws, bytes, stream);
 }
 
 extern "C" int mxgg_grouped_mm_config(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int* block_m,

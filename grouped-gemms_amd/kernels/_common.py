@@ -43,13 +43,15 @@ def _rowmajor(t: torch.Tensor) -> torch.Tensor:
 
 
 def _staging_enabled() -> bool:
-    """False when the environment sets ``MXGG_STAGING=0``: the drop-in calls
-    then allocate no room for copying operands into row pairs (less transient
-    memory per call -- up to E*N*K + M*K bytes for the forward, (N + K)*M for
-    wgrad -- at the cost of the GEMM reading row-major operands; the output
-    bits are the same).  Read per call."""
+    """True when the environment sets ``MXGG_STAGING=1``: the drop-in calls
+    then allocate room for copying operands into row pairs (up to E*N*K + M*K
+    bytes for the forward, (N + K)*M for wgrad).  The GEMM copies row-major
+    operands in whole cache lines, so the copy costs more than it saves
+    (MI355X, whole calls, unstaged / staged: dgrad (4, 16640, 8192, 8192) 931 /
+    940 us, forward (8, 16640, 8192, 5120) 613 / 645, wgrad (4, 16640, 8192,
+    8192) 900 / 962); the output bits are the same.  Read per call."""
     import os
-    return os.environ.get("MXGG_STAGING", "1") != "0"
+    return os.environ.get("MXGG_STAGING", "0") not in ("", "0")
 
 
 _OUT_CODES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,

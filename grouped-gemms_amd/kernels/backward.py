@@ -7,10 +7,9 @@ tokens), one reduction over each group's token range, output ``(E, N, K)``.
 As in the reference the stored values are rounded to bf16 whatever
 ``out_dtype`` is (backward.py:101-104, 214, 251: float32 holds the bf16
 value, float16 the bf16 value converted to half) and an empty group yields
-zeros.  On plain scales the call's re-layout launch also copies both operands
-into row pairs where the GEMM gains more than the copy costs
-(``mxgg_wgrad_staging_size``; same bits; ``MXGG_STAGING=0`` in the
-environment leaves that room out).  Step-major int32 scales (``(T, N)`` and ``(T, K)``, ``T = cdiv(M, 128)``, as
+zeros.  On plain scales a launch re-lays them first; with ``MXGG_STAGING=1`` in
+the environment it also copies both operands into row pairs
+(``mxgg_wgrad_staging_size``; same bits).  Step-major int32 scales (``(T, N)`` and ``(T, K)``, ``T = cdiv(M, 128)``, as
 ``to_mx_dim0(..., scale_layout="steps")`` writes them) skip the per-call
 re-layout (``mxgg_wgrad_steps``); with them either operand may be in row pairs
 (the view ``(N/2, 2, cdiv(M, 64), 64)``, resp. ``(K/2, ...)``, that
@@ -112,8 +111,7 @@ def triton_mxfp8_wgrad(
         return out
     gs = _u8(_rowmajor(go_scale))
     as_ = _u8(_rowmajor(ia_scale))
-    # plus room to stage both operands in row pairs where that pays for its
-    # copy (none with MXGG_STAGING=0)
+    # plus, with MXGG_STAGING=1, room to stage both operands in row pairs
     if _staging_enabled():
         ws_bytes += lib.mxgg_wgrad_staging_size(E, M, N, K)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None

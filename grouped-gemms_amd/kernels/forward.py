@@ -4,15 +4,13 @@ Drop-in for kernels/forward.py:461-606 of the reference: same name,
 positional order, defaults and return value.  ``output[s:e] = A[s:e] @ B[g]^T``
 per expert group, MX scales per 32 elements of K, fp32 accumulation, one
 rounding to ``out_dtype``.  The work runs in the hand-written HIP kernels of
-libmxgg (``mxgg_grouped_mm``): a scale re-layout launch (which also copies an
-e4m3 weight and / or the activations into row pairs where the GEMM gains more
-than the copy costs, ``mxgg_grouped_mm_staging_size``; same bits), then the
-GEMM, which builds the expert->tile routing inside the kernel from
+libmxgg (``mxgg_grouped_mm``): a scale re-layout launch (small calls need
+none), then the GEMM, which builds the expert->tile routing inside the kernel from
 ``group_end_offsets`` (no host sync), and, when the last round of tiles is
 split along K, the piece and reduce launches.  The per-call workspace (torch's
-caching allocator) holds the re-laid scales, up to 128 MiB of fp32 partial
-tiles and the staged operands; ``MXGG_STAGING=0`` in the environment leaves
-the staging room out.
+caching allocator) holds the re-laid scales and up to 128 MiB of fp32 partial
+tiles; ``MXGG_STAGING=1`` in the environment adds room for the library to copy
+operands into row pairs first (``mxgg_grouped_mm_staging_size``; same bits).
 
 Beyond the reference, the weight may be MXFP4: ``weight`` of dtype
 ``torch.float4_e2m1fn_x2`` (or uint8) with last dim K/2, two e2m1 values per
@@ -188,8 +186,7 @@ def triton_mxfp8_grouped_mm(
         return out
     a_s = _u8(_rowmajor(input_act_scales))
     b_s = _u8(_rowmajor(weight_scales))
-    # plus room to stage the weight and / or A in row pairs where that pays
-    # for its copy (none with MXGG_STAGING=0)
+    # plus, with MXGG_STAGING=1, room to stage the weight and / or A in row pairs
     if _staging_enabled():
         ws_bytes += lib.mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None

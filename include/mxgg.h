@@ -230,12 +230,14 @@ int mxgg_grouped_mm_config(int E, int64_t M, int64_t N, int64_t K, int b_fmt, in
  *            past the scales and that partial room hold the staged operands:
  *            with at least mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt) of
  *            them, an e4m3 B and / or A is first copied into row pairs at the
- *            end of the workspace (in the scale re-layout launch), which the
- *            GEMM reads in whole 128-byte lines.  A workspace of exactly the
- *            recommended size stages nothing; staging never takes room from the
+ *            end of the workspace (in the scale re-layout launch).  The GEMM
+ *            copies whole 128-byte lines of row-major operands too, so the copy
+ *            costs more than it saves (1-5% of a call measured).  A workspace of
+ *            exactly the recommended size stages nothing; staging never takes room from the
  *            partial tiles, and the output bits are the same either way.
- *            A call that stages nothing, of at most 1.2e11 flop (2*M*N*K), on
- *            scales whose rows and expert strides are 16-byte multiples at
+ *            A call that stages nothing, where the GEMM is small against the
+ *            re-layout of its scales (up to about 2e11 flop, more with few
+ *            rows per expert), on scales whose rows and expert strides are 16-byte multiples at
  *            16-byte aligned addresses, reads the plain scales directly (no
  *            re-layout launch; the scale room of the workspace is still
  *            required and left unused): the same bits.
@@ -290,9 +292,8 @@ int mxgg_grouped_mm_steps(const uint8_t* A, int64_t lda, const uint32_t* A_ss,
  * mxgg_grouped_mm without a workspace: no counterpart in the reference.  For
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid allocation).  Same arguments,
- * results and errors as mxgg_grouped_mm given a workspace of
- * MXGG_NOALLOC_SCRATCH_BYTES bytes (operands are staged only where the
- * scales, the full partial room and the staging all fit in it); the
+ * results and errors as mxgg_grouped_mm given a workspace of the recommended
+ * size, MXGG_NOALLOC_SCRATCH_BYTES bytes at most (no operand is staged); the
  * workspace is instead a device array
  * inside this library, one per GPU, allocated when the library is loaded and
  * held until the process ends.  Calls it cannot take -- the re-laid scales,
@@ -333,18 +334,17 @@ int mxgg_grouped_mm_noalloc(const uint8_t* A, int64_t lda, const uint8_t* A_s, i
  *         is not used for partial tiles.  With mxgg_wgrad_staging_size(E, M,
  *         N, K) bytes past the scales and that room, go_t and ia_t are first
  *         copied into row pairs at the end of the workspace (in the scale
- *         re-layout launch) and the GEMM reads whole 128-byte lines of them;
- *         the recommended size alone stages nothing, the partial tiles keep
+ *         re-layout launch), which costs more than it saves (7-9% of a call
+ *         measured); the recommended size alone stages nothing, the partial tiles keep
  *         their room, and the output bits are the same either way.
  */
 size_t mxgg_wgrad_workspace_size(int E, int64_t M, int64_t N, int64_t K);
 /*
  * Workspace bytes, on top of mxgg_wgrad_workspace_size, with which mxgg_wgrad
  * stages both operands in row pairs ((N + K) * M rounded up to 64, plus 512),
- * or 0 where the copy would not pay for itself: it is offered only for N and
- * K both at least 8192, or with E >= 8 groups for N + K >= 10240 (elsewhere
- * the GEMM reads row-major go_t in whole lines, XLine), and never for odd N
- * or K or for M not a multiple of 32.  No counterpart in the reference.
+ * or 0: it is offered only for N and K both at least 8192, or with E >= 8
+ * groups for N + K >= 10240, and never for odd N or K or for M not a multiple
+ * of 32.  No counterpart in the reference.
  */
 size_t mxgg_wgrad_staging_size(int E, int64_t M, int64_t N, int64_t K);
 /*
