@@ -959,15 +959,17 @@ __device__ __forceinline__ void store_partial(const v16f (&acc)[C::FM][C::FN], f
     }
 }
 
-// Store a 16-bit (bf16 / f16) accumulator tile through LDS so that every
-// global store instruction writes whole row segments: each wave transposes its
-// WTM x WTN tile into its own LDS area (rows of WTN*2 bytes, 16-byte chunks
-// XOR-swizzled by row), then 64 lanes store 64 consecutive 16-byte chunks
-// (WTN*2/16 chunks per row).  Tiles larger than the free LDS go in passes of
-// whole 32-row fragment rows.  Requires ldo % 8 == 0 and a 16-byte aligned
-// `out`; the caller must have drained every LDS-DMA load and the workgroup
-// must be past its last main-loop LDS read (this function begins with a
-// workgroup barrier).
+// Store an accumulator tile through LDS so that every global store
+// instruction writes whole row segments (1 KB of 2 rows of f32, 4 of 16 bits;
+// straight from the registers it would be 32 bytes of each of 32 rows: f32
+// wgrad (8, 2080, 2048, 2048) 51 us that way and 43 staged): each
+// wave transposes its WTM x WTN tile into its own LDS area (rows of WTN output
+// elements, 16-byte chunks XOR-swizzled by row), then 64 lanes store 64
+// consecutive 16-byte chunks.  Tiles larger than the free LDS go in passes of
+// whole 32-row fragment rows.  Requires rows that are multiples of 16 bytes
+// and a 16-byte aligned `out`; the caller must have drained every LDS-DMA load
+// and the workgroup must be past its last main-loop LDS read (this function
+// begins with a workgroup barrier).
 // Largest divisor of fm not above lim (fragment rows per staging pass).
 constexpr int store_pass_rows(int fm, int lim) {
   int best = 1;
@@ -976,13 +978,15 @@ constexpr int store_pass_rows(int fm, int lim) {
   return best;
 }
 
-// BF16: the 16-bit output type (bf16, else f16), fixed at compile time so the
-// staging loop carries no per-write type test.  RB16 (f16 only): convert the
-// bf16-rounded value (the weight gradient's store semantics).
-template <class C, bool BF16, bool RB16 = false>
+// DT: the output type, fixed at compile time so the staging loop carries no
+// per-write type test.  RB16 (f16, f32): store the bf16-rounded value (the
+// weight gradient's semantics).
+template <class C, int DT, bool RB16 = false>
 __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], uint8_t* smem,
                                                uint8_t* out, int64_t ldo, int rows, int cols) {
-  constexpr int RB = C::WTN * 2;                 // staged row bytes
+  constexpr int ES = DT == MXGG_DTYPE_F32 ? 4 : 2;
+  constexpr int EPC = 16 / ES;                   // elements per 16-byte chunk
+  constexpr int RB = C::WTN * ES;                // staged row bytes
   constexpr int NCH = RB / 16;                   // 16-byte chunks per row
   constexpr int AVAIL = C::LDS / C::NW;           // LDS bytes per wave
   constexpr int FPP = store_pass_rows(C::FM, AVAIL / (32 * RB));   // fragment rows per pass
@@ -1005,24 +1009,36 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
           const v16f& a = acc[i0 + ii][j];
-          uint32_t w0, w1;
-          if constexpr (BF16) {
-            w0 = pack_bf16x2(a[4 * q4 + 0], a[4 * q4 + 1]);
-            w1 = pack_bf16x2(a[4 * q4 + 2], a[4 * q4 + 3]);
-          } else {
-            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-            float f0 = a[4 * q4 + 0], f1 = a[4 * q4 + 1], f2 = a[4 * q4 + 2], f3 = a[4 * q4 + 3];
+          float f0 = a[4 * q4 + 0], f1 = a[4 * q4 + 1], f2 = a[4 * q4 + 2], f3 = a[4 * q4 + 3];
+          if constexpr (DT == MXGG_DTYPE_F32) {
+            const int c = 8 * j + 2 * q4 + (lane >> 5);    // 16-byte chunk (4 columns)
             if constexpr (RB16) {
-              f0 = round_bf16(f0); f1 = round_bf16(f1); f2 = round_bf16(f2); f3 = round_bf16(f3);
+              const uint32_t w0 = pack_bf16x2(f0, f1), w1 = pack_bf16x2(f2, f3);
+              f0 = bf16_to_f32(w0 & 0xffffu);
+              f1 = __uint_as_float(w0 & 0xffff0000u);
+              f2 = bf16_to_f32(w1 & 0xffffu);
+              f3 = __uint_as_float(w1 & 0xffff0000u);
             }
-            h2 x = {(_Float16)f0, (_Float16)f1};
-            h2 y = {(_Float16)f2, (_Float16)f3};
-            w0 = __builtin_bit_cast(uint32_t, x);
-            w1 = __builtin_bit_cast(uint32_t, y);
+            *reinterpret_cast<float4*>(area + m * RB + ((c ^ (m % NCH)) * 16)) = make_float4(f0, f1, f2, f3);
+          } else {
+            uint32_t w0, w1;
+            if constexpr (DT == MXGG_DTYPE_BF16) {
+              w0 = pack_bf16x2(f0, f1);
+              w1 = pack_bf16x2(f2, f3);
+            } else {
+              typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+              if constexpr (RB16) {
+                f0 = round_bf16(f0); f1 = round_bf16(f1); f2 = round_bf16(f2); f3 = round_bf16(f3);
+              }
+              h2 x = {(_Float16)f0, (_Float16)f1};
+              h2 y = {(_Float16)f2, (_Float16)f3};
+              w0 = __builtin_bit_cast(uint32_t, x);
+              w1 = __builtin_bit_cast(uint32_t, y);
+            }
+            const int c = 4 * j + q4;                      // 16-byte chunk (8 columns)
+            *reinterpret_cast<uint2*>(area + m * RB + ((c ^ (m % NCH)) * 16) + 8 * (lane >> 5)) =
+                make_uint2(w0, w1);
           }
-          const int c = 4 * j + q4;                      // 16-byte chunk (8 columns)
-          *reinterpret_cast<uint2*>(area + m * RB + ((c ^ (m % NCH)) * 16) + 8 * (lane >> 5)) =
-              make_uint2(w0, w1);
         }
       }
     }
@@ -1038,8 +1054,8 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
         const int c = lane % NCH;
         const v4i v = *reinterpret_cast<const v4i*>(area + r * RB + ((c ^ (r % NCH)) * 16));
         const int row = wm * C::WTM + i0 * 32 + r;
-        const int col = wn * C::WTN + c * 8;
-        __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(reinterpret_cast<uint16_t*>(out) + (int64_t)row * ldo + col));
+        const int col = wn * C::WTN + c * EPC;
+        __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(out + ((int64_t)row * ldo + col) * ES));
       }
     } else {
 #pragma unroll
@@ -1048,16 +1064,21 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
         const int c = lane % NCH;
         const uint4 v = *reinterpret_cast<const uint4*>(area + r * RB + ((c ^ (r % NCH)) * 16));
         const int row = wm * C::WTM + i0 * 32 + r;
-        const int col = wn * C::WTN + c * 8;
+        const int col = wn * C::WTN + c * EPC;
         if (row < rows) {
-          uint16_t* p = reinterpret_cast<uint16_t*>(out) + (int64_t)row * ldo + col;
-          if (col + 8 <= cols) {
+          uint8_t* p = out + ((int64_t)row * ldo + col) * ES;
+          if (col + EPC <= cols) {
             *reinterpret_cast<uint4*>(p) = v;
           } else {
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (col + e < cols) p[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+            for (int e = 0; e < EPC; ++e)
+              if (col + e < cols) {
+                if constexpr (ES == 4)
+                  reinterpret_cast<uint32_t*>(p)[e] = w[e];
+                else
+                  reinterpret_cast<uint16_t*>(p)[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+              }
           }
         }
       }
@@ -1213,21 +1234,45 @@ struct FwdParams {
 // Epilogue of the whole-tile kernels, fixed at compile time so that the
 // common case carries none of the others' register pressure (with every
 // variant in one kernel the allocator spilled accumulators to scratch and
-// reloaded them serially in the epilogue): kEpiBf16 / kEpiF16 are bf16 / f16
-// outputs whose rows are 16-byte aligned (row stride a multiple of 8
-// elements, 16-byte aligned base), staged through LDS; kEpiF32 stores f32
-// directly, and kEpiBf16Any / kEpiF16Any 16-bit rows off the 16-byte grid;
-// kEpiAny (the wgrad's other outputs) picks the type per call.
-constexpr int kEpiAny = 0, kEpiBf16 = 1, kEpiF16 = 2, kEpiF32 = 3, kEpiBf16Any = 4, kEpiF16Any = 5;
+// reloaded them serially in the epilogue): kEpiBf16 / kEpiF16 / kEpiF32 are
+// outputs whose rows are 16-byte aligned (row stride a multiple of 16 bytes,
+// 16-byte aligned base), staged through LDS; kEpiBf16Any / kEpiF16Any /
+// kEpiF32Any rows off the 16-byte grid, stored from the registers.
+constexpr int kEpiBf16 = 1, kEpiF16 = 2, kEpiF32 = 3, kEpiBf16Any = 4, kEpiF16Any = 5, kEpiF32Any = 6;
 
 // Epilogue of a whole-tile launch for this output (host side).
 inline int pick_epi(int out_dtype, int64_t ldo, const void* out) {
-  const bool al16 = ldo % 8 == 0 && (uintptr_t)out % 16 == 0;
-  if (al16 && out_dtype == MXGG_DTYPE_BF16) return kEpiBf16;
-  if (al16 && out_dtype == MXGG_DTYPE_F16) return kEpiF16;
-  if (out_dtype == MXGG_DTYPE_F32) return kEpiF32;
-  return out_dtype == MXGG_DTYPE_BF16 ? kEpiBf16Any : kEpiF16Any;
+  const bool f32 = out_dtype == MXGG_DTYPE_F32;
+  const bool al16 = ldo % (f32 ? 4 : 8) == 0 && (uintptr_t)out % 16 == 0;
+  if (f32) return al16 ? kEpiF32 : kEpiF32Any;
+  if (out_dtype == MXGG_DTYPE_BF16) return al16 ? kEpiBf16 : kEpiBf16Any;
+  return al16 ? kEpiF16 : kEpiF16Any;
 }
+
+// Store tile acc at `out` (the tile's first element) by epilogue EPI.
+// BF16_ONLY: the bf16-rounded value whatever the output type (wgrad).
+template <class C, int EPI, bool BF16_ONLY>
+__device__ __forceinline__ void store_epi(const v16f (&acc)[C::FM][C::FN], uint8_t* smem, uint8_t* out, int64_t ldo,
+                                          int rows, int cols) {
+  constexpr int dt = EPI == kEpiF32 || EPI == kEpiF32Any ? MXGG_DTYPE_F32
+                     : EPI == kEpiF16 || EPI == kEpiF16Any ? MXGG_DTYPE_F16
+                                                           : MXGG_DTYPE_BF16;
+  if constexpr (EPI == kEpiBf16 || EPI == kEpiF16 || EPI == kEpiF32)
+    store_tile_lds<C, dt, BF16_ONLY>(acc, smem, out, ldo, rows, cols);
+  else
+    store_tile<C, BF16_ONLY>(acc, out, ldo, rows, cols, dt);
+}
+
+// Launches `call` (a macro of one epilogue) for every epilogue.
+#define MXGG_EPI_SWITCH(epi, call) \
+  switch (epi) {                   \
+    call(kEpiBf16);                \
+    call(kEpiF16);                 \
+    call(kEpiF32);                 \
+    call(kEpiBf16Any);             \
+    call(kEpiF16Any);              \
+    call(kEpiF32Any);              \
+  }
 
 struct FwdTile {
   int expert;
@@ -1302,17 +1347,8 @@ __device__ __forceinline__ void fwd_tile_run(const FwdParams& p, uint8_t* smem, 
     store_partial<C>(acc, p.part + (int64_t)slot * (C::BM * C::BN));
   } else {
     step_mainloop<C>(smem, X, W, xs, ws, 0, K, acc);
-    if constexpr (EPI == kEpiBf16) {
-      store_tile_lds<C, true>(acc, smem, p.out + (row0 * p.ldo + n0) * 2, p.ldo, rows, cols);
-    } else if constexpr (EPI == kEpiF16) {
-      store_tile_lds<C, false>(acc, smem, p.out + (row0 * p.ldo + n0) * 2, p.ldo, rows, cols);
-    } else if constexpr (EPI == kEpiF32) {
-      store_tile<C, false>(acc, p.out + (row0 * p.ldo + n0) * 4, p.ldo, rows, cols, MXGG_DTYPE_F32);
-    } else {
-      static_assert(EPI == kEpiBf16Any || EPI == kEpiF16Any, "forward epilogue");
-      store_tile<C, false>(acc, p.out + (row0 * p.ldo + n0) * 2, p.ldo, rows, cols,
-                           EPI == kEpiBf16Any ? MXGG_DTYPE_BF16 : MXGG_DTYPE_F16);
-    }
+    constexpr int es = EPI == kEpiF32 || EPI == kEpiF32Any ? 4 : 2;
+    store_epi<C, EPI, false>(acc, smem, p.out + (row0 * p.ldo + n0) * es, p.ldo, rows, cols);
   }
 }
 
@@ -1349,7 +1385,7 @@ __global__ __launch_bounds__(C::NT) void fwd_kernel(FwdParams p) {
   const Split sp = fwd_split<C>(p, tiles);
   const int pid = blockIdx.x;
   if constexpr (PIECES) {
-    if (pid < sp.units) fwd_run<C, true, kEpiAny>(p, smem, sp.dp + pid / sp.S, pid % sp.S, sp.S, pid, tiles, wg);
+    if (pid < sp.units) fwd_run<C, true, kEpiBf16>(p, smem, sp.dp + pid / sp.S, pid % sp.S, sp.S, pid, tiles, wg);
   } else {
     if (pid < sp.dp) fwd_run<C, false, EPI>(p, smem, pid, 0, 1, 0, tiles, wg);
   }
@@ -1746,7 +1782,7 @@ __device__ __forceinline__ int wgrad_slot_group(const WgradParams& p, int y) {
 // g * tiles_n * tiles_k + x of group g = wgrad_slot_group(y) whole when below
 // wgrad_whole (epilogue EPI); true: workgroup u computes the piece
 // wgrad_unit assigns it.
-template <class C, bool PIECES, int EPI = kEpiAny>
+template <class C, bool PIECES, int EPI = kEpiBf16>
 __global__ __launch_bounds__(C::NT) void wgrad_kernel(WgradParams p) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[C::LDS];
   int lt, piece = 0, S = 1;
@@ -1793,18 +1829,8 @@ __global__ __launch_bounds__(C::NT) void wgrad_kernel(WgradParams p) {
     store_partial<C>(acc, p.part + (int64_t)blockIdx.x * (C::BM * C::BN));
     return;
   }
-  if constexpr (EPI == kEpiBf16) {
-    store_tile_lds<C, true>(acc, smem, p.out + ((int64_t)g * p.N * p.K + n0 * p.K + k0) * 2, p.K, rows, cols);
-  } else if constexpr (EPI == kEpiF16) {   // f16 of the bf16-rounded value
-    store_tile_lds<C, false, true>(acc, smem, p.out + ((int64_t)g * p.N * p.K + n0 * p.K + k0) * 2, p.K, rows,
-                                   cols);
-  } else if constexpr (EPI == kEpiF16Any) {   // the same, rows off the 16-byte grid
-    store_tile<C, true>(acc, p.out + ((int64_t)g * p.N * p.K + n0 * p.K + k0) * 2, p.K, rows, cols, MXGG_DTYPE_F16);
-  } else {   // f32, or bf16 rows off the 16-byte grid (the type known to be one of the two)
-    const int dt = p.out_dtype == MXGG_DTYPE_F32 ? MXGG_DTYPE_F32 : MXGG_DTYPE_BF16;
-    const int esz = dt == MXGG_DTYPE_F32 ? 4 : 2;
-    store_tile<C, true>(acc, p.out + ((int64_t)g * p.N * p.K + n0 * p.K + k0) * esz, p.K, rows, cols, dt);
-  }
+  constexpr int es = EPI == kEpiF32 || EPI == kEpiF32Any ? 4 : 2;
+  store_epi<C, EPI, true>(acc, smem, p.out + ((int64_t)g * p.N * p.K + n0 * p.K + k0) * es, p.K, rows, cols);
 }
 
 // Split tiles of a wgrad launch: one workgroup per item (v, c), as in
@@ -2106,31 +2132,19 @@ int launch_fwd(const FwdParams& p0, int grid_m_ub, int gm, int xcd, size_t part_
       if (split_plan(m * p.grid_n, p.par, nsteps, p.slots, C::BM * C::BN * 4 / 1024).units == 0) whole = true;
   }
   const int epi = pick_epi(p.out_dtype, p.ldo, p.out);
-  if (whole) switch (epi) {
 #define MXGG_WHOLE(E) \
   case E: hipLaunchKernelGGL((fwd_kernel<C, false, E>), dim3((unsigned)tiles_ub), dim3(C::NT), 0, st, p); break
-    MXGG_WHOLE(kEpiBf16);
-    MXGG_WHOLE(kEpiF16);
-    MXGG_WHOLE(kEpiF32);
-    MXGG_WHOLE(kEpiBf16Any);
-    MXGG_WHOLE(kEpiF16Any);
+  if (whole) MXGG_EPI_SWITCH(epi, MXGG_WHOLE)
 #undef MXGG_WHOLE
-  }
   if (int rc = launch_status("grouped_mm")) return rc;
   if constexpr (kQuads) {
     if (p.quads) {   // 4 * (T % P) <= P quarters
-      switch (epi) {
-#define MXGG_QUAD(E)                                                                                         \
+#define MXGG_QUAD(E)                                                                                        \
   case E:                                                                                                   \
-    hipLaunchKernelGGL((fwd_quad_kernel<C, Q, E>), dim3((unsigned)p.par), dim3(Q::NT), 0, st, p); \
+    hipLaunchKernelGGL((fwd_quad_kernel<C, Q, E>), dim3((unsigned)p.par), dim3(Q::NT), 0, st, p);           \
     break
-        MXGG_QUAD(kEpiBf16);
-        MXGG_QUAD(kEpiF16);
-        MXGG_QUAD(kEpiF32);
-        MXGG_QUAD(kEpiBf16Any);
-        MXGG_QUAD(kEpiF16Any);
+      MXGG_EPI_SWITCH(epi, MXGG_QUAD)
 #undef MXGG_QUAD
-      }
       if (int rc = launch_status("grouped_mm")) return rc;
     }
   }
@@ -2675,8 +2689,16 @@ static int check_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* go_s, 
 // row-major operands 7% faster than the split 256 x 256 launch, row pairs 3%
 // slower, taken on both so that the bits do not depend on the layout):
 // 128 x 128 tiles instead, four times as many, two workgroups per CU, whole.
+// So do calls of at most kSmallTokens tokens per group, most of whose time is
+// the start and the store of a tile, which the second workgroup of a CU covers
+// (MI355X, 256 / 128 tiles: (32, 4160, 2880, 2880) 241 / 197 us, (8, 2080,
+// 5120, 5120) 158 / 151, (8, 2080, 2048, 2048) f32 43.5 / 41.3, 520 tokens
+// (32, 16640, 2880, 2880) 327 / 316; 1040 tokens (8, 8320, 5120, 5120) 255 /
+// 280, (8, 8320, 2048, 2048) 50.6 / 53.2).
 // p: the call's parameters with the 256 x 256 tile counts (replaced here).
-static int launch_wgrad_small(WgradParams p, bool al16, hipStream_t st) {
+constexpr int64_t kSmallTokens = 640;
+
+static int launch_wgrad_small(WgradParams p, hipStream_t st) {
   typedef CfgF8_128 Q;
   p.tiles_n = (int)cdiv(p.N, Q::BM);
   p.tiles_k = (int)cdiv(p.K, Q::BN);
@@ -2686,14 +2708,10 @@ static int launch_wgrad_small(WgradParams p, bool al16, hipStream_t st) {
   p.units = 0;
   p.dev = 0;
   const dim3 grid((unsigned)(p.tiles_n * p.tiles_k), (unsigned)p.E);
-  if (p.out_dtype == MXGG_DTYPE_BF16 && al16)
-    hipLaunchKernelGGL((wgrad_kernel<Q, false, kEpiBf16>), grid, dim3(Q::NT), 0, st, p);
-  else if (p.out_dtype == MXGG_DTYPE_F16 && al16)
-    hipLaunchKernelGGL((wgrad_kernel<Q, false, kEpiF16>), grid, dim3(Q::NT), 0, st, p);
-  else if (p.out_dtype == MXGG_DTYPE_F16)
-    hipLaunchKernelGGL((wgrad_kernel<Q, false, kEpiF16Any>), grid, dim3(Q::NT), 0, st, p);
-  else
-    hipLaunchKernelGGL((wgrad_kernel<Q, false, kEpiAny>), grid, dim3(Q::NT), 0, st, p);
+#define MXGG_WGRAD(E) \
+  case E: hipLaunchKernelGGL((wgrad_kernel<Q, false, E>), grid, dim3(Q::NT), 0, st, p); break
+  MXGG_EPI_SWITCH(pick_epi(p.out_dtype, p.K, p.out), MXGG_WGRAD)
+#undef MXGG_WGRAD
   return launch_status("wgrad");
 }
 
@@ -2716,7 +2734,8 @@ static WgradChoice wgrad_choice(int E, int64_t M, int64_t N, int64_t K, int64_t 
   // rows would be split.
   w.dev = E > 1 && slots > 0 && split_plan((int)tiles, par, (int)cdiv(M, STEP) + 1, slots, kib).units > 0;
   const int64_t tiles128 = (int64_t)E * cdiv(N, 128) * cdiv(K, 128);
-  w.small = (!w.dev && w.sp.units == 0 && 2 * tiles <= par) || (2 * tiles <= par && tiles128 >= 2 * par);
+  w.small = (!w.dev && w.sp.units == 0 && 2 * tiles <= par) || (2 * tiles <= par && tiles128 >= 2 * par) ||
+            (!w.dev && w.sp.units == 0 && M <= kSmallTokens * (int64_t)E);
   return w;
 }
 
@@ -2755,21 +2774,16 @@ static int launch_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* gs, c
     p.par = par;
     p.slots = slots;
   }
-  const bool al16 = K % 8 == 0 && (uintptr_t)out % 16 == 0;
-  if (wc.small) return launch_wgrad_small(p, al16, st);
+  if (wc.small) return launch_wgrad_small(p, st);
   const int64_t whole_ub = p.dev ? tiles : sp.dp;
   const int64_t units_ub = p.dev ? slots : sp.units;
   const int64_t split_tiles_ub = p.dev ? tiles : (sp.units ? sp.units / sp.S : 0);
   if (whole_ub > 0) {
     const dim3 grid((unsigned)(p.tiles_n * p.tiles_k), (unsigned)E);
-    if (out_dtype == MXGG_DTYPE_BF16 && al16)
-      hipLaunchKernelGGL((wgrad_kernel<C, false, kEpiBf16>), grid, dim3(C::NT), 0, st, p);
-    else if (out_dtype == MXGG_DTYPE_F16 && al16)
-      hipLaunchKernelGGL((wgrad_kernel<C, false, kEpiF16>), grid, dim3(C::NT), 0, st, p);
-    else if (out_dtype == MXGG_DTYPE_F16)
-      hipLaunchKernelGGL((wgrad_kernel<C, false, kEpiF16Any>), grid, dim3(C::NT), 0, st, p);
-    else
-      hipLaunchKernelGGL((wgrad_kernel<C, false, kEpiAny>), grid, dim3(C::NT), 0, st, p);
+#define MXGG_WGRAD(E) \
+  case E: hipLaunchKernelGGL((wgrad_kernel<C, false, E>), grid, dim3(C::NT), 0, st, p); break
+    MXGG_EPI_SWITCH(pick_epi(out_dtype, K, out), MXGG_WGRAD)
+#undef MXGG_WGRAD
     if (int rc = launch_status("wgrad")) return rc;
   }
   if (units_ub <= 0) return MXGG_OK;

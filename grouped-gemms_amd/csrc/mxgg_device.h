@@ -133,9 +133,12 @@ __device__ __forceinline__ float round_bf16(float x) {
 // buffer resources (raw buffers: loads past num_records return zero)
 // ---------------------------------------------------------------------------
 
+// Wave-uniform by construction (readfirstlane folds away where the compiler
+// sees it too): asm that takes a resource needs it in scalar registers.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
+  const uint64_t b = (uint64_t)(uintptr_t)base;
+  const uint64_t u = (uint32_t)uniform((int)(uint32_t)b) | ((uint64_t)(uint32_t)uniform((int)(b >> 32)) << 32);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)u, (short)0, uniform((int)bytes), 0x00020000);
 }
 
 constexpr uint32_t kOOB = 0x80000000u;  // voffset that is always out of range

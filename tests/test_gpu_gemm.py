@@ -161,6 +161,32 @@ def test_fwd_out_dtypes(gpu, out_dtype):
     assert err <= (1e-4 if out_dtype == torch.float32 else 1e-3), err
 
 
+@pytest.mark.parametrize("N", [512, 300, 301, 96])     # whole tiles, 16-byte rows, rows off the grid, one narrow tile
+@pytest.mark.parametrize("tile", [128, 256])
+def test_f32_output_rounds_to_bf16_output(gpu, N, tile):
+    """Every f32 epilogue (rows staged through LDS in 16-byte chunks, partial
+    tiles, rows off the 16-byte grid) stores the accumulators that the bf16
+    call rounds: forward f32 output rounded to bf16 equals the bf16 output bit
+    for bit, and a wgrad's f32 output, bf16-rounded already, equals it as
+    stored."""
+    import kernels
+    E, M, K = 3, 1056, 416
+    offs = torch.tensor([100, 100 + 517, M], dtype=torch.int32, device=gpu)
+    sa, qa = kernels.to_mx(randn_bf16((M, K), 1.0, 1).to(gpu))
+    sb, qb = kernels.to_mx(randn_bf16((E, N, K), 0.1, 2).to(gpu))
+    outs = [kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=dt, BLOCK_M=tile, BLOCK_N=tile)
+            for dt in (torch.float32, torch.bfloat16)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].to(torch.bfloat16).view(torch.int16), outs[1].view(torch.int16))
+    if N % 8:
+        return      # dim-0 quantization needs rows of 16 bytes
+    sg, qg = kernels.to_mx_dim0(randn_bf16((M, N), 1.0, 3).to(gpu))
+    si, qi = kernels.to_mx_dim0(randn_bf16((M, K), 1.0, 4).to(gpu))
+    outs = [kernels.triton_mxfp8_wgrad(qg, sg, qi, si, offs, out_dtype=dt) for dt in (torch.float32, torch.bfloat16)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1].float())
+
+
 @pytest.mark.parametrize("gm", [3, 12])
 def test_fwd_many_groups(gpu, gm):
     """80 groups, a fifth of them empty, sizes 0..96 rows: the in-kernel tile
