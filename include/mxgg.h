@@ -193,11 +193,10 @@ int mxgg_tile_schedule(const int32_t* offs, int E, int64_t M, int64_t N, int blo
  * *xcd_swizzle on entry) are applied as mxgg_grouped_mm applies them; the
  * call returns MXGG_ERR_UNSUPPORTED when the resulting tile is not built.
  * Replaces `_pick_config` / `_BEST_CFGS` / `_FALLBACK_*`
- * (kernels/forward.py:399-459).  The answer is the one for a
- * mxgg_grouped_mm call given room to stage its operands (the drop-in call):
- * a tuned entry's GROUP_M and XCD swizzle apply only to calls on the operand
- * layout it was timed on, so a *_steps call on another layout may get the
- * built-in order (tile shape and split stay the entry's: same bits).
+ * (kernels/forward.py:399-459).  The answer holds on every operand layout.
+ * Calls of few rows per group (M <= 32, or M <= 48 E) that request no tile
+ * run weight-streaming tiles of 32 or 64 rows x 128 columns instead, which
+ * cannot be requested: same bits as the answer's tile, whole.
  */
 int mxgg_grouped_mm_config(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int* block_m,
                            int* block_n, int* group_m, int* xcd_swizzle);

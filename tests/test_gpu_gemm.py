@@ -161,6 +161,55 @@ def test_fwd_out_dtypes(gpu, out_dtype):
     assert err <= (1e-4 if out_dtype == torch.float32 else 1e-3), err
 
 
+def _routed(E, M, seed):
+    """Cumulative ends of M rows that pick one of E groups at random."""
+    n = np.bincount(np.random.default_rng(seed).integers(0, E, M), minlength=E)
+    return torch.tensor(np.cumsum(n), dtype=torch.int32)
+
+
+@pytest.mark.parametrize("E,M,N,K,elem,out_dtype", [
+    (8, 64, 384, 2048, "e4m3", torch.bfloat16),      # 32-row tiles, plain scales, 16 steps
+    (8, 61, 200, 2976, "e4m3", torch.bfloat16),      # scale rows off the 16-byte grid (re-laid), K % 128 = 32, partial columns
+    (16, 100, 130, 160, "e4m3", torch.float32),      # two steps, the second of 32 elements; empty groups; odd rows
+    (1, 1, 33, 32, "e4m3", torch.bfloat16),          # one row, one block
+    (1, 32, 128, 1152, "e4m3", torch.float16),       # one whole tile, 9 steps: a second scale group
+    (4, 40, 256, 3072, "e2m1", torch.bfloat16),      # packed weight, plain scales
+    (3, 20, 97, 1088, "e2m1", torch.float32),        # packed weight, re-laid scales, half-full last step
+    (8, 300, 256, 2048, "e4m3", torch.bfloat16),     # 64-row tiles
+    (5, 239, 136, 4192, "e4m3", torch.float16),      # 64-row tiles, 33 steps, groups past 64 rows
+    (8, 300, 128, 640, "e2m1", torch.float32),       # 64-row tiles, packed weight
+])
+def test_few_rows_match_general_tiles(gpu, E, M, N, K, elem, out_dtype):
+    """Calls of few rows per group run weight-streaming tiles: the bits of the
+    256 x 256 tiles (whose reductions, all below 4096 elements or forced whole,
+    are not split), on every scale and data layout, and the oracle's values."""
+    import kernels
+    offs = _routed(E, M, E * M + K).to(gpu)
+    f4 = elem == "e2m1"
+    dt = torch.float4_e2m1fn_x2 if f4 else torch.float8_e4m3fn
+    a, b = randn_bf16((M, K), 1.0, 5).to(gpu), randn_bf16((E, N, K), 0.05, 6).to(gpu)
+    sa, qa = kernels.to_mx(a)
+    sb, qb = kernels.to_mx(b, elem_dtype=dt)
+    mm = kernels.triton_mxfp8_grouped_mm
+    out = mm(qa, qb, sa, sb, offs, out_dtype=out_dtype)
+    torch.cuda.synchronize()
+    ref = O.grouped_mm(bits_u8(qa), bits_u8(sa), bits_u8(qb), bits_u8(sb), offs.cpu().numpy(), b_elem=elem)
+    err = O.rel_fro(ref, f32(out))
+    assert err <= {torch.float32: 1e-4, torch.float16: 1e-3, torch.bfloat16: 1e-2}[out_dtype], err
+    if K < 4096:
+        general = mm(qa, qb, sa, sb, offs, out_dtype=out_dtype, BLOCK_M=256, BLOCK_N=256)
+        assert torch.equal(general.view(torch.uint8), out.view(torch.uint8))
+    ta, _ = kernels.to_mx(a, scale_layout="steps")
+    tb, _ = kernels.to_mx(b, elem_dtype=dt, scale_layout="steps")
+    assert torch.equal(mm(qa, qb, ta, tb, offs, out_dtype=out_dtype).view(torch.uint8), out.view(torch.uint8))
+    if N % 4 == 0:
+        _, pb = kernels.to_mx(b, elem_dtype=dt, scale_layout="steps", data_layout="quads" if f4 else "pairs")
+        assert torch.equal(mm(qa, pb, ta, tb, offs, out_dtype=out_dtype).view(torch.uint8), out.view(torch.uint8))
+    if M % 2 == 0:
+        _, pa = kernels.to_mx(a, scale_layout="steps", data_layout="pairs")
+        assert torch.equal(mm(pa, qb, ta, tb, offs, out_dtype=out_dtype).view(torch.uint8), out.view(torch.uint8))
+
+
 @pytest.mark.parametrize("N", [512, 300, 301, 96])     # whole tiles, 16-byte rows, rows off the grid, one narrow tile
 @pytest.mark.parametrize("tile", [128, 256])
 def test_f32_output_rounds_to_bf16_output(gpu, N, tile):
