@@ -9,6 +9,7 @@ stubs when its kernels are unavailable (kernels/forward.py:608-612).
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -92,6 +93,7 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+_calls = None
 
 
 def _open(path: str) -> ctypes.CDLL:
@@ -110,15 +112,41 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     global _lib
     if path != LIB_PATH:
         return _open(path)
-    with _lock:
-        if _lib is None:
-            _lib = _open(path)
-        return _lib
+    if _lib is None:
+        with _lock:
+            if _lib is None:
+                _lib = _open(path)
+    return _lib
+
+
+def calls():
+    """The launching entry points as a CPython module (csrc/pycalls.c, built
+    and linked beside libmxgg.so): the same functions and arguments as the
+    ctypes ones, without their per-argument conversions."""
+    global _calls
+    if _calls is None:
+        load()
+        try:
+            from . import _calls as m
+        except ImportError as e:
+            raise NotImplementedError(f"kernels/_calls is not built (run make -C grouped-gemms_amd/csrc): {e}") from e
+        _calls = m
+    return _calls
+
+
+@functools.lru_cache(maxsize=1024)
+def grouped_mm_workspace_size(E: int, M: int, N: int, K: int) -> int:
+    return load().mxgg_grouped_mm_workspace_size(E, M, N, K)
+
+
+@functools.lru_cache(maxsize=1024)
+def wgrad_workspace_size(E: int, M: int, N: int, K: int) -> int:
+    return load().mxgg_wgrad_workspace_size(E, M, N, K)
 
 
 def available() -> bool:
     try:
-        load()
+        calls()
         return True
     except (NotImplementedError, OSError):
         return False

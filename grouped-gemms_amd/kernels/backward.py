@@ -21,7 +21,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._common import _offsets, _out_code, _pair_geometry, _require, _rowmajor, _staging_enabled, _stream_handle, _u8
+from ._common import _offsets, _out_code, _pair_geometry, _require, _rowmajor, _staging_enabled, _stream_handle
 from .forward import _split_room
 
 
@@ -89,35 +89,36 @@ def triton_mxfp8_wgrad(
         raise ValueError(f"ia_scale shape {tuple(ia_scale.shape)} != {want_i}")
     E = group_end_offsets.shape[0]
     dev = go_t.device
-    g = _u8(go_t if pg else _rowmajor(go_t))
-    a = _u8(ia_t if pi else _rowmajor(ia_t))
-    ld_g = pg[2] if pg else g.stride(0)
-    ld_a = pi[2] if pi else a.stride(0)
+    g, sg = (go_t, go_t.stride()) if pg else _rowmajor(go_t)
+    a, sa = (ia_t, ia_t.stride()) if pi else _rowmajor(ia_t)
+    ld_g = pg[2] if pg else sg[0]
+    ld_a = pi[2] if pi else sa[0]
     offs = _offsets(group_end_offsets, dev)
     code = _out_code(out_dtype)
     out = torch.empty((E, N, K), dtype=out_dtype, device=dev)
-    lib = _lib.load()
-    ws_bytes = lib.mxgg_wgrad_workspace_size(E, M, N, K)
+    calls = _lib.calls()
+    ws_bytes = _lib.wgrad_workspace_size(E, M, N, K)
     if steps:
         gss, iss = go_scale.contiguous(), ia_scale.contiguous()
         ws_bytes = _split_room(ws_bytes, 4 * T * (N + K))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        rc = lib.mxgg_wgrad_steps(
+        rc = calls.mxgg_wgrad_steps(
             g.data_ptr(), ld_g, gss.data_ptr(), a.data_ptr(), ld_a, iss.data_ptr(),
             offs.data_ptr(), E, M, N, K,
             out.data_ptr(), code, layout, ws.data_ptr() if ws is not None else None, ws_bytes,
             _stream_handle(dev))
         _lib.check(rc)
         return out
-    gs = _u8(_rowmajor(go_scale))
-    as_ = _u8(_rowmajor(ia_scale))
+    gs, sgs = _rowmajor(go_scale)
+    as_, sas = _rowmajor(ia_scale)
     # plus, with MXGG_STAGING=1, room to stage both operands in row pairs
-    if _staging_enabled():
-        ws_bytes += lib.mxgg_wgrad_staging_size(E, M, N, K)
+    # (narrower outputs stage nothing)
+    if N + K >= 10240 and _staging_enabled():
+        ws_bytes += _lib.load().mxgg_wgrad_staging_size(E, M, N, K)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    rc = lib.mxgg_wgrad(
-        g.data_ptr(), g.stride(0), gs.data_ptr(), gs.stride(0),
-        a.data_ptr(), a.stride(0), as_.data_ptr(), as_.stride(0),
+    rc = calls.mxgg_wgrad(
+        g.data_ptr(), ld_g, gs.data_ptr(), sgs[0],
+        a.data_ptr(), ld_a, as_.data_ptr(), sas[0],
         offs.data_ptr(), E, M, N, K,
         out.data_ptr(), code, ws.data_ptr() if ws is not None else None, ws_bytes,
         _stream_handle(dev))

@@ -30,7 +30,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._common import _offsets, _out_code, _pair_geometry, _require, _rowmajor, _staging_enabled, _stream_handle, _u8
+from ._common import _offsets, _out_code, _pair_geometry, _require, _rowmajor, _staging_enabled, _stream_handle
 
 # Tile shapes built into libmxgg (BLOCK_M x BLOCK_N); BLOCK_K is fixed at 128.
 BUILT_TILES = ((256, 256), (128, 128))
@@ -153,50 +153,51 @@ def triton_mxfp8_grouped_mm(
     # Tile requests are hints: a built tile is used, anything else (e.g. a
     # Triton config copied from the reference's table) falls back to the
     # library's own choice instead of failing.
-    bm = BLOCK_M or BLOCK_N or 0
-    bn = BLOCK_N or BLOCK_M or 0
+    bm = int(BLOCK_M or BLOCK_N or 0)
+    bn = int(BLOCK_N or BLOCK_M or 0)
     if (bm, bn) not in BUILT_TILES:
         bm = bn = 0
     dev = input_act.device
-    a = _u8(input_act if pa else _rowmajor(input_act))
-    b = _u8(weight if pb else _rowmajor(weight))
-    lda = pa[2] if pa else a.stride(0)
-    ldb_n = pb[2] if pb else b.stride(1)
+    a, sa = (input_act, input_act.stride()) if pa else _rowmajor(input_act)
+    b, sb = (weight, weight.stride()) if pb else _rowmajor(weight)
+    lda = pa[2] if pa else sa[0]
+    ldb_n = pb[2] if pb else sb[1]
     offs = _offsets(group_end_offsets, dev)
     out = torch.empty((M, N), dtype=out_dtype, device=dev)
     code = _out_code(out_dtype)
-    lib = _lib.load()
+    calls = _lib.calls()
     # scratch for the scales re-laid step-major and the fp32 partial tiles of a
     # split last round (overwritten by the call; torch's caching allocator
     # makes the per-call allocation cheap)
-    ws_bytes = lib.mxgg_grouped_mm_workspace_size(E, M, N, K)
+    ws_bytes = _lib.grouped_mm_workspace_size(E, M, N, K)
     if steps:
         a_ss, b_ss = input_act_scales.contiguous(), weight_scales.contiguous()
         ws_bytes = _split_room(ws_bytes, 4 * T * (M + E * N))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-        rc = lib.mxgg_grouped_mm_steps(
+        rc = calls.mxgg_grouped_mm_steps(
             a.data_ptr(), lda, a_ss.data_ptr(),
-            b.data_ptr(), b_fmt, ldb_n, b.stride(0), b_ss.data_ptr(),
+            b.data_ptr(), b_fmt, ldb_n, sb[0], b_ss.data_ptr(),
             offs.data_ptr(), E, M, N, K,
             out.data_ptr(), code, out.stride(0),
-            int(bm), int(bn), int(GROUP_M or 0), int(XCD_SWIZZLE or 0), layout,
+            bm, bn, int(GROUP_M or 0), int(XCD_SWIZZLE or 0), layout,
             ws.data_ptr() if ws is not None else None, ws_bytes,
             _stream_handle(dev))
         _lib.check(rc)
         return out
-    a_s = _u8(_rowmajor(input_act_scales))
-    b_s = _u8(_rowmajor(weight_scales))
-    # plus, with MXGG_STAGING=1, room to stage the weight and / or A in row pairs
-    if _staging_enabled():
-        ws_bytes += lib.mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt)
+    a_s, sas = _rowmajor(input_act_scales)
+    b_s, sbs = _rowmajor(weight_scales)
+    # plus, with MXGG_STAGING=1, room to stage the weight and / or A in row
+    # pairs (sizes below either bound stage nothing)
+    if (M >= 8192 * E or M * N * K > 60_000_000_000) and _staging_enabled():
+        ws_bytes += _lib.load().mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    rc = lib.mxgg_grouped_mm(
-        a.data_ptr(), a.stride(0), a_s.data_ptr(), a_s.stride(0),
-        b.data_ptr(), b_fmt, b.stride(1), b.stride(0),
-        b_s.data_ptr(), b_s.stride(1), b_s.stride(0),
+    rc = calls.mxgg_grouped_mm(
+        a.data_ptr(), lda, a_s.data_ptr(), sas[0],
+        b.data_ptr(), b_fmt, ldb_n, sb[0],
+        b_s.data_ptr(), sbs[1], sbs[0],
         offs.data_ptr(), E, M, N, K,
         out.data_ptr(), code, out.stride(0),
-        int(bm), int(bn), int(GROUP_M or 0), int(XCD_SWIZZLE or 0),
+        bm, bn, int(GROUP_M or 0), int(XCD_SWIZZLE or 0),
         ws.data_ptr() if ws is not None else None, ws_bytes,
         _stream_handle(dev))
     _lib.check(rc)

@@ -122,29 +122,26 @@ def to_mx(data: torch.Tensor, elem_dtype=torch.float8_e4m3fn, block_size: int = 
         qv, ld_q = _pair_buffer(shape[:-2], shape[-2], qcols, data.device, 4 if fp4 else 2)
         q_ptr = qv.data_ptr()
     else:
-        q = torch.empty((rows, qcols), dtype=torch.uint8, device=data.device)
+        q = torch.empty(shape[:-1] + (qcols,), dtype=torch.uint8 if fp4 else elem_dtype, device=data.device)
         q_ptr, ld_q = q.data_ptr(), qcols
     if lay == _lib.SCALES_STEPS:
         R = shape[-2] if len(shape) >= 2 else 1
         s = torch.empty(step_scales_shape(shape[:-2], R, L), dtype=torch.int32, device=data.device)
         ld_s = R
     else:
-        s = torch.empty((rows, L // 32), dtype=torch.uint8, device=data.device)
+        s = torch.empty(shape[:-1] + (L // 32,), dtype=torch.uint8, device=data.device)
         ld_s = L // 32
-    lib = _lib.load()
-    rc = lib.mxgg_quantize_mx(x.data_ptr(), code, rows, L, x.stride(0) if rows > 1 else L,
-                              _lib.FMT_E2M1 if fp4 else _lib.FMT_E4M3,
-                              q_ptr, ld_q, s.data_ptr(), ld_s,
-                              lay | ((_lib.DATA_QUADS if fp4 else _lib.DATA_PAIRS) if pairs else 0),
-                              _stream_handle(data.device))
+    rc = _lib.calls().mxgg_quantize_mx(x.data_ptr(), code, rows, L, x.stride(0) if rows > 1 else L,
+                                       _lib.FMT_E2M1 if fp4 else _lib.FMT_E4M3,
+                                       q_ptr, ld_q, s.data_ptr(), ld_s,
+                                       lay | ((_lib.DATA_QUADS if fp4 else _lib.DATA_PAIRS) if pairs else 0),
+                                       _stream_handle(data.device))
     _lib.check(rc)
     if pairs:
-        q = qv.view(_FP4 if fp4 else torch.float8_e4m3fn)
-    else:
-        q = q.view(_FP4 if fp4 else torch.float8_e4m3fn).reshape(shape[:-1] + (qcols,))
-    if lay == _lib.SCALES_STEPS:
-        return s, q
-    return s.reshape(shape[:-1] + (L // 32,)), q
+        q = qv.view(elem_dtype)
+    elif fp4:
+        q = q.view(elem_dtype)
+    return s, q
 
 
 def to_mx_dim0(data: torch.Tensor, elem_dtype=torch.float8_e4m3fn, block_size: int = 32, *,
@@ -180,10 +177,9 @@ def to_mx_dim0(data: torch.Tensor, elem_dtype=torch.float8_e4m3fn, block_size: i
     else:
         s = torch.empty((C, R // 32), dtype=torch.uint8, device=data.device)
         ld_s = R // 32
-    lib = _lib.load()
-    rc = lib.mxgg_quantize_mx_dim0(x.data_ptr(), code, R, C, x.stride(0), _lib.FMT_E4M3,
-                                   q.data_ptr(), ld_q, s.data_ptr(), ld_s, lay | (_lib.DATA_PAIRS if pairs else 0),
-                                   _stream_handle(data.device))
+    rc = _lib.calls().mxgg_quantize_mx_dim0(x.data_ptr(), code, R, C, x.stride(0), _lib.FMT_E4M3,
+                                            q.data_ptr(), ld_q, s.data_ptr(), ld_s,
+                                            lay | (_lib.DATA_PAIRS if pairs else 0), _stream_handle(data.device))
     _lib.check(rc)
     return s, q.view(torch.float8_e4m3fn)
 
@@ -228,10 +224,9 @@ def to_mx_both(data: torch.Tensor, elem_dtype=torch.float8_e4m3fn, block_size: i
         s_r = torch.empty((B, R, C // 32), dtype=torch.uint8, device=dev)
         s_c = torch.empty((B, C, R // 32), dtype=torch.uint8, device=dev)
         ld_r, ld_c = C // 32, R // 32
-    lib = _lib.load()
-    rc = lib.mxgg_quantize_mx_both(x.data_ptr(), code, B, R, C, C, q_r.data_ptr(), ld_qr, s_r.data_ptr(), ld_r,
-                                   q_c.data_ptr(), ld_qc, s_c.data_ptr(), ld_c,
-                                   lay | (_lib.DATA_PAIRS if pairs else 0), _stream_handle(dev))
+    rc = _lib.calls().mxgg_quantize_mx_both(x.data_ptr(), code, B, R, C, C, q_r.data_ptr(), ld_qr, s_r.data_ptr(),
+                                            ld_r, q_c.data_ptr(), ld_qc, s_c.data_ptr(), ld_c,
+                                            lay | (_lib.DATA_PAIRS if pairs else 0), _stream_handle(dev))
     _lib.check(rc)
     q_r, q_c = q_r.view(torch.float8_e4m3fn), q_c.view(torch.float8_e4m3fn)
     if data.dim() == 2:
