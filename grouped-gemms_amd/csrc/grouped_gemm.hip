@@ -86,8 +86,10 @@ struct Split {
   int units;    // pieces in all (rem * S, or 0)
 };
 
-__host__ __device__ inline Split split_plan(int T, int P, int nsteps, int slots, int tile_kib) {
+// saved: what the plan saves over whole tiles, by the model (ns; 0: no split).
+__host__ __device__ inline Split split_plan(int T, int P, int nsteps, int slots, int tile_kib, int* saved = nullptr) {
   Split sp{T, 1, 0};
+  if (saved) *saved = 0;
   if (T <= 0 || P <= 0 || nsteps < kMinSplitTotal || T / P > kSplitMaxRounds) return sp;
   const int rem = T % P;
   if (rem == 0) return sp;
@@ -116,6 +118,7 @@ __host__ __device__ inline Split split_plan(int T, int P, int nsteps, int slots,
   if (sp.S < 2) return sp;
   sp.dp = T - rem;
   sp.units = rem * sp.S;
+  if (saved) *saved = best;
   return sp;
 }
 
@@ -183,7 +186,7 @@ struct Cfg {
   static constexpr int PB1 = (5 * NMMA + 7) / 8;
   static constexpr int PB2 = 5 * NMMA / 4;
   static_assert(NS == 2, "the main loop alternates between two slots");
-  static_assert(XBYTES % (4096 * NW) == 0 && WBYTES % (4096 * NW) == 0, "copies in runs of four");
+  static_assert(XBYTES % (2048 * NW) == 0 && WBYTES % (2048 * NW) == 0, "even numbers of copies per wave");
   static_assert(PS || ((GSTEPS * BM * 4) % 1024 == 0 && (GSTEPS * BN * 4) % 1024 == 0 && NW % NSD == 0),
                 "scale copies: one operand each, one per wave");
   static_assert(!PS || ((SPW == 2 || SPW == 4) && (BM + BN) % (32 * NW) == 0 && (BM / 32) % SPW == 0),
@@ -1226,7 +1229,7 @@ struct FwdParams {
   uint8_t* out; int out_dtype; int64_t ldo;
   int grid_n; int group_m; int xcd;
   float* part; int par; int slots;          // split: partial slots, resident workgroups, slot count
-  int quads;                                // last round as 128 x 128 quarter tiles (quad_dp)
+  int quads;                                // the last round may run as 128 x 128 quarter tiles (fwd_plan)
   int a_pl; int b_pl;                       // operand layouts: 0 rows, 1 row pairs, 2 row quads (Operand)
   uint32_t as_ld; uint32_t bs_ld;           // plain scales: bytes per row (multiples of 16)
 };
@@ -1303,23 +1306,37 @@ __device__ __forceinline__ bool fwd_tile(const FwdParams& p, int lt, int tiles, 
   return true;
 }
 
-// Tiles of a 256 x 256 launch computed whole when its last round runs as
-// 128 x 128 quarter tiles (fwd_quad_kernel): a reduction too short to split
-// (fewer than kMinSplitTotal steps), at most kSplitMaxRounds full rounds
-// before it, and four quarters per tile of the rem = T % P tiles fit one
-// round.  A lone round of 256 x 256 tiles at K = 2048 takes about as long as
-// a full round (42 us against 38; the copies of one tile per CU are latency
-// bound), its quarters on four times the CUs about 60% of that.
-__host__ __device__ inline int quad_dp(int T, int P) {
-  if (T <= 0 || P <= 0 || T / P > kSplitMaxRounds) return T;
+// The last round of a launch of T tiles of 256 x 256 on P resident workgroups:
+// whole, cut along the reduction (split_plan), or, with `quads`, as 128 x 128
+// quarter tiles (fwd_quad_kernel: dp < T and no units).  Quarters need no
+// partial tiles and no reduce and give a whole tile's bits; up to P / 4 tiles
+// they get a CU each, up to 2 P / 5 half a CU.  Priced per step from kernel
+// times (MI355X; a 128 x 128 step waits on its copies, 0.6 to 0.85 us: 25 to
+// 35 us at K = 5120, 54 at K = 8192 with 8 experts): they must beat the split
+// by kQuadMarginNs.  (1, 2080, 8192, 5120): 96.6 us split, 89.9 quartered; (8,
+// 16640, 2048, 8192): 253 split, 262 quartered.  A reduction too short to
+// split (fewer than kMinSplitTotal steps) takes the quarters whenever they get
+// a CU each: a lone round of 256 x 256 tiles at K = 2048 takes about as long
+// as a full round.
+constexpr int kQuadNsPerStep = 650, kQuad2NsPerStep = 1000, kQuadMarginNs = 8000, kQuadMinGainNs = 3000;
+
+__host__ __device__ inline Split fwd_plan(int T, int P, int nsteps, int slots, int tile_kib, bool quads) {
+  int saved;
+  const Split sp = split_plan(T, P, nsteps, slots, tile_kib, &saved);
+  if (!quads || T <= 0 || P <= 0 || T / P > kSplitMaxRounds) return sp;
   const int rem = T % P;
-  return rem > 0 && 4 * rem <= P ? T - rem : T;
+  if (rem == 0 || 5 * rem > 2 * P) return sp;
+  const bool one = 4 * rem <= P;
+  const int n = nsteps < (1 << 20) ? nsteps : (1 << 20);
+  const int gain = ((int)kTailNsPerStep - (one ? kQuadNsPerStep : kQuad2NsPerStep)) * n;
+  if ((one && nsteps < kMinSplitTotal) || gain >= (saved ? saved + kQuadMarginNs : kQuadMinGainNs))
+    return Split{T - rem, 1, 0};
+  return sp;
 }
 
 template <class C>
 __device__ __forceinline__ Split fwd_split(const FwdParams& p, int tiles) {
-  if (p.quads) return Split{quad_dp(tiles, p.par), 1, 0};
-  return split_plan(tiles, p.par, (int)((p.K + STEP - 1) / STEP), p.slots, C::BM * C::BN * 4 / 1024);
+  return fwd_plan(tiles, p.par, (int)((p.K + STEP - 1) / STEP), p.slots, C::BM * C::BN * 4 / 1024, p.quads != 0);
 }
 
 // Tile tl whole (PIECES = false; epilogue EPI), or piece `piece` of S of it
@@ -2204,12 +2221,20 @@ namespace {
 typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 2> CfgF8_256;
 typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 2> CfgF8_128;
 typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 2> CfgF4_256;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E2M1, 2> CfgF4_128;
 // The same tiles on plain to_mx scales (drop-in calls whose scale rows are
 // 16-byte multiples): no scale re-layout launch; 16 KB scale slots of 8 steps
 // (8 KB for 128 x 128 tiles).
 typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 2, true> CfgF8_256P;
 typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 2, true> CfgF8_128P;
 typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 2, true> CfgF4_256P;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E2M1, 2, true> CfgF4_128P;
+
+// The quarter tiles of a 256 x 256 configuration (void: none).
+template <class C>
+struct QuadCfg {
+  typedef typename std::conditional<C::BM == 256, Cfg<128, 128, 2, 2, C::WFMT, C::NS, C::PS>, void>::type type;
+};
 
 // The scale-independent kernels of a configuration (the reduce): its
 // step-major twin.
@@ -2242,7 +2267,7 @@ const TunedFwd* find_tuned(int E, int64_t M, int64_t N, int64_t K, int b_fmt) {
 // tiles, the 8-XCD swizzle and expert-aligned bands of at most 12 m-blocks
 // (route_tile; 12 beat 8 and 16 on the sweep's jagged groups, and the
 // 256 x 256 tile beats 128 x 128 even at N = K = 2048); 128 x 128 tiles for
-// e4m3 problems too small to fill half the chip with 256 x 256 tiles, unless
+// problems too small to fill half the chip with 256 x 256 tiles, unless
 // the 256 x 256 plan splits that lone round along K.
 // Requests (nonzero bm, bn, gm, xcd) override field by field, and any request
 // leaves the split to the workspace (a tuned "whole tiles only" applies to
@@ -2260,13 +2285,13 @@ FwdChoice pick_fwd(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int bm, in
   const TunedFwd* t = find_tuned(E, M, N, K, b_fmt);
   if (t) {
     c = FwdChoice{t->bm, t->bn, t->group_m, t->xcd, t->split != 0};
-  } else if (b_fmt == MXGG_FMT_E4M3 && M <= 100 * (int64_t)E && E > 1) {
+  } else if (M <= 100 * (int64_t)E && E > 1) {
     // Groups that mostly fit 128 rows: (8, 512, 8192, 5120) 80.7 us as 256 x
     // 256 tiles and 72.9 as 128 x 128, (8, 768) 83.9 and 80.6, (32, 2048, 2880,
     // 2880) 95 and 86; 128 rows on average (8, 1024) 85.7 and 109.
     c.bm = 128;
     c.bn = 128;
-  } else if (b_fmt == MXGG_FMT_E4M3 && tiles256 < 128) {
+  } else if (tiles256 < 128) {
     // Under half a chip of 256 x 256 tiles: 128 x 128 tiles (two per CU)
     // spread the work over 4x the workgroups, unless the 256 x 256 launch
     // splits its lone round along K (a long reduction; judged for the full
@@ -2286,6 +2311,13 @@ FwdChoice pick_fwd(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int bm, in
   if (gm) c.group_m = gm;
   if (xcd) c.xcd = xcd;
   return c;
+}
+
+// Whether the choice's tile may run: 256 x 256, or 128 x 128 -- beside an e2m1
+// weight only where the library picks it, not on request (asked).
+bool tile_built(const FwdChoice& c, int b_fmt, bool asked) {
+  if (c.bm == 256 && c.bn == 256) return true;
+  return c.bm == 128 && c.bn == 128 && (b_fmt == MXGG_FMT_E4M3 || !asked);
 }
 
 // Workgroups of `kernel` (nt threads) resident on the current device at
@@ -2372,25 +2404,20 @@ int launch_fwd(const FwdParams& p0, int grid_m_ub, int gm, int xcd, size_t part_
   const int nsteps = (int)cdiv(p.K, STEP);
   if (p.par <= 0 || p.slots < 2 || nsteps < kMinSplitTotal) p.slots = 0;
   // Rows of every group add up to M in the usual MoE call, with half a tile
-  // of padding per group on average: when the plan for that many tiles does
-  // not split, the piece and reduce launches are skipped (p.slots = 0 makes
-  // the device plan agree).  A wrong guess costs time, never correctness.
-  if (p.slots) {
-    const int64_t est = (cdiv(p.M, C::BM) + (p.E - 1) / 2) * p.grid_n;
-    if (est > INT32_MAX || split_plan((int)est, p.par, nsteps, p.slots, C::BM * C::BN * 4 / 1024).units == 0)
-      p.slots = 0;
-  }
-  // A reduction too short to split: the last round may run as 128 x 128
-  // quarter tiles (quad_dp).  The device decides from the real tile count;
-  // the host, from the usual one, only skips the launch where it cannot help.
+  // of padding per group on average: what the plan does with that many tiles
+  // decides which launches are made (p.slots = 0 / p.quads = 0 make the device
+  // plan, from the real count, agree).  A wrong guess costs time, never
+  // correctness.
+  typedef typename QuadCfg<C>::type Q;
+  constexpr bool kQuads = !std::is_void<Q>::value;
+  const int64_t est = (cdiv(p.M, C::BM) + (p.E - 1) / 2) * p.grid_n;
   p.quads = 0;
-  constexpr bool kQuads = std::is_same<C, CfgF8_256>::value || std::is_same<C, CfgF8_256P>::value;
-  typedef typename std::conditional<C::PS, CfgF8_128P, CfgF8_128>::type Q;
-  if constexpr (kQuads) {
-    if (nsteps < kMinSplitTotal && p.par > 0) {
-      const int64_t est = (cdiv(p.M, C::BM) + (p.E - 1) / 2) * p.grid_n;
-      if (est <= INT32_MAX && quad_dp((int)est, p.par) < est) p.quads = 1;
-    }
+  if (est > INT32_MAX || p.par <= 0) {
+    p.slots = 0;
+  } else {
+    const Split e = fwd_plan((int)est, p.par, nsteps, p.slots, C::BM * C::BN * 4 / 1024, kQuads);
+    p.quads = kQuads && e.units == 0 && e.dp < est;
+    if (e.units == 0) p.slots = 0;
   }
   const int64_t tiles_ub = (int64_t)grid_m_ub * p.grid_n;
   if (tiles_ub <= 0) return MXGG_OK;
@@ -2413,10 +2440,10 @@ int launch_fwd(const FwdParams& p0, int grid_m_ub, int gm, int xcd, size_t part_
 #undef MXGG_WHOLE
   if (int rc = launch_status("grouped_mm")) return rc;
   if constexpr (kQuads) {
-    if (p.quads) {   // 4 * (T % P) <= P quarters
+    if (p.quads) {   // 4 * (T % P) < 2 P quarters
 #define MXGG_QUAD(E)                                                                                        \
   case E:                                                                                                   \
-    hipLaunchKernelGGL((fwd_quad_kernel<C, Q, E>), dim3((unsigned)p.par), dim3(Q::NT), 0, st, p);           \
+    hipLaunchKernelGGL((fwd_quad_kernel<C, Q, E>), dim3((unsigned)(2 * p.par)), dim3(Q::NT), 0, st, p);     \
     break
       MXGG_EPI_SWITCH(epi, MXGG_QUAD)
 #undef MXGG_QUAD
@@ -2432,7 +2459,6 @@ int launch_fwd(const FwdParams& p0, int grid_m_ub, int gm, int xcd, size_t part_
   // expects (at least 128, which costs little when the device plan differs):
   // a 72-tile split (1152 items) took 21 us on 128 workgroups.
   const int64_t items = (int64_t)(p.par / 2) * ReduceShape<C>::CH;
-  const int64_t est = (cdiv(p.M, C::BM) + (p.E - 1) / 2) * p.grid_n;
   const Split esp = split_plan((int)(est < INT32_MAX ? est : INT32_MAX), p.par, nsteps, p.slots,
                                C::BM * C::BN * 4 / 1024);
   int64_t rgrid = esp.S > 0 ? (int64_t)(esp.units / esp.S) * ReduceShape<C>::CH : 0;
@@ -2694,9 +2720,7 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
                              int group_m, int xcd, int layout, void* part_area, size_t part_bytes, hipStream_t st,
                              bool plain = false, int64_t ldas = 0, int64_t ldbs_n = 0, int64_t ldbs_e = 0) {
   FwdChoice c = pick_fwd(E, M, N, K, b_fmt, block_m, block_n, group_m, xcd);
-  const bool built = b_fmt == MXGG_FMT_E2M1 ? (c.bm == 256 && c.bn == 256)
-                                           : ((c.bm == 256 && c.bn == 256) || (c.bm == 128 && c.bn == 128));
-  if (!built) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm: tile %dx%d not built", c.bm, c.bn);
+  if (!tile_built(c, b_fmt, block_m || block_n)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm: tile %dx%d not built", c.bm, c.bn);
   const int64_t T = cdiv(K, STEP);
   float* part = c.split && part_area && part_bytes ? (float*)part_area : nullptr;
   FwdParams p{A, lda, B, ldb_n, ldb_e, as, (uint32_t)(4 * T * M), bs, (uint32_t)(4 * T * N), offs, E, M, N, K,
@@ -2717,6 +2741,7 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
     if (bm_stream)
       return b_fmt == MXGG_FMT_E2M1 ? launch_stream_rows<MXGG_FMT_E2M1, true>(p, bm_stream, c.group_m, c.xcd, st)
                                     : launch_stream_rows<MXGG_FMT_E4M3, true>(p, bm_stream, c.group_m, c.xcd, st);
+    if (b_fmt == MXGG_FMT_E2M1 && c.bm == 128) return launch_fwd<CfgF4_128P>(p, gm128, c.group_m, c.xcd, pb, st);
     if (b_fmt == MXGG_FMT_E2M1) return launch_fwd<CfgF4_256P>(p, gm256, c.group_m, c.xcd, pb, st);
     if (c.bm == 256) return launch_fwd<CfgF8_256P>(p, gm256, c.group_m, c.xcd, pb, st);
     return launch_fwd<CfgF8_128P>(p, gm128, c.group_m, c.xcd, pb, st);
@@ -2724,6 +2749,7 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
   if (bm_stream)
     return b_fmt == MXGG_FMT_E2M1 ? launch_stream_rows<MXGG_FMT_E2M1, false>(p, bm_stream, c.group_m, c.xcd, st)
                                   : launch_stream_rows<MXGG_FMT_E4M3, false>(p, bm_stream, c.group_m, c.xcd, st);
+  if (b_fmt == MXGG_FMT_E2M1 && c.bm == 128) return launch_fwd<CfgF4_128>(p, gm128, c.group_m, c.xcd, pb, st);
   if (b_fmt == MXGG_FMT_E2M1) return launch_fwd<CfgF4_256>(p, gm256, c.group_m, c.xcd, pb, st);
   if (c.bm == 256) return launch_fwd<CfgF8_256>(p, gm256, c.group_m, c.xcd, pb, st);
   return launch_fwd<CfgF8_128>(p, gm128, c.group_m, c.xcd, pb, st);
@@ -2887,15 +2913,14 @@ extern "C" int mxgg_grouped_mm_config(int E, int64_t M, int64_t N, int64_t K, in
     return fail(MXGG_ERR_INVALID_ARG, "grouped_mm_config: null output pointer");
   if (b_fmt != MXGG_FMT_E4M3 && b_fmt != MXGG_FMT_E2M1)
     return fail(MXGG_ERR_INVALID_ARG, "grouped_mm_config: weight format %d not E4M3/E2M1", b_fmt);
+  const bool asked = *block_m || *block_n;
   FwdChoice c = pick_fwd(E, M, N, K, b_fmt, *block_m, *block_n, *group_m,
                          *xcd_swizzle);
   *block_m = c.bm;
   *block_n = c.bn;
   *group_m = c.group_m;
   *xcd_swizzle = c.xcd;
-  const bool built = b_fmt == MXGG_FMT_E2M1 ? (c.bm == 256 && c.bn == 256)
-                                           : ((c.bm == 256 && c.bn == 256) || (c.bm == 128 && c.bn == 128));
-  if (!built) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm_config: tile %dx%d not built", c.bm, c.bn);
+  if (!tile_built(c, b_fmt, asked)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm_config: tile %dx%d not built", c.bm, c.bn);
   return MXGG_OK;
 }
 

@@ -127,6 +127,58 @@ def test_fwd_split_tail_full_size(gpu):
     assert (d <= 2.0 ** -6 * whole.float().abs().amax(dim=1).clamp_min(1.0)).all()
 
 
+@pytest.mark.parametrize("M,N,K,fmt", [
+    (2080, 8192, 4224, "e4m3"),     # 288 tiles: 32 after a full round, 33 steps: quarters beat pieces
+    (4096, 5632, 2048, "e4m3"),     # 352 tiles: 96 after a full round, quarters two to a CU
+    (2080, 8192, 2080, "e2m1"),     # the same beside a packed weight, K % 128 = 32
+])
+def test_fwd_quartered_last_round_full_size(gpu, M, N, K, fmt):
+    """Last rounds of 256 x 256 tiles run as 128 x 128 quarters on MI355X's 256
+    CUs, against an fp32 dequantize -> matmul of the last 256 rows (the tail's)
+    and, for reductions no launch splits, bit for bit against the 128 x 128
+    launch of the whole call (e4m3) or a call of one column block of 256 (e2m1),
+    which run the same multiply sequence per element."""
+    import kernels
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    a = torch.randn((M, K), device=gpu, generator=g).to(torch.bfloat16)
+    b = (torch.randn((1, N, K), device=gpu, generator=g) * 0.05).to(torch.bfloat16)
+    f4 = fmt == "e2m1"
+    sa, qa = kernels.to_mx(a)
+    sb, qb = kernels.to_mx(b, elem_dtype=torch.float4_e2m1fn_x2 if f4 else torch.float8_e4m3fn)
+    offs = torch.tensor([M - 3], dtype=torch.int32, device=gpu)
+    mm = kernels.triton_mxfp8_grouped_mm
+    out = mm(qa, qb, sa, sb, offs)[:M - 3]
+    if not f4:
+        def deq(q, s):
+            return (q.float().reshape(*s.shape, 32) * torch.exp2(s.float() - 127).unsqueeze(-1)).reshape(q.shape)
+        ref = deq(qa[M - 256:M - 3], sa[M - 256:M - 3]) @ deq(qb[0], sb[0]).t()
+        assert ((out[M - 256:].float() - ref).norm() / ref.norm()).item() <= REL_FRO_TIGHT
+        if K < 4096:
+            whole = mm(qa, qb, sa, sb, offs, BLOCK_M=128, BLOCK_N=128)[:M - 3]
+            assert torch.equal(out.view(torch.int16), whole.view(torch.int16))
+    else:
+        for n0 in range(0, N, 1024):
+            part = mm(qa, qb[:, n0:n0 + 256], sa, sb[:, n0:n0 + 256], offs)[:M - 3]
+            assert torch.equal(out[:, n0:n0 + 256].contiguous().view(torch.int16), part.view(torch.int16))
+
+
+@pytest.mark.parametrize("E,M,N,K,out_dtype", [
+    (4, 1000, 300, 640, torch.bfloat16),       # ragged columns and groups, rows off the 16-byte grid
+    (2, 512, 512, 2080, torch.float32),        # K % 128 = 32, re-laid scales
+    (8, 600, 256, 512, torch.float16),         # plain scales, 75 rows per group
+])
+def test_fwd_e2m1_128_tiles_match_256(gpu, E, M, N, K, out_dtype):
+    """Small calls beside a packed weight run 128 x 128 tiles: the bits of the
+    256 x 256 tiles (reductions too short to split)."""
+    import kernels
+    sa, qa = kernels.to_mx(randn_bf16((M, K), 1.0, 3).to(gpu))
+    sb, qb = kernels.to_mx(randn_bf16((E, N, K), 0.05, 4).to(gpu), elem_dtype=torch.float4_e2m1fn_x2)
+    offs = torch.tensor([M * (e + 1) // E - (e % 3) for e in range(E - 1)] + [M], dtype=torch.int32, device=gpu)
+    out = kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=out_dtype)
+    big = kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=out_dtype, BLOCK_M=256, BLOCK_N=256)
+    assert torch.equal(out.view(torch.uint8), big.view(torch.uint8))
+
+
 # ------------------------------------------------- quarter-tile last round
 #
 # A reduction under 32 steps is never split; instead, a last round of at most
