@@ -95,17 +95,17 @@ def time_call(fn, steps: int, warmup: int, flush_buf):
 def fwd_kernel_name(cfg: dict, rows: bool = False) -> str:
     """Device-kernel name (as rocprofv3 lists it) of the whole-tile kernel of an
     e4m3 forward/dgrad launch on step-major scales: Cfg<BLOCK_M, BLOCK_N, waves
-    along M, waves along N, B format, LDS stages, plain scales>, pieces=false,
-    bf16 epilogue; with ``rows`` (row-major A), the 256 x 256 tiles run as
-    XLine (A in two-stage LDS slots, 3 of them).  A call may also launch the
-    piece / quarter-tile / reduce kernels of a split last round; the
-    kernel-only event time covers those too."""
+    along M, waves along N, B format, 64-element half steps in LDS, plain
+    scales>, pieces=false, bf16 epilogue, whatever the data layout; with
+    ``rows``, the name older summaries list the 256 x 256 tiles of row-major A
+    under.  A call may also launch the piece / quarter-tile / reduce kernels of
+    a split last round; the kernel-only event time covers those too."""
     if rows and cfg["BLOCK_M"] == 256:
         return XLINE_KERNEL
     return f"mxgg::fwd_kernel<mxgg::Cfg<{cfg['BLOCK_M']}, {cfg['BLOCK_N']}, 2, 2, 0, 4, false>, false, 1>"
 
 
-# the 256 x 256 e4m3 forward whole-tile kernels: A in row pairs, and row-major A (XLine)
+# the 256 x 256 e4m3 forward whole-tile kernel, and the separate one for row-major A that older summaries list
 FWD_KERNEL = "mxgg::fwd_kernel<mxgg::Cfg<256, 256, 2, 2, 0, 4, false>, false, 1>"
 XLINE_KERNEL = "mxgg::fwd_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>"
 
@@ -115,17 +115,14 @@ WGRAD_KERNEL = "mxgg::wgrad_kernel<mxgg::Cfg<256, 256, 2, 2, 0, 4, false>, false
 WGRAD_XLINE = "mxgg::wgrad_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>"
 
 
-def wgrad_kernel_name(E: int, M: int, N: int, K: int, rows: bool = False) -> str:
+def wgrad_kernel_name(E: int, M: int, N: int, K: int) -> str:
     """Device-kernel name of the whole-tile kernel of a wgrad call of this
     shape: 256 x 256 (WGRAD_KERNEL) or, where the library picks them
-    (mxgg_wgrad_config, needs the GPU), 128 x 128 tiles; with ``rows``
-    (row-major go_t) the 256 x 256 tiles run as XLine (WGRAD_XLINE)."""
+    (mxgg_wgrad_config, needs the GPU), 128 x 128 tiles."""
     import ctypes
     from kernels import _lib
     b = ctypes.c_int32(0)
     _lib.check(_lib.load().mxgg_wgrad_config(E, M, N, K, ctypes.byref(b)))
-    if rows and b.value == 256:
-        return WGRAD_XLINE
     return f"mxgg::wgrad_kernel<mxgg::Cfg<{b.value}, {b.value}, 2, 2, 0, 4, false>, false, 1>"
 
 
@@ -378,11 +375,15 @@ def call_spans(trace_csv: str):
     return spans
 
 
+PLAIN_CFG = re.compile(r"Cfg<(\d+, ?){6}true>")   # a tile configuration on plain scales
+
+
 def dropin_spans(trace_csv: str):
     """Drop-in calls in a ``rocprofv3 --kernel-trace`` CSV that directly
     follow the bench's cache flush (its timed drop-in reps): the scale
-    re-layout launch (which also stages operands in row pairs where the
-    library does), then the call's GEMM dispatches.  Returns {whole-tile
+    re-layout launch (which also stages operands in row pairs with
+    MXGG_STAGING=1) or, for a call on plain scales, none; then the call's GEMM
+    dispatches.  Returns {whole-tile
     kernel of the call: [(re-layout ns, GEMM span ns, start ns), ...]} in
     trace order; a call whose every tile is split counts under the whole-tile
     kernel of its configuration."""
@@ -391,9 +392,11 @@ def dropin_spans(trace_csv: str):
                   for r in csv.DictReader(open(trace_csv)))
     out, i = {}, 0
     while i + 1 < len(rows):
-        if "FillFunctor" in rows[i][2] and rows[i + 1][2].startswith("mxgg::scale_relayout_kernel"):
-            relayout = rows[i + 1][1] - rows[i + 1][0]
-            j, g0, g1, whole, piece, reduced = i + 2, None, None, None, None, False
+        nxt = rows[i + 1][2]
+        plain = gemm_launch(nxt) is not None and PLAIN_CFG.search(nxt) is not None
+        if "FillFunctor" in rows[i][2] and (plain or nxt.startswith("mxgg::scale_relayout_kernel")):
+            relayout = 0 if plain else rows[i + 1][1] - rows[i + 1][0]
+            j, g0, g1, whole, piece, reduced = i + (1 if plain else 2), None, None, None, None, False
             while j < len(rows) and any(rows[j][2].startswith(g) for g in GEMM_KERNELS):
                 t0, t1, n = rows[j]
                 is_whole = gemm_launch(n) == "whole"
@@ -511,23 +514,20 @@ def stats_summary(stats_csv: str, bench_json: str, trace_csv: str = None) -> str
             out.append(text)
     if trace_csv and line and line.get("roofline"):
         # the GEMM launches the drop-in calls make, on the operands as the
-        # call hands them over (staged in row pairs where the library stages
-        # them); the sweep's timed drop-in reps are the first cold ones, and
+        # call hands them over; the sweep's timed drop-in reps are the first cold ones, and
         # its forward + dgrad (wgrad) calls number what the kernel-only
         # roofline counts, over the same shapes
         rf = line["roofline"]
         spans = dropin_spans(trace_csv)
-        out += ["", "Drop-in calls, from the same trace: each timed rep's scale re-layout launch (with any operand "
-                    "staging) and the span of its GEMM launches:"]
+        out += ["", "Drop-in calls, from the same trace: each timed rep's scale re-layout launch (0: a call on plain "
+                    "scales) and the span of its GEMM launches:"]
         for name, v in sorted(spans.items()):
             out.append(f"  {name:62s} calls {len(v):6d}: re-layout avg {sum(x[0] for x in v) / len(v) / 1e3:8.2f} us, "
                        f"GEMM span avg {sum(x[1] for x in v) / len(v) / 1e3:9.2f} us")
-        # the kernel-only sweep's row-major forward + dgrad calls all run the
-        # XLine kernel, their drop-in twins it or, where the call stages A in
-        # row pairs, the one-stage 256 x 256 kernel; the wgrad's likewise (the
-        # one-stage kernel where the call stages both operands): each family's
-        # calls in trace order
-        for fam in ((FWD_KERNEL, XLINE_KERNEL), (WGRAD_KERNEL, WGRAD_XLINE)):
+        # the kernel-only sweep's forward + dgrad calls all run the 256 x 256
+        # kernel on step-major scales, their drop-in twins it or its plain-scale
+        # twin: each family's calls in trace order
+        for fam in ((FWD_KERNEL, FWD_KERNEL.replace("4, false", "4, true")), (WGRAD_KERNEL,)):
             names = {canon(f) for f in fam}
             v = sorted((x for k, xs in spans.items() if canon(k) in names for x in xs), key=lambda x: x[2])
             key = next((k for k in rf["by_kernel"] if canon(k) in names), None)
@@ -793,7 +793,7 @@ def round_sweep(dev, args, flush):
     E=1, M=16384, N=8192 is 2048 tiles of 256 x 256, exactly 8 rounds of the
     256 resident workgroups (no split, no quarter-tile tail), at K = 256 ..
     8192, on row-major data and on the native layout (step-major scales both).
-    A least-squares line over K >= 1024 (the ring runs at least 6 stages)
+    A least-squares line over K >= 1024 (shorter reductions are set-up and epilogue)
     splits a round into a cost per 64-element stage and a fixed cost per tile
     (set-up, the first copies' latency, the epilogue, the dispatch gap)."""
     import torch
@@ -944,7 +944,7 @@ def main():
                     help="run only the sweep on row-pair data (for counter passes of that layout)")
     ap.add_argument("--kernel-only", action="store_true",
                     help="time only the calls on step-major scales (the row-major kernel-only figures), not the "
-                         "drop-in calls, which may stage operands in row pairs: for counter passes of the "
+                         "drop-in calls, whose scales may be re-laid first: for counter passes of the "
                          "row-major layout")
     ap.add_argument("--ep-only", action="store_true",
                     help="run only the expert-parallel shard measurement (E=1, M=2080; for kernel traces of it)")
@@ -1063,7 +1063,7 @@ def main():
                 if "bf16_us" in row:
                     row["fwd_speedup_vs_bf16"] = row["bf16_us"] / row["fwd_us"]
             kernel_only("fwd_kernel_us", lambda: triton_mxfp8_grouped_mm(qa, qw, ta, tw, offs),
-                        fwd_kernel_name(_pick_config(E, M, N, K), rows=True), flops, row)
+                        fwd_kernel_name(_pick_config(E, M, N, K)), flops, row)
             del qa, qw, sa, sw, ta, tw
         if args.only in ("all", "dgrad"):
             go = torch.randn((M, N), device=dev).to(torch.bfloat16)
@@ -1079,7 +1079,7 @@ def main():
                 row["dgrad_us"] = med * 1e3
                 row["dgrad_tflops"] = flops / (med * 1e-3) / 1e12
             kernel_only("dgrad_kernel_us", lambda: triton_mxfp8_grouped_mm(qg, qt, tg, tt, offs),
-                        fwd_kernel_name(_pick_config(E, M, K, N), rows=True), flops, row)
+                        fwd_kernel_name(_pick_config(E, M, K, N)), flops, row)
             del qg, qt, sg, st_, tg, tt
         if args.only in ("all", "wgrad"):
             go = torch.randn((M, N), device=dev).to(torch.bfloat16)
@@ -1095,7 +1095,7 @@ def main():
                 row["wgrad_us"] = med * 1e3
                 row["wgrad_tflops"] = flops / (med * 1e-3) / 1e12
             kernel_only("wgrad_kernel_us", lambda: triton_mxfp8_wgrad(qg, tg, qi, ti, offs),
-                        wgrad_kernel_name(E, M, N, K, rows=True), flops, row)
+                        wgrad_kernel_name(E, M, N, K), flops, row)
             del qg, qi, sg, si, tg, ti
         torch.cuda.empty_cache()
         rows.append(row)
@@ -1164,11 +1164,9 @@ def main():
         "fwd_speedup_vs_bf16_geomean": round(speedup_gm, 3) if speedup_gm else None,
         "fwd_speedup_vs_readme_bf16": round(fwd_gm / REF_BF16_GEOMEAN_TFLOPS, 3) if fwd_gm else None,
         "ref_speedup_vs_bf16_geomean": REF_SPEEDUP_VS_BF16,
-        "drop_in_staging": "inside the timed drop-in calls, the re-layout launch also copies an e4m3 weight "
-                           "(forward / dgrad, E <= M/8192, K >= 4096 or N >= 4096), A (N >= 8192), or both wgrad "
-                           "operands (unless "
-                           "N + K < 10240 and E*(N+K) <= 8192) into row pairs, which the GEMM reads in whole "
-                           "128-byte lines; same bits as without (mxgg_*_staging_size)",
+        "drop_in_staging": "on: operands are copied into row pairs inside the timed drop-in calls (MXGG_STAGING)"
+                           if os.environ.get("MXGG_STAGING", "0") not in ("", "0") else
+                           "off: the drop-in calls read the operands where they lie",
         "kernel_only_geomean_tflops": kernel_geomeans(rows, "_kernel_us"),
         "native_geomean_tflops": kernel_geomeans(rows, "_native_us"),
         "native_layout": "kernel-only time on the layout the kernels read fastest: step-major scales and row-pair "

@@ -5,8 +5,10 @@
 //   * scale re-layout feeding both GEMMs                    (the role of kernels/forward.py:367-397)
 //   * split of an under-filled last round along the reduction, with fp32
 //     partial tiles and a reduce kernel        (generalises kernels/backward.py:106-215)
-//   * forward last round with a reduction too short to split as 128 x 128
-//     quarter tiles (fwd_quad_kernel)
+//   * a forward last round of few tiles as 128 x 128 quarter tiles where that
+//     beats the split (fwd_quad_kernel, fwd_plan)
+//   * forward calls of few rows per group as weight-streaming tiles
+//     (fwd_stream_kernel)
 //
 // Both GEMMs are "NT" products whose two operands are contiguous along the
 // reduction dimension, so they share one main loop:
@@ -130,14 +132,15 @@ __host__ __device__ inline void split_range(int a0, int n, int s, int S, int& a,
   b = a0 + (int)((uint32_t)n * (uint32_t)(s + 1) / (uint32_t)S);
 }
 
-template <int BM_, int BN_, int WGM_, int WGN_, int WFMT_, int NS_, bool PS_ = false>
+template <int BM_, int BN_, int WGM_, int WGN_, int WFMT_, int NH_, bool PS_ = false>
 struct Cfg {
   static constexpr int BM = BM_;        // X rows per tile (output rows)
   static constexpr int BN = BN_;        // W rows per tile (output columns)
   static constexpr int WGM = WGM_;      // waves along rows
   static constexpr int WGN = WGN_;      // waves along columns
   static constexpr int WFMT = WFMT_;    // W element format (X is always e4m3)
-  static constexpr int NS = NS_;        // LDS slots (steps)
+  static constexpr int NH = NH_;        // 64-element half steps held in LDS
+  static constexpr int NS = NH / 2;     // LDS slots (steps)
   // Scale source: false, step-major dwords [step][row] (the re-layout
   // kernel's output or the quantizer's native layout); true, the plain
   // to_mx scales (row r's byte b at r * ld + b, ld a multiple of 16), read
@@ -185,7 +188,7 @@ struct Cfg {
   static constexpr int RD = NMMA / 2;
   static constexpr int PB1 = (5 * NMMA + 7) / 8;
   static constexpr int PB2 = 5 * NMMA / 4;
-  static_assert(NS == 2, "the main loop alternates between two slots");
+  static_assert(NH == 4, "the main loop alternates between two slots");
   static_assert(XBYTES % (2048 * NW) == 0 && WBYTES % (2048 * NW) == 0, "even numbers of copies per wave");
   static_assert(PS || ((GSTEPS * BM * 4) % 1024 == 0 && (GSTEPS * BN * 4) % 1024 == 0 && NW % NSD == 0),
                 "scale copies: one operand each, one per wave");
@@ -2218,28 +2221,28 @@ static size_t fwd_staging_bytes_a(int64_t M, int64_t N, int64_t K, int b_fmt) {
 
 namespace {
 
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 2> CfgF8_256;
-typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 2> CfgF8_128;
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 2> CfgF4_256;
-typedef Cfg<128, 128, 2, 2, MXGG_FMT_E2M1, 2> CfgF4_128;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 4> CfgF8_256;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 4> CfgF8_128;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 4> CfgF4_256;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E2M1, 4> CfgF4_128;
 // The same tiles on plain to_mx scales (drop-in calls whose scale rows are
 // 16-byte multiples): no scale re-layout launch; 16 KB scale slots of 8 steps
 // (8 KB for 128 x 128 tiles).
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 2, true> CfgF8_256P;
-typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 2, true> CfgF8_128P;
-typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 2, true> CfgF4_256P;
-typedef Cfg<128, 128, 2, 2, MXGG_FMT_E2M1, 2, true> CfgF4_128P;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E4M3, 4, true> CfgF8_256P;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E4M3, 4, true> CfgF8_128P;
+typedef Cfg<256, 256, 2, 2, MXGG_FMT_E2M1, 4, true> CfgF4_256P;
+typedef Cfg<128, 128, 2, 2, MXGG_FMT_E2M1, 4, true> CfgF4_128P;
 
 // The quarter tiles of a 256 x 256 configuration (void: none).
 template <class C>
 struct QuadCfg {
-  typedef typename std::conditional<C::BM == 256, Cfg<128, 128, 2, 2, C::WFMT, C::NS, C::PS>, void>::type type;
+  typedef typename std::conditional<C::BM == 256, Cfg<128, 128, 2, 2, C::WFMT, C::NH, C::PS>, void>::type type;
 };
 
 // The scale-independent kernels of a configuration (the reduce): its
 // step-major twin.
 template <class C>
-using StepCfg = Cfg<C::BM, C::BN, C::WGM, C::WGN, C::WFMT, C::NS>;
+using StepCfg = Cfg<C::BM, C::BN, C::WGM, C::WGN, C::WFMT, C::NH>;
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
