@@ -3,8 +3,8 @@
 Counterpart of the reference's tune_worker.py (tune_worker.py:21-109): one
 (E, M, N, K) problem, every launch configuration libmxgg has built, each timed
 as the median device time of a ``mxgg_grouped_mm`` call (scale re-layout
-with the operand staging the drop-in call makes, GEMM, and the piece /
-reduce launches of a split last round) with the caches
+where the call makes one, GEMM, and the piece / reduce launches of a split
+last round; with the drop-in call's operand staging under MXGG_STAGING=1) with the caches
 flushed before every repetition.  The search space is the set of built
 instantiations rather than Triton meta-parameters:
 
@@ -89,6 +89,7 @@ def sweep(E: int, M: int, N: int, K: int, fmt: str = "e4m3", limit: int | None =
     import torch
 
     from kernels import _lib
+    from kernels._common import _staging_enabled
     from utils import benchmark_cuda_function_in_microseconds
 
     dev = torch.device("cuda")
@@ -100,8 +101,8 @@ def sweep(E: int, M: int, N: int, K: int, fmt: str = "e4m3", limit: int | None =
     out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     full = lib.mxgg_grouped_mm_workspace_size(E, M, N, K)
     scales_only = 4 * ((K + 127) // 128) * (M + E * N)
-    # plus the operand staging the drop-in call makes (it keeps the split room)
-    stage = lib.mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt)
+    # plus, where the drop-in call stages operands, its staging (it keeps the split room)
+    stage = lib.mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt) if _staging_enabled() else 0
     ws = torch.empty(max(full + stage, 1), dtype=torch.uint8, device=dev)
     stream = torch.cuda.current_stream().cuda_stream
 
