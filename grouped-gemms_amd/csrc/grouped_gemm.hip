@@ -2168,13 +2168,12 @@ static int64_t staged_ld(int64_t K) { return (K + 63) / 64 * 64; }
 
 // Extra workspace for staging an e4m3 weight in row pairs, or 0 where the
 // call would not gain from it.  Staging copies the weight once (2 E N K
-// bytes of HBM traffic in the re-layout launch the call makes anyway); the
-// GEMM then copies whole 128-byte lines of it.  Measured over the sweep
-// shapes (MI355X, M = 16640, whole drop-in calls): E = 1 and 2 gain 2-10%
-// at K >= 5120 and 2-3% at K = 2048 with N >= 5120 (nothing at N = K = 2048);
-// E = 4 gains on some shapes and loses up to 3% on others: the copy's time
-// over the GEMM's is about 400 E / M (5 TB/s against 2 PFLOP/s), so
-// E <= M / 8192.  256 bytes of slack keep the staged lines 256-byte aligned.
+// bytes of HBM traffic in the re-layout launch the call makes anyway), about
+// 400 E / M of the GEMM's time (5 TB/s against 2 PFLOP/s), so E <= M / 8192 at
+// least.  The main loop copies whole lines of row-major data too, so a call
+// gains less than that now (dgrad (4, 16640, 8192, 8192) 931 us staged, 885
+// not): only callers that ask for the room stage.  256 bytes of slack keep the
+// staged lines 256-byte aligned.
 static size_t fwd_staging_bytes(int E, int64_t M, int64_t N, int64_t K, int b_fmt) {
   if (b_fmt != MXGG_FMT_E4M3 || E <= 0 || N <= 0 || N % 2 || (int64_t)E * 8192 > M) return 0;
   if (K < 2048 || (K < 4096 && N < 4096)) return 0;
@@ -2204,14 +2203,9 @@ static bool plain_pays(int E, int64_t M, int64_t N, int64_t K, int b_fmt) {
 }
 
 // The same for A (M, K), or 0: its copy's time over the GEMM's is about
-// 400 / N, and staging it paid at N >= 8192 on every sweep shape (drop-in
-// call, same box: -1 to -12% at E = 4 and 8, where the weight is not staged;
-// -0.1 to -6% at E = 1 and 2 on top of the staged weight; with e2m1
-// weights, BASELINE config 5 -2.7%), not reliably at N = 5120 (-6% to
-// +1.4%).  A is e4m3 whatever the weight's format.  Not on calls of at most
-// kPlainMaxMacs: their re-layout launch costs more than the row pairs save
-// (E = 1, M = 2080, N = 8192, K = 2048: 57.3 us staged, 52.6 us on plain
-// scales and row-major A).
+// 400 / N, so N >= 8192.  A is e4m3 whatever the weight's format.  Not on calls
+// of at most kPlainMaxMacs, whose re-layout launch alone costs more than row
+// pairs could save.
 static size_t fwd_staging_bytes_a(int64_t M, int64_t N, int64_t K, int b_fmt) {
   if ((b_fmt != MXGG_FMT_E4M3 && b_fmt != MXGG_FMT_E2M1) || M <= 0 || M % 2 || N < 8192 || K < 2048) return 0;
   if (M / 2 > (1 << 22) || K >= (1 << 22)) return 0;   // launch grid, int offsets
@@ -2278,10 +2272,8 @@ const TunedFwd* find_tuned(int E, int64_t M, int64_t N, int64_t K, int b_fmt) {
 template <class C>
 int fwd_resident();
 
-// A tuned entry applies whole on every operand layout, although the sweep
-// timed the drop-in call's (operands staged by the library's rule): calls on
-// different layouts give the same bits, and the tile order can change them --
-// the tiles of a split last round are the last ones in that order.
+// A tuned entry applies whole on every operand layout: calls on different
+// layouts give the same bits, and the tile order can change them -- the tiles of a split last round are the last ones in that order.
 FwdChoice pick_fwd(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int bm, int bn, int gm, int xcd) {
   FwdChoice c{256, 256, 12, 8, true};
   const int64_t tiles256 = (cdiv(M, 256) + E - 1) * cdiv(N, 256);
@@ -2583,15 +2575,11 @@ static size_t split_area(int64_t tiles, size_t tile_bytes, int64_t nsteps) {
 
 // Extra workspace for staging both wgrad operands (go_t (N, M), ia_t (K, M))
 // in row pairs, or 0 where that would not pay.  The copy moves 2 (N + K) M
-// bytes in the scale re-layout launch; the GEMM then copies whole lines of
-// both operands, where on row-major data the XLine kernel copies whole lines
-// of go_t only (kernel-only, row pairs are 13% faster over the sweep).  The
-// copy's time over the GEMM's is about 2000 (N + K) / (N K), so it pays only
-// at N = K = 8192; with 8 or more groups, whose token ranges are short, also
-// at N + K >= 10240.  Measured on the whole drop-in call against staging every
-// shape (MI355X, M = 16640, 36 sweep shapes, same bits on all): -2.1%
-// geomean; without any staging -1.6% (the unstaged calls up to 10% faster,
-// E = 8 at N + K >= 10240 and N = K = 8192 1-4% slower).
+// bytes in the scale re-layout launch, about 2000 (N + K) / (N K) of the
+// GEMM's time, so it is offered at N = K = 8192 and, with 8 or more groups, at
+// N + K >= 10240.  Row-major operands are copied in whole lines too: staging
+// costs 7-9% of a call more than it saves, so only callers that ask for the
+// room stage.
 static size_t wgrad_staging_bytes(int E, int64_t M, int64_t N, int64_t K) {
   if (E <= 0 || M <= 0 || M % 32 || N <= 0 || K <= 0 || N % 2 || K % 2) return 0;
   if (!((N >= 8192 && K >= 8192) || (E >= 8 && N + K >= 10240))) return 0;

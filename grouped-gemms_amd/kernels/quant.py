@@ -23,10 +23,8 @@ and 2i+1 interleaved in 64-byte pieces, returned as the strided view
 ``(*batch, R/2, 2, cdiv(L, 64), 64)`` (``_common._pair_buffer``; the pad
 bytes past L are zero; the pair stride grows by 192 unread bytes where the
 row spans a multiple of 8 cache lines that is not a power of two,
-``_common._row_group_ld``).  The GEMMs stage a 64-element slice of two adjacent
-rows per step, which is then one 128-byte line instead of halves of two:
-13% less time for the forward and 19% for the weight gradient over the
-benchmark shapes, same bits.  Packed e2m1 (32 bytes per 64-element step of a
+``_common._row_group_ld``).  The GEMMs read it 1 to 5% faster than row-major
+data at the longest reductions, same bits.  Packed e2m1 (32 bytes per 64-element step of a
 row) goes in row quads the same way (``data_layout="quads"``, the view
 ``(*batch, R/4, 4, cdiv(L/2, 32), 32)``).  The GEMM wrappers recognise such
 views (with step-major scales).

@@ -36,12 +36,11 @@
  * operands are row-major): an e4m3 operand of R rows (R even) whose rows hold
  * L bytes, with "row stride" ld >= L rounded up to 64, keeps byte k of row r
  * at (r/2)*2*ld + (k/64)*128 + (r%2)*64 + k%64.  The 64-byte pieces of rows 2i
- * and 2i+1 alternate, so the 64-element slice of two adjacent rows that the
- * GEMM stages per step is one 128-byte line (row-major, each is half of two
- * lines).  Bytes L .. L rounded up to 64 of a row are padding, which the
+ * and 2i+1 alternate, so a 64-element slice of two adjacent rows is one
+ * 128-byte line.  Bytes L .. L rounded up to 64 of a row are padding, which the
  * GEMMs do not read (they take the true K, resp. M); the quantizers write
  * zeros there.  Row quads (MXGG_DATA_QUADS, MXGG_B_QUADS) are the same for
- * packed e2m1 data, whose 64-element stage piece of a row is 32 bytes: 4 rows
+ * packed e2m1 data, whose 64-element piece of a row is 32 bytes: 4 rows
  * (R divisible by 4) interleave in 32-byte pieces, byte k of row r at
  * (r/4)*4*ld + (k/32)*128 + (r%4)*32 + k%32, ld = the row's bytes rounded up
  * to 32.
@@ -249,12 +248,12 @@ size_t mxgg_grouped_mm_workspace_size(int E, int64_t M, int64_t N, int64_t K);
 /*
  * Workspace bytes, on top of mxgg_grouped_mm_workspace_size, with which
  * mxgg_grouped_mm stages e4m3 operands in row pairs, or 0 where the copies
- * would not pay for themselves: B (E * N * K rounded up to 64, plus 256) for
+ * are never worth considering: B (E * N * K rounded up to 64, plus 256) for
  * E <= M / 8192 and K >= 4096, or K >= 2048 with N >= 4096 (e4m3 B only); A
  * (M * K rounded up to 64, plus 256) for N >= 8192, K >= 2048, M even and
- * M * N * K above 6e10 (e4m3 or e2m1 B; smaller calls skip the re-layout
- * launch instead, see mxgg_grouped_mm).  The copies then
- * cost a few percent of the GEMM's time and save more.  No counterpart in the
+ * M * N * K above 6e10 (e4m3 or e2m1 B).  With
+ * the kernels of this library the copies cost more than they save where
+ * measured (see mxgg_grouped_mm).  No counterpart in the
  * reference, whose Triton kernel reads its operands where they lie.
  */
 size_t mxgg_grouped_mm_staging_size(int E, int64_t M, int64_t N, int64_t K, int b_fmt);
