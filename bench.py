@@ -359,7 +359,7 @@ def call_spans(trace_csv: str):
             whole = gemm_launch(n) == "whole"
             if cur is not None and whole and cur[2]:
                 close()          # back-to-back calls: a call's whole-tile kernel comes first
-                cur = None
+                cur, prev = None, ""
             if cur is None:
                 cur = [t0, t1, None, "FillFunctor" in prev, None]
             cur[1] = max(cur[1], t1)
