@@ -1047,7 +1047,7 @@ def main():
                 # reference's bench does (bench.py:159-161), but with the weight as a
                 # contiguous (E, K, N) tensor: the reference passes a transposed view
                 # of (E, N, K), and transposed right operands of torch's bf16 batched
-                # products have faulted GPUs of this pool
+                # products have faulted MI355X GPUs
                 wk = w.transpose(-2, -1).contiguous()
                 bmed, _ = time_call(lambda: torch._grouped_mm(a, wk, offs, out_dtype=torch.bfloat16),
                                     args.steps, args.warmup, flush)
