@@ -2987,14 +2987,18 @@ static int check_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* go_s, 
 // row-major operands 7% faster than the split 256 x 256 launch, row pairs 3%
 // slower, taken on both so that the bits do not depend on the layout):
 // 128 x 128 tiles instead, four times as many, two workgroups per CU, whole.
-// So do calls of at most kSmallTokens tokens per group, most of whose time is
-// the start and the store of a tile, which the second workgroup of a CU covers
-// (MI355X, 256 / 128 tiles: (32, 4160, 2880, 2880) 241 / 197 us, (8, 2080,
-// 5120, 5120) 158 / 151, (8, 2080, 2048, 2048) f32 43.5 / 41.3, 520 tokens
-// (32, 16640, 2880, 2880) 327 / 316; 1040 tokens (8, 8320, 5120, 5120) 255 /
-// 280, (8, 8320, 2048, 2048) 50.6 / 53.2).
+// So do calls of at most kSmallTokens tokens per group whose 256 x 256 tiles
+// cover 8% more than the 128 x 128 ones, and of at most half that many in a
+// launch of at most kSmallOutputs outputs: most of a tile's time is its start
+// and its store, which the second workgroup of a CU covers, but a long launch
+// of whole 256 x 256 tiles reads less (MI355X, 256 / 128 tiles: (32, 4160, 2880,
+// 2880) 241 / 196 us, (16, 6048, 800, 1184) 35.6 / 27.8, (32, 16640, 2880, 2880)
+// 314 / 305; (8, 2080, 5120, 5120) 150 / 146, (8, 2080, 8192, 5120) 230 / 226,
+// (8, 2080, 2048, 2048) f32 42 / 39.5; past the lines (32, 16640, 4096, 4096)
+// 515 / 549, (16, 1024, 8192, 8192) 578 / 599, a training step of (32, 5824,
+// 3968, 3104) 965 / 978; 1040 tokens (8, 8320, 5120, 5120) 255 / 280).
 // p: the call's parameters with the 256 x 256 tile counts (replaced here).
-constexpr int64_t kSmallTokens = 640;
+constexpr int64_t kSmallTokens = 640, kSmallOutputs = (int64_t)350 * 1000 * 1000;
 
 static int launch_wgrad_small(WgradParams p, hipStream_t st) {
   typedef CfgF8_128 Q;
@@ -3033,7 +3037,9 @@ static WgradChoice wgrad_choice(int E, int64_t M, int64_t N, int64_t K, int64_t 
   w.dev = E > 1 && slots > 0 && split_plan((int)tiles, par, (int)cdiv(M, STEP) + 1, slots, kib).units > 0;
   const int64_t tiles128 = (int64_t)E * cdiv(N, 128) * cdiv(K, 128);
   w.small = (!w.dev && w.sp.units == 0 && 2 * tiles <= par) || (2 * tiles <= par && tiles128 >= 2 * par) ||
-            (!w.dev && w.sp.units == 0 && M <= kSmallTokens * (int64_t)E);
+            (!w.dev && w.sp.units == 0 && M <= kSmallTokens * (int64_t)E &&
+             (4 * 25 * tiles >= 27 * tiles128 ||
+              (2 * M <= kSmallTokens * (int64_t)E && (double)E * (double)N * (double)K <= (double)kSmallOutputs)));
   return w;
 }
 
