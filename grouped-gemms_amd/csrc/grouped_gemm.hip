@@ -2994,11 +2994,12 @@ static int check_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* go_s, 
 // of whole 256 x 256 tiles reads less (MI355X, 256 / 128 tiles: (32, 4160, 2880,
 // 2880) 241 / 196 us, (16, 6048, 800, 1184) 35.6 / 27.8, (32, 16640, 2880, 2880)
 // 314 / 305; (8, 2080, 5120, 5120) 150 / 146, (8, 2080, 8192, 5120) 230 / 226,
-// (8, 2080, 2048, 2048) f32 42 / 39.5; past the lines (32, 16640, 4096, 4096)
-// 515 / 549, (16, 1024, 8192, 8192) 578 / 599, a training step of (32, 5824,
-// 3968, 3104) 965 / 978; 1040 tokens (8, 8320, 5120, 5120) 255 / 280).
+// (8, 2080, 2048, 2048) f32 42 / 39.5, (32, 5824, 3968, 3104) 311 / 297, a
+// training step of (16, 3616, 5504, 4480) 975 / 941; past the lines (32, 16640,
+// 4096, 4096) 515 / 549, (16, 1024, 8192, 8192) 578 / 599; 1040 tokens (8, 8320,
+// 5120, 5120) 255 / 280).
 // p: the call's parameters with the 256 x 256 tile counts (replaced here).
-constexpr int64_t kSmallTokens = 640, kSmallOutputs = (int64_t)350 * 1000 * 1000;
+constexpr int64_t kSmallTokens = 640, kSmallOutputs = (int64_t)450 * 1000 * 1000;
 
 static int launch_wgrad_small(WgradParams p, hipStream_t st) {
   typedef CfgF8_128 Q;
