@@ -674,9 +674,24 @@ __device__ __forceinline__ void run_step(uint8_t* smem, const Operand& X, const 
   uint32_t xn[C::FM], wn[C::FN];
   step_pos<C, KIND, 0>(smem, X, W, ssr, P, t, F0, F1, xc, wc, xn, wn, acc);
   hold(F1, xc, wc);
-  if constexpr (KIND != kStepLast) {
+  if constexpr (KIND == kStepFull) {
     toggle_reads<C, 0>(P);
     shift_scales<C>(P, xn, wn, xc, wc);
+  } else if constexpr (KIND == kStepNoCopy) {
+    // (outside the loop nothing ties the new scales to the old ones' registers:
+    // hold those until the new ones are written)
+    toggle_reads<C, 0>(P);
+    uint32_t xs[C::FM], ws[C::FN];
+    shift_scales<C>(P, xn, wn, xs, ws);
+    hold(F1, xc, wc);
+#pragma unroll
+    for (int i = 0; i < C::FM; ++i) xc[i] = xs[i];
+#pragma unroll
+    for (int j = 0; j < C::FN; ++j) wc[j] = ws[j];
+  } else {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");   // the last MFMA reads its scales before they are reused
+#endif
   }
   MXGG_SCHED_FENCE();
 }
