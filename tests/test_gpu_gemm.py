@@ -381,6 +381,15 @@ def test_fwd_full_size_cfg5_mxfp4(gpu):
     assert 10 * torch.log10(torch.tensor(hp2 / hp_err2)).item() > 12.0
 
 
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("K", [32, 96, 128, 160, 256])
+def test_fwd_one_and_two_step_reductions(gpu, K, tile):
+    """Reductions of one 128-element step (whole or partial) and of two."""
+    offs = np.array([300, 300, 301, 700], dtype=np.int32)
+    out, ref, _ = _fwd_case(4, 700, 520, K, offs, gpu, seed=K, std_b=0.5, BLOCK_M=tile, BLOCK_N=tile)
+    _assert_close(out, ref)
+
+
 # ---------------------------------------------------------------- wgrad
 
 def _wgrad_case(E, M, N, K, offs, gpu, seed=0, out_dtype=torch.bfloat16):
@@ -487,6 +496,28 @@ def test_wgrad_any_offsets(gpu, M, offs):
             assert (o[e] == 0).all()
         prev = end
     _assert_close(o, ref)
+
+
+@pytest.mark.parametrize("offs", [[32, 64, 96, 128, 256], [5, 9, 9, 100, 256], [128, 129, 255, 256, 256],
+                                  [127, 128, 128, 200, 256]])
+def test_wgrad_groups_inside_one_step(gpu, offs):
+    """Groups that touch one 128-token step: their own tokens only, also where
+    the step's other groups hold NaN scales."""
+    import kernels
+    E, M, N, K = 5, 256, 136, 264
+    out, ref, go, ia = _wgrad_case(E, M, N, K, np.array(offs, dtype=np.int32), gpu, seed=sum(offs))
+    out = f32(out)
+    _assert_close(out, ref)
+    sg, qg = kernels.to_mx_dim0(go.to(gpu))
+    si, qi = kernels.to_mx_dim0(ia.to(gpu))
+    offs_t = torch.tensor(offs, dtype=torch.int32, device=gpu)
+    for g, (lo, hi) in enumerate(zip([0] + offs, offs)):
+        if lo % 32 or hi % 32 or lo == hi:
+            continue
+        sn, sm = sg.clone(), si.clone()
+        sn[:, :lo // 32] = sn[:, hi // 32:] = sm[:, :lo // 32] = sm[:, hi // 32:] = 255
+        got = kernels.triton_mxfp8_wgrad(qg, sn, qi, sm, offs_t)
+        assert np.array_equal(f32(got[g]), out[g]), g
 
 
 # ---------------------------------------------------------------- routing / schedule
