@@ -1109,19 +1109,31 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
         __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(out + ((int64_t)row * ldo + col) * ES));
       }
     } else {
+      // Eight LDS reads, then their stores.  Chunks that only partly lie in the
+      // output (a column count off the 16-byte grid) are the exception: their
+      // per-element branches, skipped one by one, 64 times a wave in f32, cost
+      // more than the stores (wgrad (4, 5280, 2880, 736): f32 50.0 us with them,
+      // 45.1 behind one test, bf16 45.0 and 38.6).
+      const bool parts = cols % EPC != 0;
+      constexpr int IT = FPP * 32 / RPI, NB = IT < 8 ? IT : 8;
+      static_assert(IT % NB == 0, "store batches");
 #pragma unroll
-      for (int it = 0; it < FPP * 32 / RPI; ++it) {
-        const int r = it * RPI + lane / NCH;
-        const int c = lane % NCH;
-        const uint4 v = *reinterpret_cast<const uint4*>(area + r * RB + ((c ^ (r % NCH)) * 16));
-        const int row = wm * C::WTM + i0 * 32 + r;
-        const int col = wn * C::WTN + c * EPC;
-        if (row < rows) {
+      for (int it0 = 0; it0 < IT; it0 += NB) {
+        uint4 v[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int r = (it0 + b) * RPI + lane / NCH;
+          v[b] = *reinterpret_cast<const uint4*>(area + r * RB + (((lane % NCH) ^ (r % NCH)) * 16));
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int row = wm * C::WTM + i0 * 32 + (it0 + b) * RPI + lane / NCH;
+          const int col = wn * C::WTN + (lane % NCH) * EPC;
           uint8_t* p = out + ((int64_t)row * ldo + col) * ES;
-          if (col + EPC <= cols) {
-            *reinterpret_cast<uint4*>(p) = v;
-          } else {
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+          if (row < rows && col + EPC <= cols) {
+            *reinterpret_cast<uint4*>(p) = v[b];
+          } else if (parts && row < rows) {
+            const uint32_t w[4] = {v[b].x, v[b].y, v[b].z, v[b].w};
 #pragma unroll
             for (int e = 0; e < EPC; ++e)
               if (col + e < cols) {

@@ -236,6 +236,30 @@ def test_f32_output_rounds_to_bf16_output(gpu, N, tile):
     assert torch.equal(outs[0], outs[1].float())
 
 
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("tile,N,ldo", [(0, 301, 304), (128, 301, 304), (256, 301, 304), (256, 232, 240), (128, 40, 64)])
+def test_fwd_padded_output_rows(gpu, tile, N, ldo, out_dtype):
+    """Output rows on the 16-byte grid whose columns end inside (301) or between
+    16-byte chunks: the bits of a contiguous output, the padding untouched."""
+    import kernels
+    from kernels import _lib
+    E, M, K = 3, 700, 416
+    offs = torch.tensor([100, 100 + 417, M], dtype=torch.int32, device=gpu)
+    sa, qa = kernels.to_mx(randn_bf16((M, K), 1.0, 1).to(gpu))
+    sb, qb = kernels.to_mx(randn_bf16((E, N, K), 0.1, 2).to(gpu))
+    want = kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=out_dtype, BLOCK_M=tile, BLOCK_N=tile)
+    out = torch.full((M, ldo), 7.0, dtype=out_dtype, device=gpu)
+    ws = torch.empty(_lib.grouped_mm_workspace_size(E, M, N, K), dtype=torch.uint8, device=gpu)
+    code = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16, torch.float32: _lib.DTYPE_F32}[out_dtype]
+    _lib.check(_lib.load().mxgg_grouped_mm(
+        qa.data_ptr(), K, sa.data_ptr(), K // 32, qb.data_ptr(), _lib.FMT_E4M3, K, N * K, sb.data_ptr(), K // 32,
+        N * (K // 32), offs.data_ptr(), E, M, N, K, out.data_ptr(), code, ldo, tile, tile, 0, 0, ws.data_ptr(),
+        ws.numel(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, :N].contiguous().view(torch.uint8), want.view(torch.uint8))
+    assert (out[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("gm", [3, 12])
 def test_fwd_many_groups(gpu, gm):
     """80 groups, a fifth of them empty, sizes 0..96 rows: the in-kernel tile
