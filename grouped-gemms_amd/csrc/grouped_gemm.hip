@@ -953,12 +953,16 @@ __device__ __forceinline__ bool store4_vec(const uint8_t* out, int64_t ldo, int 
                                      : ((ldo % 4) == 0 && ((uintptr_t)out % 8) == 0);
 }
 
-// The lane, computed here: the epilogues start from it, so that none of their
-// addresses is computed, and kept or spilled, before the main loop.
-__device__ __forceinline__ int fresh_lane() {
+// The lane, as an epilogue starts from it.  256 x 256 tiles: a value of its
+// own, so that none of the epilogue's addresses is computed, and kept or
+// spilled, before the main loop.  Smaller tiles have the registers, and the
+// time: their addresses are computed while the first copies fly (wgrad (8,
+// 1280, 2048, 2048), 128 x 128 tiles: 20.5 us, 21.1 computed after the loop).
+template <class C>
+__device__ __forceinline__ int store_lane() {
   int lane = threadIdx.x % kWave;
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" : "+v"(lane));
+  if constexpr (C::FM * C::FN >= 16) asm volatile("" : "+v"(lane));
 #endif
   return lane;
 }
@@ -969,7 +973,7 @@ template <class C, bool BF16_ONLY>
 __device__ __forceinline__ void store_tile(const v16f (&acc)[C::FM][C::FN], uint8_t* out,
                                            int64_t ldo, int rows, int cols, int out_dtype) {
   const int wave = wave_id();
-  const int lane = fresh_lane();
+  const int lane = store_lane<C>();
   const int wm = wave / C::WGN, wn = wave % C::WGN;
   const bool vec = store4_vec(out, ldo, out_dtype);
 #pragma unroll
@@ -1044,7 +1048,7 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
   static_assert(FPP >= 1 && C::FM % FPP == 0, "store staging");
   static_assert(64 % NCH == 0, "store row width");
   const int wave = wave_id();
-  const int lane = fresh_lane();
+  const int lane = store_lane<C>();
   const int wm = wave / C::WGN, wn = wave % C::WGN;
   uint8_t* area = smem + wave * (FPP * 32 * RB);
   // a wave's rows and columns all inside the output: no per-store checks
