@@ -1286,9 +1286,10 @@ struct FwdParams {
   // A scales: step-major [T][M] dwords (T = cdiv(K, 128)), or (plain-scale
   // kernels, Cfg::PS) to_mx's (M, K/32) bytes with row stride as_ld; B
   // scales: step-major [E][T][N] dwords, or plain (E, N, K/32) with row
-  // stride bs_ld.  as_bytes / bs_expert: bytes of A's / of one expert's scales.
+  // stride bs_ld.  as_bytes / bs_bytes: bytes of A's / of one expert's scales
+  // that may be read; bs_expert: bytes from one expert's scales to the next.
   const uint8_t* as; uint32_t as_bytes;
-  const uint8_t* bs; uint32_t bs_expert;
+  const uint8_t* bs; uint32_t bs_bytes; uint32_t bs_expert;
   const int32_t* offs; int E; int64_t M; int64_t N; int64_t K;
   uint8_t* out; int out_dtype; int64_t ldo;
   int grid_n; int group_m; int xcd;
@@ -1414,7 +1415,7 @@ __device__ __forceinline__ void fwd_tile_run(const FwdParams& p, uint8_t* smem, 
   const Operand X = make_operand(p.a, p.lda, p.a_pl, row0, rows);
   const Operand W = make_operand(p.b + (int64_t)tl.expert * p.ldb_e, p.ldb_n, p.b_pl, n0, cols);
   const ScaleSrc xs{make_rsrc(p.as, p.as_bytes), C::PS ? p.as_ld : (uint32_t)p.M, (uint32_t)row0};
-  const ScaleSrc ws{make_rsrc(p.bs + (int64_t)tl.expert * p.bs_expert, p.bs_expert), C::PS ? p.bs_ld : (uint32_t)p.N,
+  const ScaleSrc ws{make_rsrc(p.bs + (int64_t)tl.expert * p.bs_expert, p.bs_bytes), C::PS ? p.bs_ld : (uint32_t)p.N,
                     (uint32_t)n0};
 
   v16f acc[C::FM][C::FN];   // set by step_mainloop
@@ -1721,7 +1722,7 @@ __global__ __launch_bounds__(C::NT) void fwd_stream_kernel(FwdParams p) {
   const Operand X = make_operand(p.a, p.lda, p.a_pl, tl.row0, tl.rows);
   const Operand W = make_operand(p.b + (int64_t)tl.expert * p.ldb_e, p.ldb_n, p.b_pl, tl.n0, tl.cols);
   const ScaleSrc xs{make_rsrc(p.as, p.as_bytes), C::PS ? p.as_ld : (uint32_t)p.M, (uint32_t)tl.row0};
-  const ScaleSrc ws{make_rsrc(p.bs + (int64_t)tl.expert * p.bs_expert, p.bs_expert), C::PS ? p.bs_ld : (uint32_t)p.N,
+  const ScaleSrc ws{make_rsrc(p.bs + (int64_t)tl.expert * p.bs_expert, p.bs_bytes), C::PS ? p.bs_ld : (uint32_t)p.N,
                     (uint32_t)tl.n0};
   v16f acc[C::FM][C::FN];
   stream_mainloop<C>(smem, X, W, xs, ws, (int)p.K, acc);
@@ -2775,8 +2776,8 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
   if (!tile_built(c, b_fmt, block_m || block_n)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm: tile %dx%d not built", c.bm, c.bn);
   const int64_t T = cdiv(K, STEP);
   float* part = c.split && part_area && part_bytes ? (float*)part_area : nullptr;
-  FwdParams p{A, lda, B, ldb_n, ldb_e, as, (uint32_t)(4 * T * M), bs, (uint32_t)(4 * T * N), offs, E, M, N, K,
-              (uint8_t*)out, out_dtype, ldo, 0, 0, 0, part, 0, 0, 0,
+  FwdParams p{A, lda, B, ldb_n, ldb_e, as, (uint32_t)(4 * T * M), bs, (uint32_t)(4 * T * N), (uint32_t)(4 * T * N),
+              offs, E, M, N, K, (uint8_t*)out, out_dtype, ldo, 0, 0, 0, part, 0, 0, 0,
               (layout & MXGG_A_PAIRS) ? 1 : 0, (layout & MXGG_B_PAIRS) ? 1 : ((layout & MXGG_B_QUADS) ? 2 : 0)};
   // no more room than the split plans of this shape can use (ws_layout)
   const size_t cap = fwd_part_cap(E, M, N, K);
@@ -2786,8 +2787,13 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
   const int bm_stream = block_m || block_n ? 0 : stream_rows(E, M);   // not a tile of pick_fwd's
   const int gm256 = (int)(cdiv(M, 256) + E - 1), gm128 = (int)(cdiv(M, 128) + E - 1);
   if (plain) {
-    p.as_bytes = (uint32_t)(M * ldas);
-    p.bs_expert = (uint32_t)(E > 1 ? ldbs_e : N * ldbs_n);
+    // Up to the end of the last row's last 16-byte chunk: copies run past the
+    // rows, K and N of a tile, and what lies behind the last row of a view (its
+    // row stride's rest, the gap to a next expert) need not be the caller's.
+    const int64_t row = (K / 32 + 15) / 16 * 16;
+    p.as_bytes = (uint32_t)((M - 1) * ldas + row);
+    p.bs_bytes = (uint32_t)((N - 1) * ldbs_n + row);
+    p.bs_expert = (uint32_t)(E > 1 ? ldbs_e : 0);
     p.as_ld = (uint32_t)ldas;
     p.bs_ld = (uint32_t)ldbs_n;
     if (bm_stream)

@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import bits_u8, bits_u16, seeded_offs
+from helpers import bits_u8, bits_u16, randn_bf16, seeded_offs
 from oracle import mx_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -158,6 +158,30 @@ def test_fwd_plain_scales_padded_strides(gpu):
     got = kernels.triton_mxfp8_grouped_mm(qa, qw, pa[:, :nb].view(sa.dtype), pw_v.view(sw.dtype), offs_t)
     torch.cuda.synchronize()
     assert torch.equal(want.view(torch.int16), got.view(torch.int16))
+
+
+@pytest.mark.parametrize("E,M,N,K,tile", [(3, 300, 200, 544, 256), (3, 300, 200, 544, 128), (8, 70, 200, 1056, None),
+                                          (2, 600, 300, 8224, 256)])      # the last: pieces of 8-step groups
+def test_fwd_plain_scales_end_with_their_last_row(gpu, E, M, N, K, tile):
+    """Scale views whose storage ends with the last row's last byte, wide rows
+    and gaps between experts holding NaN scales: the contiguous call's bits."""
+    import kernels
+    nb, ld = K // 32, (K // 32 + 47) // 16 * 16
+    offs = torch.tensor([M * (e + 1) // E for e in range(E)], dtype=torch.int32, device=gpu)
+    sa, qa = kernels.to_mx(randn_bf16((M, K), 1.0, 1).to(gpu))
+    sb, qb = kernels.to_mx(randn_bf16((E, N, K), 0.1, 2).to(gpu))
+    va = torch.full(((M - 1) * ld + nb,), 255, dtype=torch.uint8, device=gpu).as_strided((M, nb), (ld, 1))
+    gap = N * ld + 4096
+    vb = torch.full(((E - 1) * gap + (N - 1) * ld + nb,), 255, dtype=torch.uint8,
+                    device=gpu).as_strided((E, N, nb), (gap, ld, 1))
+    va.copy_(sa)
+    vb.copy_(sb)
+    kw = {"BLOCK_M": tile, "BLOCK_N": tile}
+    out = kernels.triton_mxfp8_grouped_mm(qa, qb, va, vb, offs, **kw)
+    ta, _ = kernels.to_mx(randn_bf16((M, K), 1.0, 1).to(gpu), scale_layout="steps")
+    tb, _ = kernels.to_mx(randn_bf16((E, N, K), 0.1, 2).to(gpu), scale_layout="steps")
+    want = kernels.triton_mxfp8_grouped_mm(qa, qb, ta, tb, offs, **kw)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("E,M,N,K,offs", [
