@@ -2371,10 +2371,12 @@ FwdChoice pick_fwd(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int bm, in
 }
 
 // Whether the choice's tile may run: 256 x 256, or 128 x 128 -- beside an e2m1
-// weight only where the library picks it, not on request (asked).
-bool tile_built(const FwdChoice& c, int b_fmt, bool asked) {
+// weight only in calls for which the library picks it by itself (so that its
+// answer, mxgg_grouped_mm_config's, may be passed back as a request).
+bool tile_built(const FwdChoice& c, int E, int64_t M, int64_t N, int64_t K, int b_fmt) {
   if (c.bm == 256 && c.bn == 256) return true;
-  return c.bm == 128 && c.bn == 128 && (b_fmt == MXGG_FMT_E4M3 || !asked);
+  if (c.bm != 128 || c.bn != 128) return false;
+  return b_fmt == MXGG_FMT_E4M3 || pick_fwd(E, M, N, K, b_fmt, 0, 0, 0, 0).bm == 128;
 }
 
 // Workgroups of `kernel` (nt threads) resident on the current device at
@@ -2773,7 +2775,7 @@ static int launch_grouped_mm(const uint8_t* A, int64_t lda, const uint8_t* as, c
                              int group_m, int xcd, int layout, void* part_area, size_t part_bytes, hipStream_t st,
                              bool plain = false, int64_t ldas = 0, int64_t ldbs_n = 0, int64_t ldbs_e = 0) {
   FwdChoice c = pick_fwd(E, M, N, K, b_fmt, block_m, block_n, group_m, xcd);
-  if (!tile_built(c, b_fmt, block_m || block_n)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm: tile %dx%d not built", c.bm, c.bn);
+  if (!tile_built(c, E, M, N, K, b_fmt)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm: tile %dx%d not built", c.bm, c.bn);
   const int64_t T = cdiv(K, STEP);
   float* part = c.split && part_area && part_bytes ? (float*)part_area : nullptr;
   FwdParams p{A, lda, B, ldb_n, ldb_e, as, (uint32_t)(4 * T * M), bs, (uint32_t)(4 * T * N), (uint32_t)(4 * T * N),
@@ -2971,14 +2973,13 @@ extern "C" int mxgg_grouped_mm_config(int E, int64_t M, int64_t N, int64_t K, in
     return fail(MXGG_ERR_INVALID_ARG, "grouped_mm_config: null output pointer");
   if (b_fmt != MXGG_FMT_E4M3 && b_fmt != MXGG_FMT_E2M1)
     return fail(MXGG_ERR_INVALID_ARG, "grouped_mm_config: weight format %d not E4M3/E2M1", b_fmt);
-  const bool asked = *block_m || *block_n;
   FwdChoice c = pick_fwd(E, M, N, K, b_fmt, *block_m, *block_n, *group_m,
                          *xcd_swizzle);
   *block_m = c.bm;
   *block_n = c.bn;
   *group_m = c.group_m;
   *xcd_swizzle = c.xcd;
-  if (!tile_built(c, b_fmt, asked)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm_config: tile %dx%d not built", c.bm, c.bn);
+  if (!tile_built(c, E, M, N, K, b_fmt)) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm_config: tile %dx%d not built", c.bm, c.bn);
   return MXGG_OK;
 }
 

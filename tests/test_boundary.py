@@ -72,6 +72,20 @@ def test_launch_config_query():
         _pick_config(1, 16640, 2048, 2048, b_fmt=3)
 
 
+@pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
+@pytest.mark.parametrize("E,M,N,K", [(4, 1024, 512, 512), (8, 512, 2048, 2048), (2, 512, 4096, 4096), (32, 1146, 992, 5280),
+                                     (1, 16, 2048, 8192), (1, 2080, 2048, 8192), (8, 16640, 8192, 5120), (1, 1, 32, 32)])
+def test_launch_config_answer_is_a_valid_request(fmt, E, M, N, K):
+    """What mxgg_grouped_mm_config answers may be passed back to it, as to a
+    call, and is answered unchanged."""
+    from kernels import _lib
+    from kernels.forward import _pick_config
+    b_fmt = _lib.FMT_E2M1 if fmt == "e2m1" else _lib.FMT_E4M3
+    c = _pick_config(E, M, N, K, b_fmt=b_fmt)
+    again = _pick_config(E, M, N, K, b_fmt=b_fmt, **{k: c[k] for k in ("BLOCK_M", "BLOCK_N", "GROUP_M", "XCD_SWIZZLE")})
+    assert again == c
+
+
 @pytest.mark.parametrize("args,needle", [
     (dict(b_fmt=3), "weight format"),
     (dict(out_dtype=9), "out_dtype"),

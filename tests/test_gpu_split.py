@@ -177,6 +177,8 @@ def test_fwd_e2m1_128_tiles_match_256(gpu, E, M, N, K, out_dtype):
     out = kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=out_dtype)
     big = kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=out_dtype, BLOCK_M=256, BLOCK_N=256)
     assert torch.equal(out.view(torch.uint8), big.view(torch.uint8))
+    asked = kernels.triton_mxfp8_grouped_mm(qa, qb, sa, sb, offs, out_dtype=out_dtype, BLOCK_M=128, BLOCK_N=128)
+    assert torch.equal(asked.view(torch.uint8), big.view(torch.uint8))
 
 
 # ------------------------------------------------- quarter-tile last round
