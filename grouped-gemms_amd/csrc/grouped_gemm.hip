@@ -2352,9 +2352,10 @@ FwdChoice pick_fwd(int E, int64_t M, int64_t N, int64_t K, int b_fmt, int bm, in
     // Under half a chip of 256 x 256 tiles: 128 x 128 tiles (two per CU)
     // spread the work over 4x the workgroups, unless the 256 x 256 launch
     // splits its lone round along K (a long reduction; judged for the full
-    // workspace that mxgg_grouped_mm_workspace_size recommends).  E=1, M=2080 (one
-    // GPU's share of E=8 under 8-way expert parallelism), N=2048: K=5120
-    // 77 -> 54 us; K=8192 splits (70 us, against 76 us as 128 x 128).
+    // workspace that mxgg_grouped_mm_workspace_size recommends; the launch may
+    // then still prefer quarter tiles, see fwd_plan).  E=1, M=2080 (one GPU's
+    // share of E=8 under 8-way expert parallelism), N=2048: K=5120 77 -> 54 us;
+    // K=8192 splits (70 us, against 76 us as 128 x 128).
     const int par = fwd_resident<CfgF8_256>();
     const int slots = (int)(kSplitBytes / ((size_t)256 * 256 * 4));
     if (split_plan((int)tiles256, par > 0 ? par : 256, (int)cdiv(K, STEP), slots, 256).units == 0) {
@@ -2483,14 +2484,15 @@ int launch_fwd(const FwdParams& p0, int grid_m_ub, int gm, int xcd, size_t part_
   if (tiles_ub > INT32_MAX) return fail(MXGG_ERR_UNSUPPORTED, "grouped_mm: grid too large");
   // The device's tile count is m * grid_n for some m <= grid_m_ub (each
   // group adds whole m-blocks of grid_n tiles).  When every such count is
-  // below one round and its plan splits, no tile runs whole: the whole-tile
-  // launch would only route and exit (4.5 us on the expert-parallel shard's
-  // N = 2048, K = 8192 call), so it is left out.
+  // below one round and its plan splits or quarters it, no tile runs whole: the
+  // whole-tile launch would only route and exit (4.5 us on the expert-parallel
+  // shard's N = 2048, K = 8192 call), so it is left out.  (E = 1, M = N = 2048,
+  // K = 8192, quarter tiles: 41.0 us with that launch, 39.7 without, 51.0 split.)
   bool whole = true;
-  if (p.slots && tiles_ub < p.par) {
+  if ((p.slots || p.quads) && tiles_ub < p.par) {
     whole = false;
     for (int m = 1; m <= grid_m_ub && !whole; ++m)
-      if (split_plan(m * p.grid_n, p.par, nsteps, p.slots, C::BM * C::BN * 4 / 1024).units == 0) whole = true;
+      if (fwd_plan(m * p.grid_n, p.par, nsteps, p.slots, C::BM * C::BN * 4 / 1024, p.quads != 0).dp != 0) whole = true;
   }
   const int epi = pick_epi(p.out_dtype, p.ldo, p.out);
 #define MXGG_WHOLE(E) \

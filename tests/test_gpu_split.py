@@ -131,6 +131,7 @@ def test_fwd_split_tail_full_size(gpu):
     (2080, 8192, 4224, "e4m3"),     # 288 tiles: 32 after a full round, 33 steps: quarters beat pieces
     (4096, 5632, 2048, "e4m3"),     # 352 tiles: 96 after a full round, quarters two to a CU
     (2080, 8192, 2080, "e2m1"),     # the same beside a packed weight, K % 128 = 32
+    (2048, 2048, 8192, "e4m3"),     # 64 tiles, a lone round: no whole-tile launch
 ])
 def test_fwd_quartered_last_round_full_size(gpu, M, N, K, fmt):
     """Last rounds of 256 x 256 tiles run as 128 x 128 quarters on MI355X's 256
