@@ -2681,6 +2681,13 @@ extern "C" size_t mxgg_grouped_mm_workspace_size(int E, int64_t M, int64_t N, in
   return part ? align256(sc) + part : sc;
 }
 
+extern "C" size_t mxgg_grouped_mm_tile_workspace_size(int E, int64_t M, int64_t N, int64_t K, int block_m,
+                                                      int block_n) {
+  if (E <= 0 || M < 0 || N < 0 || K < 0) return 0;
+  if (!block_m && !block_n && stream_rows(E, M)) return fwd_scale_bytes(E, M, N, K);   // never split
+  return mxgg_grouped_mm_workspace_size(E, M, N, K);
+}
+
 // Where the parts of a caller's workspace go (plain-scale entry points): the
 // re-laid scales (`need` bytes) first; then, 256-byte aligned, the partial
 // tiles, given at most `cap` bytes; then, from the bytes past those, the

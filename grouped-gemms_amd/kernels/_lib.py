@@ -58,6 +58,7 @@ SIGNATURES = {
     "mxgg_tile_schedule": (_c_i32, [_c_p, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
                                     _c_p, _c_p]),
     "mxgg_grouped_mm_workspace_size": (_c_sz, [_c_i32, _c_i64, _c_i64, _c_i64]),
+    "mxgg_grouped_mm_tile_workspace_size": (_c_sz, [_c_i32, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32]),
     "mxgg_grouped_mm_staging_size": (_c_sz, [_c_i32, _c_i64, _c_i64, _c_i64, _c_i32]),
     "mxgg_grouped_mm": (_c_i32, [_c_p, _c_i64, _c_p, _c_i64,
                                  _c_p, _c_i32, _c_i64, _c_i64,
@@ -135,8 +136,8 @@ def calls():
 
 
 @functools.lru_cache(maxsize=1024)
-def grouped_mm_workspace_size(E: int, M: int, N: int, K: int) -> int:
-    return load().mxgg_grouped_mm_workspace_size(E, M, N, K)
+def grouped_mm_workspace_size(E: int, M: int, N: int, K: int, block_m: int = 0, block_n: int = 0) -> int:
+    return load().mxgg_grouped_mm_tile_workspace_size(E, M, N, K, block_m, block_n)
 
 
 @functools.lru_cache(maxsize=1024)

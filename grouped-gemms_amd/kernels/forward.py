@@ -9,7 +9,7 @@ none), then the GEMM, which builds the expert->tile routing inside the kernel fr
 ``group_end_offsets`` (no host sync), and, when the last round of tiles is
 split along K, the piece and reduce launches.  The per-call workspace (torch's
 caching allocator) holds the re-laid scales and up to 128 MiB of fp32 partial
-tiles; ``MXGG_STAGING=1`` in the environment adds room for the library to copy
+tiles (none for a few rows per group); ``MXGG_STAGING=1`` in the environment adds room for the library to copy
 operands into row pairs first (``mxgg_grouped_mm_staging_size``; same bits).
 
 Beyond the reference, the weight may be MXFP4: ``weight`` of dtype
@@ -169,7 +169,7 @@ def triton_mxfp8_grouped_mm(
     # scratch for the scales re-laid step-major and the fp32 partial tiles of a
     # split last round (overwritten by the call; torch's caching allocator
     # makes the per-call allocation cheap)
-    ws_bytes = _lib.grouped_mm_workspace_size(E, M, N, K)
+    ws_bytes = _lib.grouped_mm_workspace_size(E, M, N, K, bm, bn)
     if steps:
         a_ss, b_ss = input_act_scales.contiguous(), weight_scales.contiguous()
         ws_bytes = _split_room(ws_bytes, 4 * T * (M + E * N))
@@ -189,7 +189,8 @@ def triton_mxfp8_grouped_mm(
     # plus, with MXGG_STAGING=1, room to stage the weight and / or A in row
     # pairs (sizes below either bound stage nothing)
     if (M >= 8192 * E or M * N * K > 60_000_000_000) and _staging_enabled():
-        ws_bytes += _lib.load().mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt)
+        lib = _lib.load()
+        ws_bytes = lib.mxgg_grouped_mm_workspace_size(E, M, N, K) + lib.mxgg_grouped_mm_staging_size(E, M, N, K, b_fmt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
     rc = calls.mxgg_grouped_mm(
         a.data_ptr(), lda, a_s.data_ptr(), sas[0],

@@ -246,6 +246,13 @@ int mxgg_grouped_mm_config(int E, int64_t M, int64_t N, int64_t K, int b_fmt, in
  */
 size_t mxgg_grouped_mm_workspace_size(int E, int64_t M, int64_t N, int64_t K);
 /*
+ * The same for a call with this tile request (0, 0: none): the recommended
+ * size, or the scales alone where the call runs weight-streaming tiles (few
+ * rows per group, see mxgg_grouped_mm_config), which are never cut along K.
+ * More room changes nothing for such a call.  No counterpart in the reference.
+ */
+size_t mxgg_grouped_mm_tile_workspace_size(int E, int64_t M, int64_t N, int64_t K, int block_m, int block_n);
+/*
  * Workspace bytes, on top of mxgg_grouped_mm_workspace_size, with which
  * mxgg_grouped_mm stages e4m3 operands in row pairs, or 0 where the copies
  * are never worth considering: B (E * N * K rounded up to 64, plus 256) for

@@ -126,6 +126,13 @@ def test_grouped_mm_workspace_without_gpu():
     # M=N=256, K=4096: 32 steps -> 8 pieces; one 256x256 tile (8 x 256 KiB) or
     # four 128x128 tiles (32 x 64 KiB): 2 MiB after 65536 bytes of scales
     assert lib.mxgg_grouped_mm_workspace_size(1, 256, 256, 4096) == 4 * 32 * (256 + 256) + 2 * MiB
+    # few rows per group and no tile request: weight-streaming tiles, never split -> scales only
+    tile_size = lib.mxgg_grouped_mm_tile_workspace_size
+    for E, M in ((8, 64), (8, 384), (1, 32), (32, 100)):
+        sc, full = 4 * 40 * (M + E * 8192), lib.mxgg_grouped_mm_workspace_size(E, M, 8192, 5120)
+        assert tile_size(E, M, 8192, 5120, 0, 0) == sc < full
+        assert tile_size(E, M, 8192, 5120, 256, 256) == tile_size(E, M, 8192, 5120, 128, 128) == full
+    assert tile_size(8, 385, 8192, 5120, 0, 0) == lib.mxgg_grouped_mm_workspace_size(8, 385, 8192, 5120)
     # wgrad E=4, M=16640: 33 steps per average group -> 8 pieces; 640 tiles -> cap
     assert lib.mxgg_wgrad_workspace_size(4, 16640, 2048, 5120) == 4 * 130 * (2048 + 5120) + 128 * MiB
     # wgrad E=8, N=K=256: 8 tiles; with several groups the room is sized for one

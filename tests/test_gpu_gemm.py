@@ -210,6 +210,25 @@ def test_few_rows_match_general_tiles(gpu, E, M, N, K, elem, out_dtype):
         assert torch.equal(mm(pa, qb, ta, tb, offs, out_dtype=out_dtype).view(torch.uint8), out.view(torch.uint8))
 
 
+def test_few_rows_workspace_holds_scales_only(gpu):
+    """A call of few rows per group, whose tiles are never split, allocates its
+    output and the scale room: no partial-tile room (128 MiB at this shape)."""
+    import kernels
+    E, M, N, K = 8, 64, 2048, 5120
+    sa, qa = kernels.to_mx(randn_bf16((M, K), 1.0, 1).to(gpu))
+    sb, qb = kernels.to_mx(randn_bf16((E, N, K), 0.05, 2).to(gpu))
+    offs = _routed(E, M, 3).to(gpu)
+    for scales in ((sa, sb), tuple(kernels.to_mx(x, scale_layout="steps")[0]
+                                   for x in (randn_bf16((M, K), 1.0, 1).to(gpu), randn_bf16((E, N, K), 0.05, 2).to(gpu)))):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = kernels.triton_mxfp8_grouped_mm(qa, qb, *scales, offs)
+        used = torch.cuda.max_memory_allocated() - before
+        assert used <= out.numel() * 2 + 4 * (K // 128) * (M + E * N) + 2048, used
+        del out
+
+
 @pytest.mark.parametrize("N", [512, 300, 301, 96])     # whole tiles, 16-byte rows, rows off the grid, one narrow tile
 @pytest.mark.parametrize("tile", [128, 256])
 def test_f32_output_rounds_to_bf16_output(gpu, N, tile):
