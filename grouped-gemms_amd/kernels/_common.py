@@ -41,13 +41,14 @@ def _rowmajor(t: torch.Tensor) -> tuple:
     """``(t, its strides in bytes)`` with unit stride along the last dim (the MX
     block dim); other strides kept.  e4m3, e8m0 and packed fp4 tensors are
     taken as bytes (kernels/forward.py:534-535); a wider type as its bytes."""
+    st = t.stride()
+    if st and st[-1] != 1 and t.shape[-1] > 1:
+        t = t.contiguous()
+        st = t.stride()
     if t.element_size() != 1:
         t = t.view(torch.uint8)
-    st = t.stride()
-    if not st or st[-1] == 1 or t.shape[-1] <= 1:
-        return t, st
-    t = t.contiguous()
-    return t, t.stride()
+        st = t.stride()
+    return t, st
 
 
 def _staging_enabled() -> bool:

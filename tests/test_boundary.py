@@ -414,3 +414,20 @@ def test_generate_jagged_offs_same_draws_as_reference_algorithm():
     assert o.tolist() == want and o.dtype == torch.int32
     with pytest.raises(ValueError):
         utils.generate_jagged_offs(2, 100, device="cpu")
+
+
+def test_rowmajor_takes_wide_types_of_any_strides():
+    """A type wider than a byte is taken as its bytes, made contiguous first
+    where its last dim is strided; byte tensors keep their strides."""
+    import torch
+    from kernels._common import _rowmajor
+    x = torch.arange(24, dtype=torch.int16).reshape(4, 6)
+    t, st = _rowmajor(x.t())
+    assert st == (8, 1) and torch.equal(t, x.t().contiguous().view(torch.uint8))
+    t, st = _rowmajor(x[:, :4])
+    assert st == (12, 1) and t.data_ptr() == x.data_ptr()
+    b = torch.zeros((4, 32), dtype=torch.uint8)
+    t, st = _rowmajor(b[:, :16])
+    assert st == (32, 1) and t.data_ptr() == b.data_ptr()
+    t, st = _rowmajor(b.t())
+    assert st == (4, 1)
