@@ -121,16 +121,17 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
 
 
 def calls():
-    """The launching entry points as a CPython module (csrc/pycalls.c, built
-    and linked beside libmxgg.so): the same functions and arguments as the
-    ctypes ones, without their per-argument conversions."""
+    """The launching entry points of libmxgg.so: the CPython module built and
+    linked beside it (csrc/pycalls.c), which spares the per-argument conversions
+    of ctypes, or, for an interpreter it was not built for, the ctypes functions
+    themselves.  Same names and arguments."""
     global _calls
     if _calls is None:
-        load()
+        lib = load()
         try:
             from . import _calls as m
-        except ImportError as e:
-            raise NotImplementedError(f"kernels/_calls is not built (run make -C grouped-gemms_amd/csrc): {e}") from e
+        except ImportError:
+            m = lib
         _calls = m
     return _calls
 
@@ -147,7 +148,7 @@ def wgrad_workspace_size(E: int, M: int, N: int, K: int) -> int:
 
 def available() -> bool:
     try:
-        calls()
+        load()
         return True
     except (NotImplementedError, OSError):
         return False

@@ -431,3 +431,34 @@ def test_rowmajor_takes_wide_types_of_any_strides():
     assert st == (32, 1) and t.data_ptr() == b.data_ptr()
     t, st = _rowmajor(b.t())
     assert st == (4, 1)
+
+
+def test_interpreter_without_the_call_module_uses_ctypes(monkeypatch):
+    """The CPython module belongs to one interpreter; any other calls the same
+    functions through ctypes."""
+    import sys
+    import kernels
+    from kernels import _lib
+    monkeypatch.setattr(_lib, "_calls", None)
+    monkeypatch.delattr(kernels, "_calls", raising=False)
+    monkeypatch.setitem(sys.modules, "kernels._calls", None)      # import fails
+    c = _lib.calls()
+    assert c is _lib.load() and _lib.available()
+    assert c.mxgg_quantize_mx(None, 0, 0, 64, 64, 0, None, 64, None, 2, 0, None) == 0
+
+
+def test_library_builds_without_python_headers():
+    """The library's build needs no Python: without headers the call module is
+    left out, and with them its name carries the interpreter's tag."""
+    import subprocess
+    import sys
+    import sysconfig
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "grouped-gemms_amd", "csrc")
+
+    def dry(*args):
+        return subprocess.run(["make", "-n", "-B", "-C", csrc, *args], capture_output=True, text=True, check=True).stdout
+
+    bare = dry("PYINC=/nonexistent")
+    assert "libmxgg.so" in bare and "pycalls.c" not in bare
+    if os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        assert "_calls" + sysconfig.get_config_var("EXT_SUFFIX") in dry(f"PYTHON={sys.executable}")
