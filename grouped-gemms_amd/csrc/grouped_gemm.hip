@@ -310,6 +310,8 @@ struct Plan {
 // state after a write at the earliest).  The copies are issued in asm: M0 then
 // changes where it must and not per copy, and the compiler, which does not
 // see them, adds no waits of its own.  Callers order them with vmcnt waits.
+// (M0 is reserved: the compiler keeps no value of its own in it, and warns of a
+// declared clobber.)
 __device__ __forceinline__ void set_m0(uint32_t lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds));

@@ -84,3 +84,27 @@ def test_accumulators_are_cleared_and_read_once(code):
         moves = sum(x[0].startswith("v_accvgpr") for x in ins)
         assert moves <= (3 if "wgrad" in name else 2) * 256 + 16, (name, moves)
     assert seen
+
+
+def test_lds_copies_find_their_scalar_operands(code):
+    """The hardware needs five wait states between a vector instruction that
+    writes a scalar register and a copy that reads it, and one between a write
+    of M0 and an LDS copy; the compiler adds none around asm.  M0 is written
+    for the copies only."""
+    seen, bad = 0, []
+    for name, ins in code.items():
+        for i, x in enumerate(ins):
+            if x[0].startswith(("s_", "v_readfirstlane")) and len(x) > 1 and x[1] == "m0,":
+                if ins[i + 1][0] != "s_nop":
+                    bad.append((name, " ".join(x), " ".join(ins[i + 1])))
+            if not (x[0].startswith("buffer_load") and "lds" in x[-1]):
+                continue
+            seen += 1
+            reads = set().union(*(_regs(t, "s") for t in x[1:]))
+            slots, k = 0, i - 1
+            while slots < 5 and k >= 0:
+                if ins[k][0].startswith("v_") and len(ins[k]) > 1 and _regs(ins[k][1], "s") & reads:
+                    bad.append((name, " ".join(ins[k]), " ".join(x), slots))
+                slots += _idle(ins[k])
+                k -= 1
+    assert seen and not bad, bad[:5]
