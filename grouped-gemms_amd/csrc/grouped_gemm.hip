@@ -3066,19 +3066,29 @@ static int check_wgrad(const uint8_t* go_t, int64_t ld_go, const uint8_t* go_s, 
 // row-major operands 7% faster than the split 256 x 256 launch, row pairs 3%
 // slower, taken on both so that the bits do not depend on the layout):
 // 128 x 128 tiles instead, four times as many, two workgroups per CU, whole.
-// So do calls of at most kSmallTokens tokens per group whose 256 x 256 tiles
-// cover 8% more than the 128 x 128 ones, and of at most half that many in a
-// launch of at most kSmallOutputs outputs: most of a tile's time is its start
-// and its store, which the second workgroup of a CU covers, but a long launch
-// of whole 256 x 256 tiles reads less (MI355X, 256 / 128 tiles: (32, 4160, 2880,
-// 2880) 241 / 196 us, (16, 6048, 800, 1184) 35.6 / 27.8, (32, 16640, 2880, 2880)
-// 314 / 305; (8, 2080, 5120, 5120) 150 / 146, (8, 2080, 8192, 5120) 230 / 226,
-// (8, 2080, 2048, 2048) f32 42 / 39.5, (32, 5824, 3968, 3104) 311 / 297, a
-// training step of (16, 3616, 5504, 4480) 975 / 941; past the lines (32, 16640,
-// 4096, 4096) 515 / 549, (16, 1024, 8192, 8192) 578 / 599; 1040 tokens (8, 8320,
-// 5120, 5120) 255 / 280).
+// So do calls of at most kSmallTokens tokens per group with few outputs:
+// kSmallOutputs, or kSmallOutputs8 with at most 8 groups.  Most of such a
+// tile's time is its start and its store, which the second workgroup of a CU
+// covers; 256 x 256 tiles read half as much and win in longer launches, the
+// sooner the more groups there are.  Time as 256 x 256 over time as 128 x 128
+// tiles, groups of 64 to 320 tokens, even and uneven (MI355X):
+//   outputs   E = 8          E = 16         E = 32
+//   3.4e7     1.01 .. 1.29
+//   7e7       1.01 .. 1.17   0.95 .. 1.22
+//   1.3e8     0.98 .. 1.10                  0.90 .. 1.00
+//   1.5e8                    0.91 .. 1.00
+//   2.1e8     1.04
+//   2.7e8                    0.94 .. 1.01
+//   3.0e8                                   0.90 .. 0.95
+//   3.4e8     1.03
+// E = 4 to 6.7e7 outputs 0.98 .. 1.32.  Whole training steps agree in sign
+// where they differ by more than 1%: (8, 2080, 5120, 5120) 495 / 488 us, (32,
+// 2080, 4096, 4096) 1090 / 1110, (32, 5824, 3968, 3104) 943 / 958; (16, 3616,
+// 5504, 4480) 903 / 893, its gradient alone 275 / 298.  More tokens: (16, 5120,
+// 4096, 4096) 184 / 192, (32, 16640, 2880, 2880) 261 / 293.
 // p: the call's parameters with the 256 x 256 tile counts (replaced here).
-constexpr int64_t kSmallTokens = 640, kSmallOutputs = (int64_t)450 * 1000 * 1000;
+constexpr int64_t kSmallTokens = 320, kSmallOutputs = (int64_t)100 * 1000 * 1000,
+                  kSmallOutputs8 = (int64_t)350 * 1000 * 1000;
 
 static int launch_wgrad_small(WgradParams p, hipStream_t st) {
   typedef CfgF8_128 Q;
@@ -3118,8 +3128,7 @@ static WgradChoice wgrad_choice(int E, int64_t M, int64_t N, int64_t K, int64_t 
   const int64_t tiles128 = (int64_t)E * cdiv(N, 128) * cdiv(K, 128);
   w.small = (!w.dev && w.sp.units == 0 && 2 * tiles <= par) || (2 * tiles <= par && tiles128 >= 2 * par) ||
             (!w.dev && w.sp.units == 0 && M <= kSmallTokens * (int64_t)E &&
-             (4 * 25 * tiles >= 27 * tiles128 ||
-              (2 * M <= kSmallTokens * (int64_t)E && (double)E * (double)N * (double)K <= (double)kSmallOutputs)));
+             (double)E * (double)N * (double)K <= (double)(E <= 8 ? kSmallOutputs8 : kSmallOutputs));
   return w;
 }
 

@@ -357,8 +357,9 @@ size_t mxgg_wgrad_staging_size(int E, int64_t M, int64_t N, int64_t K);
  * mxgg_wgrad_steps call of this shape given the recommended workspace
  * (mxgg_wgrad_workspace_size): 128 x 128 tiles where 256 x 256 tiles would
  * fill at most half the chip and either no tile of them is cut along the
- * tokens or 128 x 128 tiles fill at least one round; else 256 x 256.  Reads
- * the device's resident workgroup count (MXGG_ERR_NO_DEVICE without one).
+ * tokens or 128 x 128 tiles fill at least one round, and in calls of short
+ * groups (320 tokens on average) with few outputs (1e8, or 3.5e8 with at most
+ * 8 groups); else 256 x 256.  Reads the device's resident workgroup count (MXGG_ERR_NO_DEVICE without one).
  * Replaces the tile and split choice of `triton_mxfp8_wgrad`
  * (kernels/backward.py:245-254), as mxgg_grouped_mm_config does the
  * forward's.

@@ -454,6 +454,12 @@ def _wgrad_case(E, M, N, K, offs, gpu, seed=0, out_dtype=torch.bfloat16):
     (1, 2080, 2048, 2048, 128),     # 17 steps: too short to split, 64 tiles of 256
     (4, 16640, 2048, 2048, 256),    # 256 tiles: a full round
     (8, 16640, 8192, 8192, 256),
+    (8, 2080, 5120, 5120, 128),     # short groups: 2.1e8 outputs of 8 groups
+    (8, 2080, 8192, 8192, 256),     # ... 5.4e8
+    (16, 4096, 2048, 2048, 128),    # 256 tokens a group, 6.7e7 outputs
+    (32, 8192, 2048, 2048, 256),    # the same groups, 1.3e8 outputs
+    (16, 6048, 2048, 2048, 256),    # 378 tokens a group
+    (32, 4160, 2880, 2880, 256),    # columns that fill neither tile
 ])
 def test_wgrad_config_tiles(gpu, E, M, N, K, block):
     """mxgg_wgrad_config on MI355X (256 CUs, one 256 x 256 workgroup each)."""
