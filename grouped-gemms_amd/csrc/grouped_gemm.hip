@@ -2421,7 +2421,11 @@ int split_slots(size_t bytes) {
 // 37.7 / 39.9; (16, 50, 544, 5216) e2m1 56 / 20 / 23; (1, 16, 2048, 8192) 28.6
 // / 23.3 / 28.3; (8, 256, 8192, 5120) 76.5 / 80 / 66.6, (8, 384) 78.7 / 86 /
 // 68.9, (32, 1024, 2880, 2880) 90 / 79 / 70.5; 64 rows per group (8, 512) 80.7
-// / 102 / 86: not past 48.
+// / 102 / 86: not past 48.  The average is of balanced routing: with half the
+// rows in one group 64-row and 128 x 128 tiles are level ((8, 384, 8192, 5120)
+// 80 / 95, (32, 1024, 2880, 2880) 69 / 67, (32, 1536, 8192, 5120) 304 / 297, even
+// groups 252 / 264), with all of them in one, where they re-read its weight once
+// per 64 rows, 64-row tiles lose ((8, 384) 38 / 25 us, (32, 1536) 116 / 68).
 static int stream_rows(int E, int64_t M) {
   if (M <= 32 || M <= 8 * (int64_t)E) return 32;
   return M <= 48 * (int64_t)E ? 64 : 0;

@@ -119,9 +119,10 @@ def emit_header(best: dict, source: str = "", min_gain: float | None = None) -> 
     rows.sort()
     lines = [
         "// Tuned forward launch configurations, one per swept shape, consulted by",
-        "// pick_fwd (grouped_gemm.hip) before its built-in rule.  Written by",
-        "// `python grouped-gemms_amd/tune_driver.py --emit-header` from the sweep's",
-        "// best.json; regenerate rather than edit.  An entry applies to calls with",
+        "// pick_fwd (grouped_gemm.hip) before its built-in rule.  Proposed by",
+        "// `python grouped-gemms_amd/tune_driver.py --emit-header` from a sweep's",
+        "// best.json; an entry stays while whole calls, entry and built-in rule in turn,",
+        "// gain at least 1% by it.  An entry applies to calls with",
         "// the same E, N, K and weight format and M within a factor of two of the",
         "// swept M, on every operand layout (the tile order can change the bits of a",
         "// call whose last round is split).  Fields: E, M, N, K, b_fmt (0 e4m3, 4",
