@@ -92,27 +92,22 @@ def time_call(fn, steps: int, warmup: int, flush_buf):
     return statistics.median(ts), sum(ts) / len(ts)
 
 
-def fwd_kernel_name(cfg: dict, rows: bool = False) -> str:
+def fwd_kernel_name(cfg: dict) -> str:
     """Device-kernel name (as rocprofv3 lists it) of the whole-tile kernel of an
     e4m3 forward/dgrad launch on step-major scales: Cfg<BLOCK_M, BLOCK_N, waves
     along M, waves along N, B format, 64-element half steps in LDS, plain
-    scales>, pieces=false, bf16 epilogue, whatever the data layout; with
-    ``rows``, the name older summaries list the 256 x 256 tiles of row-major A
-    under.  A call may also launch the piece / quarter-tile / reduce kernels of
-    a split last round; the kernel-only event time covers those too."""
-    if rows and cfg["BLOCK_M"] == 256:
-        return XLINE_KERNEL
+    scales>, pieces=false, bf16 epilogue, whatever the data layout.  A call may
+    also launch the piece / quarter-tile / reduce kernels of a split last round;
+    the kernel-only event time covers those too."""
     return f"mxgg::fwd_kernel<mxgg::Cfg<{cfg['BLOCK_M']}, {cfg['BLOCK_N']}, 2, 2, 0, 4, false>, false, 1>"
 
 
-# the 256 x 256 e4m3 forward whole-tile kernel, and the separate one for row-major A that older summaries list
+# the 256 x 256 e4m3 forward whole-tile kernel
 FWD_KERNEL = "mxgg::fwd_kernel<mxgg::Cfg<256, 256, 2, 2, 0, 4, false>, false, 1>"
-XLINE_KERNEL = "mxgg::fwd_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>"
 
 
 # whole-tile kernels with the bf16 epilogue (template argument 1): the bench's outputs are bf16 with aligned rows
 WGRAD_KERNEL = "mxgg::wgrad_kernel<mxgg::Cfg<256, 256, 2, 2, 0, 4, false>, false, 1>"
-WGRAD_XLINE = "mxgg::wgrad_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>"
 
 
 def wgrad_kernel_name(E: int, M: int, N: int, K: int) -> str:

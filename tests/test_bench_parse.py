@@ -22,11 +22,7 @@ def test_gemm_launch_kinds():
         "mxgg::fwd_quad_kernel<mxgg::Cfg<256, 256, 2, 2, 0, 4, true>, mxgg::Cfg<128, 128, 2, 2, 0, 4, true>, 1>": None,
         "mxgg::fwd_reduce_kernel<mxgg::Cfg<256, 256, 2, 2, 0, 4, false> >": None,
         "mxgg::scale_relayout_kernel": None,
-        "void mxgg::fwd_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>(mxgg::FwdParams)":
-            "whole",
-        "mxgg::fwd_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, true, 0>": "piece",
-        "mxgg::fwd_quad_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, "
-        "mxgg::Cfg<128, 128, 2, 2, 0, 4, false>, 1>": None,
+        "mxgg::fwd_stream_kernel<mxgg::StreamCfg<32, 0, 3, true>, 1>(mxgg::FwdParams)": None,
     }
     for name, kind in kinds.items():
         assert bench.gemm_launch(name) == kind, name
@@ -43,14 +39,9 @@ def test_canon_matches_summaries_without_scale_source():
     assert bench.fwd_kernel_name({"BLOCK_M": 256, "BLOCK_N": 256}) == new
 
 
-def test_fwd_kernel_names_by_layout():
-    # row-major A runs the 256 x 256 tiles as XLine (the demangled name of
-    # fwd_kernel<XLine<Cfg<256, 256, 2, 2, 0, 3>>, false, 1>); row pairs, and
-    # 128 x 128 tiles on either layout, the one-stage configuration
-    xl = "void mxgg::fwd_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>(mxgg::FwdParams)"
-    assert bench.canon(bench.fwd_kernel_name({"BLOCK_M": 256, "BLOCK_N": 256}, rows=True)) == bench.canon(xl)
+def test_fwd_kernel_names_by_tile():
     assert bench.fwd_kernel_name({"BLOCK_M": 256, "BLOCK_N": 256}) == bench.FWD_KERNEL
-    assert bench.fwd_kernel_name({"BLOCK_M": 128, "BLOCK_N": 128}, rows=True) == \
+    assert bench.fwd_kernel_name({"BLOCK_M": 128, "BLOCK_N": 128}) == \
         "mxgg::fwd_kernel<mxgg::Cfg<128, 128, 2, 2, 0, 4, false>, false, 1>"
 
 
@@ -59,7 +50,7 @@ def test_summary_lines_parse(tmp_path, monkeypatch):
     # stats_summary writes them, read back by the bench's roofline
     prof = tmp_path / "profiles"
     prof.mkdir()
-    fw, xl = bench.FWD_KERNEL, bench.XLINE_KERNEL
+    fw, xl = bench.FWD_KERNEL, bench.FWD_KERNEL.replace("4, false", "4, true")   # step-major, plain scales
     (prof / "kernel_stats_sweep.txt").write_text(
         f"  {xl:62s} all calls   5000: avg    400.00 us;  right after the cache flush   4400: avg    410.00 us;"
         f"  the sweep's first 4320: avg    420.50 us\n"
@@ -75,11 +66,8 @@ def test_summary_lines_parse(tmp_path, monkeypatch):
     assert d is not None and d["calls"] == 4320 and d["frac"] == 0.435 and d["frac_with_relayout"] == 0.413
     assert bench.read_dropin_gemm(fw)["kernels"] == [fw, xl]
     assert bench.read_dropin_gemm(bench.WGRAD_KERNEL) is None
-    # the wgrad family's line: the one-stage kernel where the call stages both
-    # operands, XLine on row-major go_t
-    wk, wx = bench.WGRAD_KERNEL, bench.WGRAD_XLINE
-    assert bench.canon(wx) == bench.canon(
-        "void mxgg::wgrad_kernel<mxgg::XLine<mxgg::Cfg<256, 256, 2, 2, 0, 3, false> >, false, 1>(mxgg::WgradParams)")
+    # the wgrad family's line
+    wk, wx = bench.WGRAD_KERNEL, bench.WGRAD_KERNEL.replace("256, 256", "128, 128")
     with open(prof / "kernel_stats_sweep.txt", "a") as f:
         f.write(f"  the sweep's 2100 drop-in calls of {wk} and {wx}: GEMM launches 300.00 us = 2000.0 TFLOP/s = "
                 f"0.400 of 5000.0 (dense MXFP8); with the re-layout launch (20.00 us) 1875.0 TFLOP/s = 0.375\n")
