@@ -68,9 +68,9 @@ def _aligned_rows(batch: tuple, rows: int, length: int, device) -> tuple:
     128-byte grid: a view of a buffer with the row stride rounded up to a
     multiple of 128 when ``length`` is not one (e.g. the token-major operands
     of the weight gradient, whose length is the token count).  The GEMM
-    copies operand rows in 64-byte pieces; rows off the 128-byte grid put a
-    quarter of them across two cache lines (wgrad at 2080 tokens: 12-16%
-    slower).  Returns ``(view, row stride)``."""
+    copies 128 bytes of an operand row at a time, whole cache lines on that
+    grid and halves of two off it (wgrad at 2080 tokens, copied in 64-byte
+    pieces: 12-16% slower).  Returns ``(view, row stride)``."""
     ld = (length + 127) // 128 * 128
     buf = torch.empty(tuple(batch) + (rows, ld), dtype=torch.uint8, device=device)
     return buf[..., :length], ld

@@ -14,8 +14,8 @@ bounds off the 32-token grid, empty groups, ragged N and K
 (operands from the fused transposing quantizer where their rows allow it,
 else from to_mx of the transposed copy, as the reference quantizes them).
 Sizes keep the fp64 oracle near a second per case.  Row-major against row
-pairs: the XLine main loop and the one-stage one give the same bits on random
-256 x 256 launches (no oracle needed: the two layouts are the same numbers).
+pairs: the same bits on random 256 x 256 launches (no oracle needed: the two
+layouts are the same numbers).
 """
 
 import random
@@ -125,10 +125,9 @@ def test_wgrad_fuzz(gpu, case):
 
 @pytest.mark.parametrize("case", range(24))
 def test_row_major_matches_row_pairs_fuzz(gpu, case):
-    """256 x 256 tiles on random shapes: row-major operands (the XLine main
-    loop, the X operand in two-stage LDS slots) give, bit for bit, the
-    one-stage kernel's result on the same operands in row pairs, for the
-    forward and the wgrad (odd stage counts, ragged groups, split calls)."""
+    """256 x 256 tiles on random shapes: row-major operands give, bit for bit,
+    the result of the same operands in row pairs, for the forward and the wgrad
+    (odd step counts, ragged groups, split calls)."""
     import kernels
     rng = random.Random(9100 + case)
     E = rng.choice([1, 1, 2, 3, 4, 8])

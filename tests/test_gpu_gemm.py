@@ -178,6 +178,8 @@ def _routed(E, M, seed):
     (8, 300, 256, 2048, "e4m3", torch.bfloat16),     # 64-row tiles
     (5, 239, 136, 4192, "e4m3", torch.float16),      # 64-row tiles, 33 steps, groups past 64 rows
     (8, 300, 128, 640, "e2m1", torch.float32),       # 64-row tiles, packed weight
+    (80, 300, 200, 544, "e4m3", torch.bfloat16),     # more than 64 groups (offsets scanned in chunks), some empty
+    (70, 900, 136, 512, "e2m1", torch.float16),      # the same, 64-row tiles
 ])
 def test_few_rows_match_general_tiles(gpu, E, M, N, K, elem, out_dtype):
     """Calls of few rows per group run weight-streaming tiles: the bits of the
@@ -232,11 +234,12 @@ def test_few_rows_workspace_holds_scales_only(gpu):
 @pytest.mark.parametrize("N", [512, 300, 301, 96])     # whole tiles, 16-byte rows, rows off the grid, one narrow tile
 @pytest.mark.parametrize("tile", [128, 256])
 def test_f32_output_rounds_to_bf16_output(gpu, N, tile):
-    """Every f32 epilogue (rows staged through LDS in 16-byte chunks, partial
-    tiles, rows off the 16-byte grid) stores the accumulators that the bf16
-    call rounds: forward f32 output rounded to bf16 equals the bf16 output bit
-    for bit, and a wgrad's f32 output, bf16-rounded already, equals it as
-    stored."""
+    """The f32 epilogues of the forward's tiles and of 128 x 128 wgrad tiles
+    (rows staged through LDS in 16-byte chunks, partial tiles, rows off the
+    16-byte grid) store the accumulators that the bf16 call rounds: forward f32
+    output rounded to bf16 equals the bf16 output bit for bit, and a wgrad's f32
+    output, bf16-rounded already, equals it as stored.  (256 x 256 wgrad tiles:
+    the next test.)"""
     import kernels
     E, M, K = 3, 1056, 416
     offs = torch.tensor([100, 100 + 517, M], dtype=torch.int32, device=gpu)
@@ -253,6 +256,28 @@ def test_f32_output_rounds_to_bf16_output(gpu, N, tile):
     outs = [kernels.triton_mxfp8_wgrad(qg, sg, qi, si, offs, out_dtype=dt) for dt in (torch.float32, torch.bfloat16)]
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1].float())
+
+
+@pytest.mark.parametrize("N,K", [(2048, 1792), (1800, 1640), (1800, 1638)])   # whole tiles, ragged, rows off the grid
+def test_wgrad_f32_output_of_256_tiles(gpu, N, K):
+    """f32 weight gradients of whole 256 x 256 tiles hold the bf16 call's values
+    and agree with the oracle."""
+    import ctypes
+    import kernels
+    from kernels import _lib
+    E, M = 3, 1056
+    block = ctypes.c_int32(0)
+    _lib.check(_lib.load().mxgg_wgrad_config(E, M, N, K, ctypes.byref(block)))
+    assert block.value == 256
+    offs = [300, 300 + 420, M]
+    sg, qg = _quant(randn_bf16((N, M), 1.0, 3), gpu)
+    si, qi = _quant(randn_bf16((K, M), 1.0, 4), gpu)
+    o = torch.tensor(offs, dtype=torch.int32, device=gpu)
+    f, b = (kernels.triton_mxfp8_wgrad(qg, sg, qi, si, o, out_dtype=dt) for dt in (torch.float32, torch.bfloat16))
+    torch.cuda.synchronize()
+    assert torch.equal(f, b.float())
+    ref = O.wgrad(bits_u8(qg), bits_u8(sg), bits_u8(qi), bits_u8(si), offs)
+    _assert_close(f.cpu().numpy(), ref)
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])

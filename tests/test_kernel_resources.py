@@ -76,7 +76,7 @@ def _kernels():
 def test_code_objects_found():
     ks = _kernels()
     names = " ".join(ks)
-    for part in ("fwd_kernel", "wgrad_kernel", "fwd_quad_kernel", "fwd_reduce_kernel", "wgrad_reduce_kernel",
+    for part in ("fwd_kernel", "wgrad_kernel", "fwd_quad_kernel", "fwd_stream_kernel", "fwd_reduce_kernel", "wgrad_reduce_kernel",
                  "scale_relayout_kernel", "quant_rows_kernel", "quant_tile_kernel", "schedule_kernel",
                  "routing_kernel"):
         assert part in names, f"no {part} in the gfx950 code objects"
@@ -99,7 +99,7 @@ def test_gemm_kernels_one_wave_per_simd():
     256 x 256 tiles) with at most 512 registers per lane (``.vgpr_count`` is the unified count, AGPRs
     included); anything else means the tile configuration or launch bounds
     changed."""
-    gemm = {n: k for n, k in _kernels().items() if re.search(r"(fwd|wgrad)_kernel", n)}
+    gemm = {n: k for n, k in _kernels().items() if re.search(r"(fwd|wgrad|fwd_quad|fwd_stream)_kernel", n)}
     assert gemm
     for n, k in gemm.items():
         assert k[".wavefront_size"] == 64, n
