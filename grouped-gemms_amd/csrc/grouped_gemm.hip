@@ -31,8 +31,9 @@
 //     contiguous 1 KB pieces, copied into a two-slot scale area every two
 //     steps (small calls copy the plain scales themselves, 8 steps of a row
 //     at a time); each MFMA picks its lane's byte with op_sel.
-//   * everything but the MFMAs is kept to four instructions per MFMA: one
-//     wave per SIMD issues them all.
+//   * everything but the MFMAs is kept to about four instructions per MFMA
+//     (131 to 136 beside the 32 of a 256 x 256 step): one wave per SIMD issues
+//     them all.
 #include <mutex>
 #include <type_traits>
 
@@ -640,7 +641,7 @@ __device__ __forceinline__ void zero_acc(v16f (&acc)[C::FM][C::FN]) {
 //                       since MFMA NMMA - 1) and its scales
 // A scheduling fence after every MFMA keeps the order.  With a wave alone on
 // its SIMD every other instruction between two MFMAs is issue time the matrix
-// core waits for: 256 x 256 e4m3 tiles issue about 150 per step of 32 MFMAs.
+// core waits for: 256 x 256 tiles issue 131 to 136 per step of 32 MFMAs.
 constexpr int kStepFull = 0, kStepNoCopy = 1, kStepLast = 2;
 template <class C, int KIND, int P0>
 __device__ __forceinline__ void step_pos(uint8_t* smem, const Operand& X, const Operand& W, __amdgpu_buffer_rsrc_t ssr,
