@@ -1116,13 +1116,17 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
         __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(out + ((int64_t)row * ldo + col) * ES));
       }
     } else {
-      // Eight LDS reads, then their stores.  Chunks that only partly lie in the
-      // output (a column count off the 16-byte grid) are the exception: their
-      // per-element branches, skipped one by one, 64 times a wave in f32, cost
-      // more than the stores (wgrad (4, 5280, 2880, 736): f32 50.0 us with them,
-      // 45.1 behind one test, bf16 45.0 and 38.6).
+      // Chunks that only partly lie in the output (a column count off the
+      // 16-byte grid) are the exception: their per-element branches, skipped
+      // one by one, 64 times a wave in f32, cost more than the stores (wgrad
+      // (4, 5280, 2880, 736): f32 50.2 us with them, 45.1 behind one test, bf16
+      // 45.0 and 38.6).  16-bit rows are read from LDS eight chunks at a time
+      // before their stores (forward (16, 11360, 640, 512) 12.8 us one by one,
+      // 12.6); f32 gains nothing by that.
       const bool parts = cols % EPC != 0;
-      constexpr int IT = FPP * 32 / RPI, NB = IT < 8 ? IT : 8;
+      const int col = wn * C::WTN + (lane % NCH) * EPC;
+      const bool inside = col + EPC <= cols;             // the lane's chunk of every row
+      constexpr int IT = FPP * 32 / RPI, NB = ES == 4 ? 1 : (IT < 8 ? IT : 8);
       static_assert(IT % NB == 0, "store batches");
 #pragma unroll
       for (int it0 = 0; it0 < IT; it0 += NB) {
@@ -1135,11 +1139,11 @@ __device__ __forceinline__ void store_tile_lds(const v16f (&acc)[C::FM][C::FN], 
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
           const int row = wm * C::WTM + i0 * 32 + (it0 + b) * RPI + lane / NCH;
-          const int col = wn * C::WTN + (lane % NCH) * EPC;
           uint8_t* p = out + ((int64_t)row * ldo + col) * ES;
-          if (row < rows && col + EPC <= cols) {
+          if (row >= rows) continue;
+          if (inside) {
             *reinterpret_cast<uint4*>(p) = v[b];
-          } else if (parts && row < rows) {
+          } else if (parts) {
             const uint32_t w[4] = {v[b].x, v[b].y, v[b].z, v[b].w};
 #pragma unroll
             for (int e = 0; e < EPC; ++e)
